@@ -2,11 +2,12 @@
 //
 // With T = double and -ffp-contract=off these reproduce Flou.jl's Float64 arithmetic term
 // by term: left folds for n-ary sums, `a / 2b` as a / (2*b), `x^2` as x*x, `x^3` as
-// (x*x)*x, divisions by 3, 5, 7 kept as divisions.  With T = float the same structure runs
-// in single precision.
+// (x*x)*x, divisions by 3, 5, 7 rounded as divisions (exact_div.hpp).  With T = float the
+// same structure runs in single precision.
 #pragma once
 
 #include "common.hpp"
+#include "exact_div.hpp"
 
 namespace flouhip {
 namespace plain {
@@ -20,38 +21,42 @@ template <typename T> __device__ inline T dlog(T x, int* err) {
     return log(x);
 }
 
-// pressure (FlouCommon/Euler.jl:142-155)
+// pressure (FlouCommon/Euler.jl:142-155); ir: the reciprocal of Q[0]
 template <typename T, int ND>
-__device__ inline T pressure(const T* Q, T gamma) {
+__device__ inline T pressure(const T* Q, T gamma, const Recip<T>& ir) {
     T s = Q[1] * Q[1];
 #pragma unroll
     for (int k = 1; k < ND; ++k) s = s + Q[1 + k] * Q[1 + k];
-    return (gamma - T(1)) * (Q[ND + 1] - s / (T(2) * Q[0]));
+    return (gamma - T(1)) * (Q[ND + 1] - ir.div2(s));
 }
 
 // vars_cons2prim (FlouCommon/Euler.jl:237-253)
 template <typename T, int ND>
-__device__ inline void cons2prim(const T* Q, T gamma, T* P) {
-    const T p = pressure<T, ND>(Q, gamma);
+__device__ inline void cons2prim(const T* Q, T gamma, T* P, const Recip<T>& ir) {
+    const T p = pressure<T, ND>(Q, gamma, ir);
     P[0] = Q[0];
 #pragma unroll
-    for (int k = 0; k < ND; ++k) P[1 + k] = Q[1 + k] / Q[0];
+    for (int k = 0; k < ND; ++k) P[1 + k] = ir.div(Q[1 + k]);
     P[ND + 1] = p;
+}
+template <typename T, int ND>
+__device__ inline void cons2prim(const T* Q, T gamma, T* P) {
+    cons2prim<T, ND>(Q, gamma, P, Recip<T>(Q[0]));
 }
 
 // logarithmic_mean (FlouCommon/Utilities.jl:34-44)
 template <typename T>
 __device__ inline T logarithmic_mean(T al, T ar, int* err) {
-    const T xi = al / ar;
-    const T f = (xi - T(1)) / (xi + T(1));
+    const T xi = xdiv(al, ar);
+    const T f = xdiv(xi - T(1), xi + T(1));
     const T u = f * f;
     T F;
     if (u < T(0.01)) {
-        F = ((T(1) + u / T(3)) + (u * u) / T(5)) + ((u * u) * u) / T(7);
+        F = ((T(1) + cdiv<3>(u)) + cdiv<5>(u * u)) + cdiv<7>((u * u) * u);
     } else {
-        F = dlog(xi, err) / (T(2) * f);
+        F = xdiv(dlog(xi, err), T(2) * f);
     }
-    return (al + ar) / (T(2) * F);
+    return xdiv(al + ar, T(2) * F);
 }
 
 // Contravariant physical volume flux in direction dir (OpDivergence.jl:28-37,
@@ -66,10 +71,11 @@ __device__ inline void contravariant_flux(const T* Q, const T* M, int dir, T gam
 #pragma unroll
         for (int k = 0; k < ND; ++k) F[k][0] = avel[k] * Q[0];
     } else {
+        const Recip<T> ir(Q[0]);
         T u[ND];
 #pragma unroll
-        for (int m = 0; m < ND; ++m) u[m] = Q[1 + m] / Q[0];
-        const T p = pressure<T, ND>(Q, gamma);
+        for (int m = 0; m < ND; ++m) u[m] = ir.div(Q[1 + m]);
+        const T p = pressure<T, ND>(Q, gamma, ir);
 #pragma unroll
         for (int k = 0; k < ND; ++k) {
             F[k][0] = Q[1 + k];
@@ -90,8 +96,16 @@ __device__ inline void contravariant_flux(const T* Q, const T* M, int dir, T gam
     }
 }
 
+// The node scalar the two-point flux reads beside the primitives: E/ρ for Kennedy-Gruber,
+// else β = ρ/(2p); ir: the reciprocal of ρ.
+template <typename T, int ND, int TP>
+__device__ inline T tp_scalar(const T* Q, const T* P, const Recip<T>& ir) {
+    return TP == TP_KENNEDY_GRUBER ? ir.div(Q[ND + 1]) : xdiv(P[0], T(2) * P[ND + 1]);
+}
+
 // Two-point volume flux (Equations/Euler.jl:385-536; Equations/LinearAdvection.jl:44-47).
-// P1/P2: cached primitives (ρ, u.., p); b1/b2: ρ/(2p).  Ja1/Ja2: metric column `dir`.
+// P1/P2: cached primitives (ρ, u.., p); b1/b2: the node's tp_scalar (ρ/(2p), or the specific
+// energy for Kennedy-Gruber).  Ja1/Ja2: metric column `dir`.
 template <typename T, int ND, int EQ, int TP>
 __device__ inline void twopointflux(const T* Q1, const T* Q2, const T* P1, const T* P2, T b1,
                                     T b2, const T* Ja1, const T* Ja2, T gamma, const T* avel,
@@ -128,15 +142,15 @@ __device__ inline void twopointflux(const T* Q1, const T* Q2, const T* P1, const
 #pragma unroll
         for (int k = 0; k < ND; ++k) um[k] = (P1[1 + k] + P2[1 + k]) / T(2);
         const T rho = logarithmic_mean(rho1, rho2, err);
-        const T p = (rho1 + rho2) / (T(2) * (b1 + b2));
+        const T p = xdiv(rho1 + rho2, T(2) * (b1 + b2));
         const T beta = logarithmic_mean(b1, b2, err);
         T sq = P1[1] * P1[1];
 #pragma unroll
         for (int k = 1; k < ND; ++k) sq = sq + P1[1 + k] * P1[1 + k];
 #pragma unroll
         for (int k = 0; k < ND; ++k) sq = sq + P2[1 + k] * P2[1 + k];
-        T h = T(1) / ((T(2) * beta) * (gamma - T(1))) - sq / T(4);
-        h = h + p / rho;
+        T h = xdiv(T(1), (T(2) * beta) * (gamma - T(1))) - sq / T(4);
+        h = h + xdiv(p, rho);
 #pragma unroll
         for (int k = 0; k < ND; ++k) h = h + um[k] * um[k];
 #pragma unroll
@@ -156,7 +170,7 @@ __device__ inline void twopointflux(const T* Q1, const T* Q2, const T* P1, const
 #pragma unroll
         for (int k = 0; k < ND; ++k) um[k] = (P1[1 + k] + P2[1 + k]) / T(2);
         const T p = (p1 + p2) / T(2);
-        const T e = (Q1[ND + 1] / Q1[0] + Q2[ND + 1] / Q2[0]) / T(2);
+        const T e = (b1 + b2) / T(2);
 #pragma unroll
         for (int k = 0; k < ND; ++k) {
             const T m = rho * um[k];
@@ -221,24 +235,27 @@ __device__ inline void rotate2phys(const T* R, const T* fr, T* Q) {
 // vars_cons2entropy (FlouCommon/Euler.jl:273-307)
 template <typename T, int ND>
 __device__ inline void cons2entropy(const T* Q, T gamma, int* err, T* W) {
-    const T p = pressure<T, ND>(Q, gamma);
+    const Recip<T> ir(Q[0]);
+    const T p = pressure<T, ND>(Q, gamma, ir);
+    const Recip<T> ip(p);
     const T s = dlog(p, err) - gamma * dlog(Q[0], err);
     T m2 = Q[1] * Q[1];
 #pragma unroll
     for (int k = 1; k < ND; ++k) m2 = m2 + Q[1 + k] * Q[1 + k];
-    W[0] = (gamma - s) / (gamma - T(1)) - (m2 / Q[0]) / (T(2) * p);
+    W[0] = xdiv(gamma - s, gamma - T(1)) - ip.div2(ir.div(m2));
 #pragma unroll
-    for (int k = 0; k < ND; ++k) W[1 + k] = Q[1 + k] / p;
-    W[ND + 1] = -Q[0] / p;
+    for (int k = 0; k < ND; ++k) W[1 + k] = ip.div(Q[1 + k]);
+    W[ND + 1] = ip.div(-Q[0]);
 }
 
 // vars_entropy2prim then vars_prim2cons (FlouCommon/Euler.jl:309-339, 255-271).
 template <typename T, int ND>
 __device__ inline void entropy2cons(const T* W, T gamma, int* err, T* Q) {
     const T wl = W[ND + 1];
+    const Recip<T> iw(wl);
     T u[ND];
 #pragma unroll
-    for (int k = 0; k < ND; ++k) u[k] = -W[1 + k] / wl;
+    for (int k = 0; k < ND; ++k) u[k] = iw.div(-W[1 + k]);
     T q2 = u[0] * u[0];
 #pragma unroll
     for (int k = 1; k < ND; ++k) q2 = q2 + u[k] * u[k];
@@ -251,7 +268,7 @@ __device__ inline void entropy2cons(const T* W, T gamma, int* err, T* Q) {
     Q[0] = rho;
 #pragma unroll
     for (int k = 0; k < ND; ++k) Q[1 + k] = rho * u[k];
-    Q[ND + 1] = p / (gamma - T(1)) + (rho * q2) / T(2);
+    Q[ND + 1] = xdiv(p, gamma - T(1)) + (rho * q2) / T(2);
 }
 
 // Euler numerical flux in the face frame (Equations/Euler.jl:99-380).
@@ -260,8 +277,9 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
                                            int typo, T intensity, T g, int* err, T* Fn) {
     constexpr int NV = ND + 2;
     T Pl[NV], Pr[NV];
-    cons2prim<T, ND>(Ql, g, Pl);
-    cons2prim<T, ND>(Qr, g, Pr);
+    const Recip<T> irl(Ql[0]), irr(Qr[0]);
+    cons2prim<T, ND>(Ql, g, Pl, irl);
+    cons2prim<T, ND>(Qr, g, Pr, irr);
     const T pl = Pl[ND + 1], pr = Pr[ND + 1];
     const T ul = Pl[1], ur = Pr[1];
     if (savg == AVG_STD) {
@@ -277,9 +295,9 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
         T um[ND];
 #pragma unroll
         for (int k = 0; k < ND; ++k) um[k] = (Pl[1 + k] + Pr[1 + k]) / T(2);
-        const T bl = rl / (T(2) * pl), br = rr / (T(2) * pr);
+        const T bl = xdiv(rl, T(2) * pl), br = xdiv(rr, T(2) * pr);
         const T rho = logarithmic_mean(rl, rr, err);
-        const T p = (rl + rr) / (T(2) * (bl + br));
+        const T p = xdiv(rl + rr, T(2) * (bl + br));
         const T beta = logarithmic_mean(bl, br, err);
         T sq = Pl[1] * Pl[1];
 #pragma unroll
@@ -289,8 +307,8 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
             const T c = (ND == 3 && k == 2 && typo) ? Pl[ND] : Pr[1 + k];
             sq = sq + c * c;
         }
-        T h = T(1) / ((T(2) * beta) * (g - T(1))) - sq / T(4);
-        h = h + p / rho;
+        T h = xdiv(T(1), (T(2) * beta) * (g - T(1))) - sq / T(4);
+        h = h + xdiv(p, rho);
 #pragma unroll
         for (int k = 0; k < ND; ++k) h = h + um[k] * um[k];
         Fn[0] = rho * um[0];
@@ -300,8 +318,8 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
         Fn[ND + 1] = (rho * um[0]) * h;
     }
     if (sdiss == DISS_LXF) {
-        const T al = dsqrt(g * pl / Pl[0], err);
-        const T ar = dsqrt(g * pr / Pr[0], err);
+        const T al = dsqrt(irl.div(g * pl), err);
+        const T ar = dsqrt(irr.div(g * pr), err);
         const T la = fabs(ul) + al, lb = fabs(ur) + ar;
         const T lam = (la < lb) ? lb : la;
 #pragma unroll
@@ -314,23 +332,23 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
 #pragma unroll
         for (int k = 0; k < ND; ++k) um[k] = (Pl[1 + k] + Pr[1 + k]) / T(2);
         const T rho = (rl + rr) / T(2);
-        const T bl = rl / (T(2) * pl), br = rr / (T(2) * pr);
+        const T bl = xdiv(rl, T(2) * pl), br = xdiv(rr, T(2) * pr);
         const T beta = logarithmic_mean(bl, br, err);
-        const T al = dsqrt(g * pl / rl, err);
-        const T ar = dsqrt(g * pr / rr, err);
+        const T al = dsqrt(irl.div(g * pl), err);
+        const T ar = dsqrt(irr.div(g * pr), err);
         const T la = fabs(ul) + al, lb = fabs(ur) + ar;
         const T lam = (la < lb) ? lb : la;
         T D[NV];
         D[0] = rr - rl;
 #pragma unroll
         for (int k = 0; k < ND; ++k) D[1 + k] = Qr[1 + k] - ((ND == 3 && typo) ? Qr[1 + k] : Ql[1 + k]);
-        T s = (T(1) / beta) / (g - T(1)) + Pl[1] * Pr[1];
+        T s = xdiv(xdiv(T(1), beta), g - T(1)) + Pl[1] * Pr[1];
 #pragma unroll
         for (int k = 1; k < ND; ++k) s = s + Pl[1 + k] * Pr[1 + k];
         T t = um[0] * (Pr[1] - Pl[1]);
 #pragma unroll
         for (int k = 1; k < ND; ++k) t = t + um[k] * (Pr[1 + k] - Pl[1 + k]);
-        t = t + (T(1) / br - T(1) / bl) / (T(2) * (g - T(1)));
+        t = t + xdiv(xdiv(T(1), br) - xdiv(T(1), bl), T(2) * (g - T(1)));
         D[ND + 1] = (s * (rr - rl)) / T(2) + rho * t;
 #pragma unroll
         for (int v = 0; v < NV; ++v) Fn[v] = Fn[v] - ((lam / T(2)) * D[v]) * intensity;
@@ -348,12 +366,12 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
 #pragma unroll
         for (int k = 0; k < ND; ++k) q2 = q2 + Pr[1 + k] * Pr[1 + k];
         const T v2 = T(2) * m2 - q2 / T(2);
-        const T bl = rl / (T(2) * pl), br = rr / (T(2) * pr);
+        const T bl = xdiv(rl, T(2) * pl), br = xdiv(rr, T(2) * pr);
         const T rho = logarithmic_mean(rl, rr, err);
-        const T p = (rl + rr) / (T(2) * (bl + br));
+        const T p = xdiv(rl + rr, T(2) * (bl + br));
         const T beta = logarithmic_mean(bl, br, err);
-        const T a = dsqrt(g * p / rho, err);
-        const T h = ((g / (T(2) * beta)) / (g - T(1))) + v2 / T(2);
+        const T a = dsqrt(xdiv(g * p, rho), err);
+        const T h = xdiv(xdiv(g, T(2) * beta), g - T(1)) + v2 / T(2);
         T Wl[NV], Wr[NV], dW[NV];
         cons2entropy<T, ND>(Ql, g, err, Wl);
         cons2entropy<T, ND>(Qr, g, err, Wr);
@@ -369,11 +387,12 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
         Lam[NV - 1] = fabs(u + a);
 #pragma unroll
         for (int c = 1; c < NV - 1; ++c) Lam[c] = fabs(u);
-        Tm[0] = rho / (T(2) * g);
-        Tm[1] = ((g - T(1)) * rho) / g;
+        const Recip<T> ig(g);
+        Tm[0] = ig.div2(rho);
+        Tm[1] = ig.div((g - T(1)) * rho);
 #pragma unroll
         for (int c = 2; c < NV - 1; ++c) Tm[c] = p;
-        Tm[NV - 1] = rho / (T(2) * g);
+        Tm[NV - 1] = Tm[0];
         R[0][0] = T(1); R[1][0] = u - a;
 #pragma unroll
         for (int k = 1; k < ND; ++k) R[1 + k][0] = um[k];
@@ -439,7 +458,7 @@ __device__ inline void subgrid_frame(int dir, T sjac, T* g) {
 template <typename T>
 __device__ inline T hybrid_delta(T b, T c, int* err) {
     T s = dsqrt(b * b + c, err);
-    s = (s - b) / s;
+    s = xdiv(s - b, s);
     return (s < T(0.5)) ? T(0.5) : s;
 }
 

@@ -112,11 +112,12 @@ __device__ void hybrid_nb_line_phases(const RhsArgs<T>& a, const T* sOps, T (&sQ
     }
     __syncthreads();
     if (valid) {
+        const Recip<T> iw(w[ii]);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const T l = ii == 0 ? -sFn[le][2 * dir][v][f] : sHs[le][v][line_node<ND, N>(dir, f, ii - 1)];
             const T r = ii == N - 1 ? sFn[le][2 * dir + 1][v][f] : sHs[le][v][node];
-            acc[v] = acc[v] + (l - r) / w[ii];
+            acc[v] = acc[v] + iw.div(l - r);
         }
     }
 }
@@ -238,10 +239,11 @@ __global__ void __launch_bounds__((Cfg<ND, N>::TPB)) k_plain(const RhsArgs<T> a)
         for (int v = 0; v < NV; ++v) q[v] = sQ[le][v][node];
         if constexpr (EQ == EQ_EULER) {
             T P[NV];
-            plain::cons2prim<T, ND>(q, a.gamma, P);
+            const Recip<T> ir(q[0]);
+            plain::cons2prim<T, ND>(q, a.gamma, P, ir);
 #pragma unroll
             for (int v = 0; v < NV; ++v) sP[le][v][node] = P[v];
-            sP[le][NV][node] = P[0] / (T(2) * P[ND + 1]);
+            sP[le][NV][node] = plain::tp_scalar<T, ND, TP>(q, P, ir);
         }
         if constexpr (VOL == VOL_STRONG) {
             const T* Mp = &sG[le][0];
@@ -432,11 +434,12 @@ __global__ void __launch_bounds__((Cfg<ND, N>::TPB)) k_plain(const RhsArgs<T> a)
             if (valid) {
                 int f, ii;
                 node_line<ND, N>(node, dir, f, ii);
+                const Recip<T> iw(w[ii]);
 #pragma unroll
                 for (int v = 0; v < NV; ++v) {
                     const T l = ii == 0 ? T(0) : sFb[le][v][f][ii];
                     const T r = ii == N - 1 ? T(0) : sFb[le][v][f][ii + 1];
-                    acc[v] = acc[v] + (l - r) / w[ii];
+                    acc[v] = acc[v] + iw.div(l - r);
                 }
             }
             __syncthreads();
@@ -620,13 +623,14 @@ __global__ void __launch_bounds__((Cfg<ND, N>::TPB)) k_plain(const RhsArgs<T> a)
                 for (int side = 0; side < 2; ++side) {
                     T Qe[NV], Pe[NV];
                     plain::entropy2cons<T, ND>(side ? Wr : Wl, a.gamma, a.errflag, Qe);
-                    plain::cons2prim<T, ND>(Qe, a.gamma, Pe);
+                    const Recip<T> ie(Qe[0]);
+                    plain::cons2prim<T, ND>(Qe, a.gamma, Pe, ie);
 #pragma unroll
                     for (int v = 0; v < NV; ++v) {
                         sNb[le2][f][side][v] = Qe[v];
                         sNb[le2][f][side][NV + v] = Pe[v];
                     }
-                    sNb[le2][f][side][2 * NV] = Pe[0] / (T(2) * Pe[ND + 1]);
+                    sNb[le2][f][side][2 * NV] = plain::tp_scalar<T, ND, TP>(Qe, Pe, ie);
                 }
             }
             __syncthreads();
@@ -717,9 +721,10 @@ __global__ void __launch_bounds__((Cfg<ND, N>::TPB)) k_plain(const RhsArgs<T> a)
 
     // Mass matrix (ldiv! by Diagonal(J)) and the stage epilogue
     const int64_t gi = gnode;
+    const Recip<T> iJ(J), i3(T(3));
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
-        const T kv = acc[v] / J;
+        const T kv = iJ.div(acc[v]);
         const int64_t idx = v * Nd + gi;
         const T uin = sQ[le][v][node];
         switch (a.mode) {
@@ -739,7 +744,7 @@ __global__ void __launch_bounds__((Cfg<ND, N>::TPB)) k_plain(const RhsArgs<T> a)
                 a.out[idx] = ((T(3) * (PF ? pf_aux[v] : a.ubase[idx]) + uin) + a.dt * kv) / T(4);
                 break;
             default:
-                a.out[idx] = (((PF ? pf_aux[v] : a.ubase[idx]) + T(2) * uin) + (T(2) * a.dt) * kv) / T(3);
+                a.out[idx] = i3.div(((PF ? pf_aux[v] : a.ubase[idx]) + T(2) * uin) + (T(2) * a.dt) * kv);
                 break;
         }
     }

@@ -38,6 +38,8 @@ def units():
     # the fast adjoint, one unit per two-point flux (StdAverage, Chandrasekhar, Kennedy-Gruber)
     for tp, name in ((0, "std"), (1, "ch"), (2, "kg")):
         u.append((f"vjp_fast_{name}.o", "vjp_fast.hip", ["-ffp-contract=fast", f"-DFLOUHIP_FVJP_TP={tp}"]))
+    for nd in (1, 2, 3):
+        u.append((f"rhs_split_{nd}d.o", "rhs_split.hip", EXACT + [f"-DFLOUHIP_ND={nd}"]))
     for prec in ("F64", "F32"):
         for nd in (1, 2, 3):
             u.append((f"rhs_plain_{prec.lower()}_{nd}d.o", "rhs_plain.hip",

@@ -175,6 +175,26 @@ std::string& create_error() {
     return msg;
 }
 
+// Affine elements whose metric is diagonal and whose face frames are (±e_k, ±e_{k+1}, ±e_{k+2})
+// along the direction k of both elements of the face, zeros exact: Flou's CartesianMesh.
+bool axis_aligned(const flou_hip_desc* d) {
+    const int nd = d->nd;
+    for (int64_t e = 0; e < d->nelements; ++e)
+        for (int r = 0; r < nd; ++r)
+            for (int c = 0; c < nd; ++c)
+                if (r != c && d->elem_metric[(e * nd + c) * nd + r] != 0.0) return false;
+    for (int64_t f = 0; f < d->nfaces; ++f) {
+        const int k = d->face_elempos[f * 2] >> 1;
+        if (d->face_eleminds[f * 2 + 1] >= 0 && d->face_elempos[f * 2 + 1] >> 1 != k) return false;
+        for (int v = 0; v < nd; ++v)  // n, t and (3-D) b
+            for (int c = 0; c < nd; ++c) {
+                const double x = d->face_frames[(f * 3 + v) * nd + c];
+                if (c == (k + v) % nd ? std::fabs(x) != 1.0 : x != 0.0) return false;
+            }
+    }
+    return true;
+}
+
 template <typename T>
 RhsArgs<T> make_args(flou_hip_handle* h) {
     RhsArgs<T> a;
@@ -591,6 +611,13 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
                          : (nd == 2 ? plain_f64_2d(n, h->eq, kvol, h->tp, h->curved)
                                     : plain_f64_3d(n, h->eq, kvol, h->tp, h->curved));
         if (!h->l64) return bad(FLOU_HIP_EUNSUPPORTED, "no kernel for this combination");
+        // split-form Euler with the StdAverage/LxF surface flux on axis-aligned affine elements:
+        // the same results from a kernel without the terms that this geometry makes exact
+        // zeros (3-D N=5, 10.5 M nodes: 0.99 ms per stage against 1.65 ms)
+        if (kvol == VOL_SPLIT && h->eq == FLOU_HIP_EULER && h->savg == FLOU_HIP_AVG_STD &&
+            (h->sdiss == FLOU_HIP_DISS_NONE || h->sdiss == FLOU_HIP_DISS_LXF) && !h->curved && !oriented &&
+            h->gather && h->lift_end && axis_aligned(d))
+            h->l64 = nd == 1 ? split_f64_1(n, h->tp) : (nd == 2 ? split_f64_2(n, h->tp) : split_f64_3(n, h->tp));
     } else {
         h->l32 = nd == 1 ? plain_f32_1d(n, h->eq, kvol, h->tp, h->curved)
                          : (nd == 2 ? plain_f32_2d(n, h->eq, kvol, h->tp, h->curved)

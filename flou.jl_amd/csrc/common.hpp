@@ -204,6 +204,12 @@ RhsLauncherF32 plain_f32_1d(int n, int eq, int vol, int tp, int curved);
 RhsLauncherF32 plain_f32_2d(int n, int eq, int vol, int tp, int curved);
 RhsLauncherF32 plain_f32_3d(int n, int eq, int vol, int tp, int curved);
 
+// FP64 split-form Euler kernels on axis-aligned affine elements, GLL nodes, StdAverage or
+// LxF(StdAverage) surface flux (rhs_split.hip): the plain kernels' results.
+RhsLauncherF64 split_f64_1(int n, int tp);
+RhsLauncherF64 split_f64_2(int n, int tp);
+RhsLauncherF64 split_f64_3(int n, int tp);
+
 typedef hipError_t (*VjpLauncherF64)(const VjpArgs<double>&, hipStream_t);
 typedef hipError_t (*VjpLauncherF32)(const VjpArgs<float>&, hipStream_t);
 VjpLauncherF64 vjp_f64_1d(int n, int eq, int vol, int tp, int curved, int gen);

@@ -42,6 +42,8 @@ def units():
         u.append((f"rhs_split_{nd}d.o", "rhs_split.hip", EXACT + [f"-DFLOUHIP_ND={nd}"]))
     for prec in ("F64", "F32"):
         for nd in (1, 2, 3):
+            u.append((f"rhs_hybrid_{prec.lower()}_{nd}d.o", "rhs_hybrid.hip",
+                      EXACT + [f"-DFLOUHIP_PREC_{prec}", f"-DFLOUHIP_ND={nd}"]))
             u.append((f"rhs_plain_{prec.lower()}_{nd}d.o", "rhs_plain.hip",
                       EXACT + [f"-DFLOUHIP_PREC_{prec}", f"-DFLOUHIP_ND={nd}"]))
             u.append((f"vjp_plain_{prec.lower()}_{nd}d.o", "vjp_plain.hip",

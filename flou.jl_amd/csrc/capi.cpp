@@ -606,7 +606,16 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
     if (kvol == VOL_SPLIT_NB && (h->eq != FLOU_HIP_EULER || h->curved))
         return bad(FLOU_HIP_EUNSUPPORTED,
                    "the split form on Gauss nodes is implemented for the Euler equations on Cartesian elements");
-    if (h->prec == FLOU_HIP_FP64) {
+    const bool diag = !h->curved && axis_aligned(d);
+    if (kvol == VOL_HYBRID) {
+        if (h->prec == FLOU_HIP_FP64)
+            h->l64 = nd == 1 ? hybrid_f64_1(n, h->tp, diag)
+                             : (nd == 2 ? hybrid_f64_2(n, h->tp, diag) : hybrid_f64_3(n, h->tp, diag));
+        else
+            h->l32 = nd == 1 ? hybrid_f32_1(n, h->tp, diag)
+                             : (nd == 2 ? hybrid_f32_2(n, h->tp, diag) : hybrid_f32_3(n, h->tp, diag));
+        if (!h->l64 && !h->l32) return bad(FLOU_HIP_EUNSUPPORTED, "no kernel for this combination");
+    } else if (h->prec == FLOU_HIP_FP64) {
         h->l64 = nd == 1 ? plain_f64_1d(n, h->eq, kvol, h->tp, h->curved)
                          : (nd == 2 ? plain_f64_2d(n, h->eq, kvol, h->tp, h->curved)
                                     : plain_f64_3d(n, h->eq, kvol, h->tp, h->curved));
@@ -615,8 +624,8 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
         // the same results from a kernel without the terms that this geometry makes exact
         // zeros (3-D N=5, 10.5 M nodes: 0.99 ms per stage against 1.65 ms)
         if (kvol == VOL_SPLIT && h->eq == FLOU_HIP_EULER && h->savg == FLOU_HIP_AVG_STD &&
-            (h->sdiss == FLOU_HIP_DISS_NONE || h->sdiss == FLOU_HIP_DISS_LXF) && !h->curved && !oriented &&
-            h->gather && h->lift_end && axis_aligned(d))
+            (h->sdiss == FLOU_HIP_DISS_NONE || h->sdiss == FLOU_HIP_DISS_LXF) && diag && !oriented &&
+            h->gather && h->lift_end)
             h->l64 = nd == 1 ? split_f64_1(n, h->tp) : (nd == 2 ? split_f64_2(n, h->tp) : split_f64_3(n, h->tp));
     } else {
         h->l32 = nd == 1 ? plain_f32_1d(n, h->eq, kvol, h->tp, h->curved)
@@ -881,7 +890,7 @@ int flou_hip_rhs(flou_hip_handle* h, void* dQ, const void* Q, double t) {
 }
 
 namespace {
-// Zhang & Shu limiter in place on Q (Euler.jl:619-653), one thread per element.
+// Zhang & Shu limiter in place on Q (Euler.jl:619-653).
 int apply_limiter(flou_hip_handle* h, void* Q, double minval) {
     hipError_t e;
     if (h->prec == FLOU_HIP_FP64)

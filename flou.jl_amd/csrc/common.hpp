@@ -204,6 +204,14 @@ RhsLauncherF32 plain_f32_1d(int n, int eq, int vol, int tp, int curved);
 RhsLauncherF32 plain_f32_2d(int n, int eq, int vol, int tp, int curved);
 RhsLauncherF32 plain_f32_3d(int n, int eq, int vol, int tp, int curved);
 
+// HybridDivOperator on GLL nodes (rhs_hybrid.hip); diag: axis-aligned affine elements.
+RhsLauncherF64 hybrid_f64_1(int n, int tp, bool diag);
+RhsLauncherF64 hybrid_f64_2(int n, int tp, bool diag);
+RhsLauncherF64 hybrid_f64_3(int n, int tp, bool diag);
+RhsLauncherF32 hybrid_f32_1(int n, int tp, bool diag);
+RhsLauncherF32 hybrid_f32_2(int n, int tp, bool diag);
+RhsLauncherF32 hybrid_f32_3(int n, int tp, bool diag);
+
 // FP64 split-form Euler kernels on axis-aligned affine elements, GLL nodes, StdAverage or
 // LxF(StdAverage) surface flux (rhs_split.hip): the plain kernels' results.
 RhsLauncherF64 split_f64_1(int n, int tp);

@@ -193,6 +193,95 @@ __device__ inline void twopointflux(const T* Q1, const T* Q2, const T* P1, const
     }
 }
 
+// Node values that pair_flux reads (slots): ρ, u.. and the flux's scalars: Chandrasekhar β; Kennedy-Gruber p and
+// E/ρ; StdAverage p, m.. and E.
+template <int ND, int TP>
+constexpr int tp_slots() {
+    return TP == TP_CHANDRASEKHAR ? ND + 2 : (TP == TP_KENNEDY_GRUBER ? ND + 3 : 2 * ND + 3);
+}
+
+// Component DIR of the two-point flux between the lower (1) and higher (2) line position
+// times the metric Ja_dd: twopointflux with a diagonal metric, A and B the nodes' slots.
+template <typename T, int ND, int TP, int DIR>
+__device__ __forceinline__ void pair_flux(const T* A, const T* B, T ja, T gm1, int* err, T* F) {
+    T f[ND + 2];
+    if constexpr (TP == TP_STDAVG) {
+        // slots: ρ, u.., p, m.., E
+        const T p1 = A[ND + 1], p2 = B[ND + 1];
+        const T* m1 = A + ND + 2;
+        const T* m2 = B + ND + 2;
+        f[0] = (m1[DIR] + m2[DIR]) / T(2);
+#pragma unroll
+        for (int c = 0; c < ND; ++c) {
+            T s = m1[c] * A[1 + DIR];
+            if (c == DIR) s = s + p1;
+            s = s + m2[c] * B[1 + DIR];
+            if (c == DIR) s = s + p2;
+            f[1 + c] = s / T(2);
+        }
+        f[ND + 1] = ((m1[ND] + p1) * A[1 + DIR] + (m2[ND] + p2) * B[1 + DIR]) / T(2);
+    } else if constexpr (TP == TP_CHANDRASEKHAR) {
+        const T rho1 = A[0], rho2 = B[0], b1 = A[ND + 1], b2 = B[ND + 1];
+        T um[ND];
+#pragma unroll
+        for (int k = 0; k < ND; ++k) um[k] = (A[1 + k] + B[1 + k]) / T(2);
+        const T rho = logarithmic_mean(rho1, rho2, err);
+        const T p = xdiv(rho1 + rho2, T(2) * (b1 + b2));
+        const T beta = logarithmic_mean(b1, b2, err);
+        T sq = A[1] * A[1];
+#pragma unroll
+        for (int k = 1; k < ND; ++k) sq = sq + A[1 + k] * A[1 + k];
+#pragma unroll
+        for (int k = 0; k < ND; ++k) sq = sq + B[1 + k] * B[1 + k];
+        T h = xdiv(T(1), (T(2) * beta) * gm1) - sq / T(4);
+        h = h + xdiv(p, rho);
+#pragma unroll
+        for (int k = 0; k < ND; ++k) h = h + um[k] * um[k];
+        f[0] = rho * um[DIR];
+#pragma unroll
+        for (int c = 0; c < ND; ++c) {
+            if (c == DIR) f[1 + c] = rho * (um[DIR] * um[DIR]) + p;
+            else f[1 + c] = (rho * um[c < DIR ? c : DIR]) * um[c < DIR ? DIR : c];
+        }
+        f[ND + 1] = (rho * um[DIR]) * h;
+    } else {
+        const T rho = (A[0] + B[0]) / T(2);
+        const T p = (A[ND + 1] + B[ND + 1]) / T(2);
+        const T e = (A[ND + 2] + B[ND + 2]) / T(2);
+        const T ud = (A[1 + DIR] + B[1 + DIR]) / T(2);
+        const T m = rho * ud;
+        f[0] = m;
+#pragma unroll
+        for (int c = 0; c < ND; ++c) {
+            if (c == DIR) f[1 + c] = m * ud + p;
+            else f[1 + c] = m * ((A[1 + c] + B[1 + c]) / T(2));
+        }
+        f[ND + 1] = m * e + p * ud;
+    }
+#pragma unroll
+    for (int v = 0; v < ND + 2; ++v) F[v] = f[v] * ja;
+}
+
+// The slots of a node (see tp_slots) in an array of stride S; CONS false: without the
+// conservative ones of StdAverage (m.., E).
+template <typename T, int ND, int TP, int S, bool CONS = true>
+__device__ __forceinline__ void put_slots(T* s, const T* q, const T* P, const Recip<T>& ir) {
+    s[0] = q[0];
+#pragma unroll
+    for (int k = 0; k < ND; ++k) s[(1 + k) * S] = P[1 + k];
+    if constexpr (TP == TP_CHANDRASEKHAR) {
+        s[(ND + 1) * S] = tp_scalar<T, ND, TP>(q, P, ir);
+    } else {
+        s[(ND + 1) * S] = P[ND + 1];
+        if constexpr (TP == TP_KENNEDY_GRUBER) {
+            s[(ND + 2) * S] = tp_scalar<T, ND, TP>(q, P, ir);
+        } else if constexpr (CONS) {
+#pragma unroll
+            for (int c = 0; c <= ND; ++c) s[(ND + 2 + c) * S] = q[1 + c];
+        }
+    }
+}
+
 // rotate2face / rotate2phys (Equations/Euler.jl:16-64).  fr = (n, t, b), nd each.
 template <typename T, int ND>
 __device__ inline void rotate2face(const T* Q, const T* fr, T* R) {
@@ -271,10 +360,14 @@ __device__ inline void entropy2cons(const T* W, T gamma, int* err, T* Q) {
     Q[ND + 1] = xdiv(p, gamma - T(1)) + (rho * q2) / T(2);
 }
 
-// Euler numerical flux in the face frame (Equations/Euler.jl:99-380).
+// Euler numerical flux in the face frame (Equations/Euler.jl:99-380).  Wl, Wr: the sides'
+// entropy variables in that frame where the caller has them, else null (MatrixDissipation
+// computes them then).  The logarithmic means and the mean pressure that the Chandrasekhar
+// average and the dissipations share are computed once.
 template <typename T, int ND>
 __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, int sdiss,
-                                           int typo, T intensity, T g, int* err, T* Fn) {
+                                           int typo, T intensity, T g, int* err, T* Fn,
+                                           const T* Wl_ = nullptr, const T* Wr_ = nullptr) {
     constexpr int NV = ND + 2;
     T Pl[NV], Pr[NV];
     const Recip<T> irl(Ql[0]), irr(Qr[0]);
@@ -282,6 +375,16 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
     cons2prim<T, ND>(Qr, g, Pr, irr);
     const T pl = Pl[ND + 1], pr = Pr[ND + 1];
     const T ul = Pl[1], ur = Pr[1];
+    T lbl = T(0), lbr = T(0), lbeta = T(0), lrho = T(0), lp = T(0);
+    if (savg == AVG_CHANDRASEKHAR || sdiss == DISS_SCALAR || sdiss == DISS_MATRIX) {
+        lbl = xdiv(Pl[0], T(2) * pl);
+        lbr = xdiv(Pr[0], T(2) * pr);
+        lbeta = logarithmic_mean(lbl, lbr, err);
+        if (savg == AVG_CHANDRASEKHAR || sdiss == DISS_MATRIX) {
+            lrho = logarithmic_mean(Pl[0], Pr[0], err);
+            lp = xdiv(Pl[0] + Pr[0], T(2) * (lbl + lbr));
+        }
+    }
     if (savg == AVG_STD) {
         Fn[0] = (Ql[1] + Qr[1]) / T(2);
         Fn[1] = (((Ql[1] * ul + pl) + Qr[1] * ur) + pr) / T(2);
@@ -291,14 +394,10 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
     } else {
         // ChandrasekharAverage numerical flux (Euler.jl:169-226).  `typo` reproduces
         // Euler.jl:216, which squares wl where wr is meant (3-D only).
-        const T rl = Pl[0], rr = Pr[0];
         T um[ND];
 #pragma unroll
         for (int k = 0; k < ND; ++k) um[k] = (Pl[1 + k] + Pr[1 + k]) / T(2);
-        const T bl = xdiv(rl, T(2) * pl), br = xdiv(rr, T(2) * pr);
-        const T rho = logarithmic_mean(rl, rr, err);
-        const T p = xdiv(rl + rr, T(2) * (bl + br));
-        const T beta = logarithmic_mean(bl, br, err);
+        const T rho = lrho, p = lp, beta = lbeta;
         T sq = Pl[1] * Pl[1];
 #pragma unroll
         for (int k = 1; k < ND; ++k) sq = sq + Pl[1 + k] * Pl[1 + k];
@@ -332,8 +431,7 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
 #pragma unroll
         for (int k = 0; k < ND; ++k) um[k] = (Pl[1 + k] + Pr[1 + k]) / T(2);
         const T rho = (rl + rr) / T(2);
-        const T bl = xdiv(rl, T(2) * pl), br = xdiv(rr, T(2) * pr);
-        const T beta = logarithmic_mean(bl, br, err);
+        const T bl = lbl, br = lbr, beta = lbeta;
         const T al = dsqrt(irl.div(g * pl), err);
         const T ar = dsqrt(irr.div(g * pr), err);
         const T la = fabs(ul) + al, lb = fabs(ur) + ar;
@@ -353,7 +451,6 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
 #pragma unroll
         for (int v = 0; v < NV; ++v) Fn[v] = Fn[v] - ((lam / T(2)) * D[v]) * intensity;
     } else if (sdiss == DISS_MATRIX) {
-        const T rl = Pl[0], rr = Pr[0];
         T um[ND];
 #pragma unroll
         for (int k = 0; k < ND; ++k) um[k] = (Pl[1 + k] + Pr[1 + k]) / T(2);
@@ -366,17 +463,16 @@ __device__ inline void euler_numericalflux(const T* Ql, const T* Qr, int savg, i
 #pragma unroll
         for (int k = 0; k < ND; ++k) q2 = q2 + Pr[1 + k] * Pr[1 + k];
         const T v2 = T(2) * m2 - q2 / T(2);
-        const T bl = xdiv(rl, T(2) * pl), br = xdiv(rr, T(2) * pr);
-        const T rho = logarithmic_mean(rl, rr, err);
-        const T p = xdiv(rl + rr, T(2) * (bl + br));
-        const T beta = logarithmic_mean(bl, br, err);
+        const T rho = lrho, p = lp, beta = lbeta;
         const T a = dsqrt(xdiv(g * p, rho), err);
         const T h = xdiv(xdiv(g, T(2) * beta), g - T(1)) + v2 / T(2);
         T Wl[NV], Wr[NV], dW[NV];
-        cons2entropy<T, ND>(Ql, g, err, Wl);
-        cons2entropy<T, ND>(Qr, g, err, Wr);
+        if (!Wl_) {
+            cons2entropy<T, ND>(Ql, g, err, Wl);
+            cons2entropy<T, ND>(Qr, g, err, Wr);
+        }
 #pragma unroll
-        for (int v = 0; v < NV; ++v) dW[v] = Wl[v] - Wr[v];
+        for (int v = 0; v < NV; ++v) dW[v] = Wl_ ? Wl_[v] - Wr_[v] : Wl[v] - Wr[v];
         const T u = um[0];
         T Lam[NV], Tm[NV], R[NV][NV];
 #pragma unroll

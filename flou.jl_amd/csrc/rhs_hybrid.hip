@@ -1,0 +1,344 @@
+// HybridDivOperator on GLL nodes (OpDivergence.jl:441-620, 781-801; Cartesian elements,
+// Euler) with the numerical flux, the FR lift, 1/J and the RK stage epilogue, in the
+// reference's order (every value rounded where the reference rounds it).
+//
+// Per direction: F̄_s = Σ_{k >= s} Σ_{l < s} (2ω_l D_lk) f♯(Q_l, Q_k) on the interface between
+// line positions s-1 and s, blended with the surface flux of those two nodes by the entropy
+// production of F̄, then dQ_i += (F̄_i - F̄_{i+1})/ω_i.
+//
+// What bounds it: FP64 VALU issue.  The form that evaluated each interface's sum and flux by
+// itself computed the N(N-1)/2 pair fluxes of a line Σ_s s(N-s) times in all (35 instead of 15
+// at N=6) and every node's entropy variables (two logarithms) twice per interface.  Here the
+// block computes
+//   * every pair of a direction once, into an LDS table, with the one flux component that a
+//     diagonal metric keeps (DIAG; pair_flux);
+//   * the entropy variables once per node, read for the blending and, in 1-D and 2-D, where
+//     the face frame is a relabelling that keeps every rounding, for MatrixDissipation;
+//   * the interface sums from the table, one thread per (line, interface), interface-major so
+//     that the lanes of a wave run the same sum; the interface fluxes then replace the table.
+// Blocks of at most 192 threads in 2-D: small meshes then spread evenly over the CUs (7
+// elements per block at N=5 left 55 of 256 CUs with twice the others' work on 2175 elements).
+// Measured: 2-D N=5, 2175 elements, Chandrasekhar and MatrixDissipation: 57 -> 25.5 us per stage.
+// Compile with -DFLOUHIP_PREC_F64 or -DFLOUHIP_PREC_F32 and -DFLOUHIP_ND=1|2|3.
+#include "common.hpp"
+#include "physics_plain.hpp"
+#include "stage.hpp"
+
+namespace flouhip {
+namespace hybrid {
+
+template <int ND, int N>
+struct HCfg {
+    static constexpr int NPE = Cfg<ND, N>::NPE, NPF = Cfg<ND, N>::NPF, NF = 2 * ND, NV = ND + 2;
+    static constexpr int EPB = ND == 2 ? (N == 7 ? 5 : 192 / NPE) : Cfg<ND, N>::EPB;
+    static constexpr int NN = EPB * NPE;
+    static constexpr int TPB = ((NN + 63) / 64) * 64;
+    static constexpr int NL = EPB * NPF;                 // lines per block and direction
+    static constexpr int NPAIR = N * (N - 1) / 2;
+    static constexpr int NPR = NL * NPAIR;
+};
+
+// Flux input slots held beside the conservative states.
+template <int ND, int TP>
+constexpr int lds_slots() {
+    return TP == TP_STDAVG ? ND + 2 : plain::tp_slots<ND, TP>();
+}
+
+// Both sides' states (and entropy variables) of an interface of direction DIR in the
+// subcell frame, n = e_DIR, t and b the next axes: signs of t and b commute with every
+// rounding of the surface fluxes.
+template <typename T, int ND, int DIR>
+__device__ __forceinline__ void to_frame(const T* x, T* r) {
+    r[0] = x[0];
+#pragma unroll
+    for (int c = 0; c < ND; ++c) r[1 + c] = x[1 + (DIR + c) % ND];
+    r[ND + 1] = x[ND + 1];
+}
+
+template <typename T, int ND, int N, int TP, bool DIAG, int DIR>
+__device__ __forceinline__ void direction(const RhsArgs<T>& a, const T* sS, const T* sQ, const T* sW, T* sTab,
+                                          const T* sC, const T* sw, const T* sM, int nel, int tid, int le, int node,
+                                          bool valid, T (&acc)[ND + 2]) {
+    using C = HCfg<ND, N>;
+    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NN = C::NN, NL = C::NL;
+    constexpr int NS = plain::tp_slots<ND, TP>(), NSL = lds_slots<ND, TP>();
+    constexpr int ST = DIR == 0 ? 1 : (DIR == 1 ? N : N * N);
+    const T gm1 = a.gamma - T(1);
+    const T avel[3] = {T(0), T(0), T(0)};
+    // pair fluxes, each once
+#pragma unroll 1
+    for (int k = tid; k < C::NPR; k += C::TPB) {
+        const int pr = k / NL, l = k - pr * NL;
+        const int le2 = C::EPB == 1 ? 0 : l / NPF, f = l - le2 * NPF;
+        if (le2 >= nel) continue;
+        const int ab = pair_ab<N>(pr);
+        const int base = le2 * NPE + line_node<ND, N>(DIR, f, 0);
+        const T* pa = sS + base + (ab >> 3) * ST;
+        const T* pb = sS + base + (ab & 7) * ST;
+        T A[NS], B[NS], F[NV];
+#pragma unroll
+        for (int c = 0; c < NS; ++c) {  // StdAverage's conservative slots lie in sQ
+            A[c] = c < NSL ? pa[c * NN] : sQ[(pa - sS) + (1 + c - NSL) * NN];
+            B[c] = c < NSL ? pb[c * NN] : sQ[(pb - sS) + (1 + c - NSL) * NN];
+        }
+        if constexpr (DIAG) {
+            plain::pair_flux<T, ND, TP, DIR>(A, B, sM[DIR * (ND + 1)], gm1, a.errflag, F);
+        } else {
+            // the general form takes conservative and primitive states
+            T qa[NV], qb[NV], Pa[NV], Pb[NV];
+            const T* ca = sQ + (pa - sS);
+            const T* cb = sQ + (pb - sS);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) { qa[v] = ca[v * NN]; qb[v] = cb[v * NN]; }
+#pragma unroll
+            for (int v = 0; v < NV; ++v) { Pa[v] = A[v]; Pb[v] = B[v]; }  // slot ND+1: p (Chandrasekhar: unread)
+            constexpr int SC = TP == TP_CHANDRASEKHAR ? ND + 1 : (TP == TP_KENNEDY_GRUBER ? ND + 2 : 0);
+            plain::twopointflux<T, ND, EQ_EULER, TP>(qa, qb, Pa, Pb, A[SC], B[SC], sM + ND * DIR, sM + ND * DIR,
+                                                     a.gamma, avel, a.errflag, F);
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) sTab[k * NV + v] = F[v];
+    }
+    __syncthreads();
+    // interface fluxes: at most one per thread (NL (N-1) <= NN)
+    const int s = 1 + tid / NL, l = tid % NL;
+    const bool item = s < N && l / NPF < nel;
+    T Fx[NV];
+    if (item) {
+        T Fb[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) Fb[v] = T(0);
+        for (int ik = s; ik < N; ++ik)
+            for (int il = 0; il < s; ++il) {
+                const int pr = il * (2 * N - il - 1) / 2 + (ik - il - 1);
+                const T* t = sTab + (pr * NL + l) * NV;
+                const T c = sC[il * N + ik];
+#pragma unroll
+                for (int v = 0; v < NV; ++v) Fb[v] = Fb[v] + c * t[v];
+            }
+        const int nr = (l / NPF) * NPE + line_node<ND, N>(DIR, l % NPF, 0) + s * ST, nl = nr - ST;
+        T Ql[NV], Qr[NV], Wl[NV], Wr[NV], Rl[NV], Rr[NV], Vl[NV], Vr[NV], Fr[NV], Fv[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            Ql[v] = sQ[v * NN + nl]; Qr[v] = sQ[v * NN + nr];
+            Wl[v] = sW[v * NN + nl]; Wr[v] = sW[v * NN + nr];
+        }
+        to_frame<T, ND, DIR>(Ql, Rl);
+        to_frame<T, ND, DIR>(Qr, Rr);
+        to_frame<T, ND, DIR>(Wl, Vl);
+        to_frame<T, ND, DIR>(Wr, Vr);
+        plain::euler_numericalflux<T, ND>(Rl, Rr, a.savg, a.sdiss, a.typo, a.intensity, a.gamma, a.errflag, Fr,
+                                          ND <= 2 ? Vl : nullptr, ND <= 2 ? Vr : nullptr);
+        Fv[0] = Fr[0];
+#pragma unroll
+        for (int c = 0; c < ND; ++c) Fv[1 + (DIR + c) % ND] = Fr[1 + c];
+        Fv[NV - 1] = Fr[NV - 1];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) Fv[v] = Fv[v] * a.sjac[DIR];
+        T b = (Wr[0] - Wl[0]) * (Fb[0] - Fv[0]);
+#pragma unroll
+        for (int v = 1; v < NV; ++v) b = b + (Wr[v] - Wl[v]) * (Fb[v] - Fv[v]);
+        const T dl = plain::hybrid_delta(b, a.blend, a.errflag);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) Fx[v] = (T(1) - dl) * Fv[v] + dl * Fb[v];
+    }
+    __syncthreads();  // the table has been read
+    if (item) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) sTab[(v * N + s) * NL + l] = Fx[v];
+    }
+    __syncthreads();
+    if (valid) {
+        int f, ii;
+        node_line<ND, N>(node, DIR, f, ii);
+        const int ln = le * NPF + f;
+        const Recip<T> iw(sw[ii]);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const T x = ii == 0 ? T(0) : sTab[(v * N + ii) * NL + ln];
+            const T y = ii == N - 1 ? T(0) : sTab[(v * N + ii + 1) * NL + ln];
+            acc[v] = acc[v] + iw.div(x - y);
+        }
+    }
+    __syncthreads();  // the interface fluxes have been read
+}
+
+template <typename T, int ND, int N, int TP, bool DIAG>
+__global__ void __launch_bounds__((HCfg<ND, N>::TPB)) k_hybrid(const RhsArgs<T> a) {
+    using C = HCfg<ND, N>;
+    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, EPB = C::EPB, TPB = C::TPB, NN = C::NN;
+    constexpr int NS = lds_slots<ND, TP>();
+    constexpr int TAB = NV * (C::NPR > N * C::NL ? C::NPR : N * C::NL);
+    __shared__ T sS[NS * NN];            // two-point flux inputs
+    __shared__ T sQ[NV * NN];            // conservative states
+    __shared__ T sW[NV * NN];            // entropy variables
+    __shared__ T sTab[TAB];              // pair table of one direction, then its interface fluxes
+    __shared__ T sFn[EPB * NF * NV * NPF];
+    __shared__ T sC[N * N], sw[N], sM[ND * ND];
+
+    const int tid = threadIdx.x;
+    const int e0 = xcd_remap(blockIdx.x, gridDim.x) * EPB;
+    const int64_t Nd = a.ndofs;
+    const int nel = a.ne - e0 < EPB ? a.ne - e0 : EPB;
+    const bool valid = tid < nel * NPE;
+    const int le = tid / NPE, node = tid - le * NPE;
+    const int64_t g0 = (int64_t)e0 * NPE;
+
+    T q[NV], xv[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) q[v] = valid ? a.Q[v * Nd + g0 + tid] : T(1);
+    const T* aux = stage_aux(a);
+    if (aux && valid) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) xv[v] = aux[v * Nd + g0 + tid];
+    }
+    for (int i = tid; i < N * N; i += TPB) sC[i] = (T(2) * a.ops[ops_w(N) + i / N]) * a.ops[ops_D(N) + i];
+    for (int i = tid; i < N; i += TPB) sw[i] = a.ops[ops_w(N) + i];
+    for (int i = tid; i < ND * ND; i += TPB) sM[i] = a.egeom[i];
+    if (valid) {
+        T P[NV], W[NV];
+        const Recip<T> ir(q[0]);
+        plain::cons2prim<T, ND>(q, a.gamma, P, ir);
+        plain::put_slots<T, ND, TP, NN, false>(sS + tid, q, P, ir);
+        plain::cons2entropy<T, ND>(q, a.gamma, a.errflag, W);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            sQ[v * NN + tid] = q[v];
+            sW[v * NN + tid] = W[v];
+        }
+    }
+    __syncthreads();
+
+    // numerical fluxes on the element's faces (interface_fluxes!, applyBCs!); faces of a
+    // Cartesian mesh have orientation 0 or are paired through face_nb_node
+    for (int it = tid; it < EPB * NF * NPF; it += TPB) {
+        const int le2 = it / (NF * NPF), r = it - le2 * (NF * NPF);
+        const int k = r / NPF, f = r - k * NPF;
+        if (le2 >= nel) continue;
+        const int slot = (e0 + le2) * NF + k;
+        const int info = a.finfo[slot], nbe = a.nb[slot];
+        const T* g = a.fgeom + (int64_t)a.fgi[slot] * (3 * ND + 1);
+        const int on = le2 * NPE + line_node<ND, N>(k >> 1, f, (k & 1) ? N - 1 : 0);
+        T own[NV], ext[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) own[v] = sQ[v * NN + on];
+        if (nbe >= 0) {
+            const int kp = finfo_nbpos(info);
+            const T* Qn = a.Q + (int64_t)nbe * NPE +
+                          line_node<ND, N>(kp >> 1, face_nb_node<ND, N>(f, info), (kp & 1) ? N - 1 : 0);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) ext[v] = Qn[v * Nd];
+        } else {
+            const int bd = finfo_bd(info);
+            const int type = a.bctype[bd];
+            const T* src = type == BC_DIRICHLET ? a.bcstate + ((int64_t)a.fid[slot] * NPF + f) * NV
+                                                : a.bcconst + bd * NV;
+#pragma unroll
+            for (int v = 0; v < NV; ++v) ext[v] = type == BC_DIRICHLET || type == BC_INFLOW ? src[v] : own[v];
+            if (type == BC_SLIP) {
+                T R[NV];
+                plain::rotate2face<T, ND>(own, g, R);
+                R[1] = -R[1];
+                plain::rotate2phys<T, ND>(R, g, ext);
+            }
+        }
+        const bool slave = finfo_side(info);
+        T Ql[NV], Qr[NV], Rl[NV], Rr[NV], Fr[NV], F[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            Ql[v] = slave ? ext[v] : own[v];
+            Qr[v] = slave ? own[v] : ext[v];
+        }
+        plain::rotate2face<T, ND>(Ql, g, Rl);
+        plain::rotate2face<T, ND>(Qr, g, Rr);
+        plain::euler_numericalflux<T, ND>(Rl, Rr, a.savg, a.sdiss, a.typo, a.intensity, a.gamma, a.errflag, Fr);
+        plain::rotate2phys<T, ND>(Fr, g, F);
+        const T jac = g[3 * ND];
+        T* o = sFn + ((le2 * NF + k) * NV) * NPF + f;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const T x = F[v] * jac;
+            o[v * NPF] = slave ? -x : x;
+        }
+    }
+
+    T acc[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[v] = T(0);
+    direction<T, ND, N, TP, DIAG, 0>(a, sS, sQ, sW, sTab, sC, sw, sM, nel, tid, le, node, valid, acc);
+    if constexpr (ND >= 2)
+        direction<T, ND, N, TP, DIAG, 1>(a, sS, sQ, sW, sTab, sC, sw, sM, nel, tid, le, node, valid, acc);
+    if constexpr (ND >= 3)
+        direction<T, ND, N, TP, DIAG, 2>(a, sS, sQ, sW, sTab, sC, sw, sM, nel, tid, le, node, valid, acc);
+    if (!valid) return;
+
+    // FR lift: dQ[line[ii]] -= ∂gl[ii]*Fn_left + ∂gr[ii]*Fn_right, direction by direction
+#pragma unroll
+    for (int dir = 0; dir < ND; ++dir) {
+        int f, ii;
+        node_line<ND, N>(node, dir, f, ii);
+        const T gm = a.ops[ops_gm(N) + ii], gp = a.ops[ops_gp(N) + ii];
+        const T* s = sFn + ((le * NF + 2 * dir) * NV) * NPF + f;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) acc[v] = acc[v] - (gm * s[v * NPF] + gp * s[(NV + v) * NPF]);
+    }
+    const Recip<T> iJ(a.egeom[ND * ND]);
+    const StageOut<T> so(a);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) so.put(v * Nd + g0 + tid, iJ.div(acc[v]), q[v], xv[v]);
+}
+
+template <typename T, int ND, int N, int TP, bool DIAG>
+static hipError_t launch(const RhsArgs<T>& a, hipStream_t s) {
+    using C = HCfg<ND, N>;
+    hipLaunchKernelGGL((k_hybrid<T, ND, N, TP, DIAG>), dim3((a.ne + C::EPB - 1) / C::EPB), dim3(C::TPB), 0, s, a);
+    return hipGetLastError();
+}
+
+template <typename T, int ND, int N, bool DIAG>
+static hipError_t (*pick_tp(int tp))(const RhsArgs<T>&, hipStream_t) {
+    switch (tp) {
+        case TP_STDAVG: return &launch<T, ND, N, TP_STDAVG, DIAG>;
+        case TP_CHANDRASEKHAR: return &launch<T, ND, N, TP_CHANDRASEKHAR, DIAG>;
+        case TP_KENNEDY_GRUBER: return &launch<T, ND, N, TP_KENNEDY_GRUBER, DIAG>;
+        default: return nullptr;
+    }
+}
+
+template <typename T, int ND, bool DIAG>
+static hipError_t (*pick_n(int n, int tp))(const RhsArgs<T>&, hipStream_t) {
+    switch (n) {
+        case 2: return pick_tp<T, ND, 2, DIAG>(tp);
+        case 3: return pick_tp<T, ND, 3, DIAG>(tp);
+        case 4: return pick_tp<T, ND, 4, DIAG>(tp);
+        case 5: return pick_tp<T, ND, 5, DIAG>(tp);
+        case 6: return pick_tp<T, ND, 6, DIAG>(tp);
+        case 7: return pick_tp<T, ND, 7, DIAG>(tp);
+        case 8: return pick_tp<T, ND, 8, DIAG>(tp);
+        default: return nullptr;
+    }
+}
+
+}  // namespace hybrid
+
+#if defined(FLOUHIP_PREC_F64)
+#define FLOUHIP_SCALAR double
+#define FLOUHIP_PTAG f64
+#elif defined(FLOUHIP_PREC_F32)
+#define FLOUHIP_SCALAR float
+#define FLOUHIP_PTAG f32
+#else
+#error "define FLOUHIP_PREC_F64 or FLOUHIP_PREC_F32"
+#endif
+#define FLOUHIP_CAT_(p, d) hybrid_##p##_##d
+#define FLOUHIP_CAT(p, d) FLOUHIP_CAT_(p, d)
+
+hipError_t (*FLOUHIP_CAT(FLOUHIP_PTAG, FLOUHIP_ND)(int n, int tp, bool diag))(const RhsArgs<FLOUHIP_SCALAR>&,
+                                                                              hipStream_t) {
+#if FLOUHIP_ND > 1
+    if (!diag) return hybrid::pick_n<FLOUHIP_SCALAR, FLOUHIP_ND, false>(n, tp);
+#endif
+    return hybrid::pick_n<FLOUHIP_SCALAR, FLOUHIP_ND, true>(n, tp);
+}
+
+}  // namespace flouhip

@@ -20,6 +20,7 @@
 #include "common.hpp"
 #include <type_traits>
 #include "physics_plain.hpp"
+#include "stage.hpp"
 
 namespace flouhip {
 
@@ -138,9 +139,6 @@ __global__ void __launch_bounds__((Cfg<ND, N>::TPB)) k_plain(const RhsArgs<T> a)
     __shared__ T sP[EPB][NP][NPE];
     __shared__ T sFt[EPB][NFT][NPE];
     __shared__ T sFn[EPB][NF][NV][NPF];
-    // HybridDivOperator: subcell-interface fluxes of one direction, [le][v][line][s]
-    constexpr int HB = VOL == VOL_HYBRID ? 1 : 0;
-    __shared__ T sFb[HB ? EPB : 1][HB ? NV : 1][HB ? NPF : 1][HB ? N : 1];
     // Split and hybrid forms on Gauss nodes: projected end states (Q, primitives, β) of every
     // line and the two-point fluxes of every node with them, one direction at a time
     constexpr int NB = (VOL == VOL_SPLIT_NB || VOL == VOL_HYBRID_NB) ? 1 : 0;
@@ -204,8 +202,7 @@ __global__ void __launch_bounds__((Cfg<ND, N>::TPB)) k_plain(const RhsArgs<T> a)
 #pragma unroll
         for (int c = 0; c < 3 * ND + 1; ++c) pf_g[c] = g[c];
     }
-    const T* aux = (a.mode == MODE_2N && !a.first) ? a.reg
-                 : ((a.mode == MODE_SSP2 || a.mode == MODE_SSP3) ? a.ubase : nullptr);
+    const T* aux = stage_aux(a);
     if (PF && aux && e0 + tid / NPE < a.ne) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) pf_aux[v] = aux[v * Nd + (int64_t)e0 * NPE + tid];
@@ -372,79 +369,6 @@ __global__ void __launch_bounds__((Cfg<ND, N>::TPB)) k_plain(const RhsArgs<T> a)
     T acc[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) acc[v] = T(0);
-    if constexpr (VOL == VOL_HYBRID) {
-        // Telescopic subcell form (OpDivergence.jl:500-620), direction by direction:
-        // F̄[s] on the interface between line positions s-1 and s (F̄[0] = F̄[N] = 0), then
-        // dQ[i] += (F̄[i] - F̄[i+1]) / ω[i].
-        const T* D = &sOps[ops_D(N)];
-        const T* w = &sOps[ops_w(N)];
-        for (int dir = 0; dir < ND; ++dir) {
-            T gs[3 * ND + 1];
-            plain::subgrid_frame<T, ND>(dir, a.sjac[dir], gs);
-            for (int it = tid; it < EPB * NPF * (N - 1); it += TPB) {
-                const int le2 = it / (NPF * (N - 1)), r = it % (NPF * (N - 1));
-                const int f = r / (N - 1), sp = 1 + r % (N - 1);
-                if (e0 + le2 >= a.ne) continue;
-                const T* M = &sG[le2][0] + ND * dir;
-                T Fb[NV];
-#pragma unroll
-                for (int v = 0; v < NV; ++v) Fb[v] = T(0);
-                for (int ik = sp; ik < N; ++ik) {
-                    const int nk = line_node<ND, N>(dir, f, ik);
-                    T qk[NV], Pk[NV];
-#pragma unroll
-                    for (int v = 0; v < NV; ++v) { qk[v] = sQ[le2][v][nk]; Pk[v] = sP[le2][v][nk]; }
-                    const T bk = sP[le2][NV][nk];
-                    for (int il = 0; il < sp; ++il) {
-                        const int nl = line_node<ND, N>(dir, f, il);
-                        T ql[NV], Pl[NV], Ft[NV];
-#pragma unroll
-                        for (int v = 0; v < NV; ++v) { ql[v] = sQ[le2][v][nl]; Pl[v] = sP[le2][v][nl]; }
-                        const T bl = sP[le2][NV][nl];
-                        plain::twopointflux<T, ND, EQ, TP>(ql, qk, Pl, Pk, bl, bk, M, M, a.gamma, avel,
-                                                           a.errflag, Ft);
-                        const T c = (T(2) * w[il]) * D[il * N + ik];
-#pragma unroll
-                        for (int v = 0; v < NV; ++v) Fb[v] = Fb[v] + c * Ft[v];
-                    }
-                }
-                // FV flux between positions sp-1 and sp on the subcell-interface frame
-                const int nl = line_node<ND, N>(dir, f, sp - 1), nr = line_node<ND, N>(dir, f, sp);
-                T Ql[NV], Qr[NV], Rl[NV], Rr[NV], Fr[NV], Fv[NV], Wl[NV], Wr[NV];
-#pragma unroll
-                for (int v = 0; v < NV; ++v) { Ql[v] = sQ[le2][v][nl]; Qr[v] = sQ[le2][v][nr]; }
-                plain::rotate2face<T, ND>(Ql, gs, Rl);
-                plain::rotate2face<T, ND>(Qr, gs, Rr);
-                plain::euler_numericalflux<T, ND>(Rl, Rr, a.savg, a.sdiss, a.typo, a.intensity, a.gamma,
-                                                  a.errflag, Fr);
-                plain::rotate2phys<T, ND>(Fr, gs, Fv);
-#pragma unroll
-                for (int v = 0; v < NV; ++v) Fv[v] = Fv[v] * gs[3 * ND];
-                // blending on the entropy production of the high-order interface flux
-                plain::cons2entropy<T, ND>(Ql, a.gamma, a.errflag, Wl);
-                plain::cons2entropy<T, ND>(Qr, a.gamma, a.errflag, Wr);
-                T b = (Wr[0] - Wl[0]) * (Fb[0] - Fv[0]);
-#pragma unroll
-                for (int v = 1; v < NV; ++v) b = b + (Wr[v] - Wl[v]) * (Fb[v] - Fv[v]);
-                const T dl = plain::hybrid_delta(b, a.blend, a.errflag);
-#pragma unroll
-                for (int v = 0; v < NV; ++v) sFb[le2][v][f][sp] = (T(1) - dl) * Fv[v] + dl * Fb[v];
-            }
-            __syncthreads();
-            if (valid) {
-                int f, ii;
-                node_line<ND, N>(node, dir, f, ii);
-                const Recip<T> iw(w[ii]);
-#pragma unroll
-                for (int v = 0; v < NV; ++v) {
-                    const T l = ii == 0 ? T(0) : sFb[le][v][f][ii];
-                    const T r = ii == N - 1 ? T(0) : sFb[le][v][f][ii + 1];
-                    acc[v] = acc[v] + iw.div(l - r);
-                }
-            }
-            __syncthreads();
-        }
-    }
     // The Gauss split form has block-wide phases after the volume terms: its threads past
     // the last element stay, skipping every per-node step.
     // The split form's pair phases are block-wide too.
@@ -532,7 +456,7 @@ __global__ void __launch_bounds__((Cfg<ND, N>::TPB)) k_plain(const RhsArgs<T> a)
         if (!valid) return;
     }
 #pragma unroll
-    for (int dir = 0; dir < ((VOL == VOL_HYBRID || VOL == VOL_HYBRID_NB || PS) ? 0 : ND) && valid; ++dir) {
+    for (int dir = 0; dir < ((VOL == VOL_HYBRID_NB || PS) ? 0 : ND) && valid; ++dir) {
         int f, ii;
         node_line<ND, N>(node, dir, f, ii);
         if constexpr (VOL == VOL_STRONG) {
@@ -761,7 +685,7 @@ static hipError_t launch_plain(const RhsArgs<T>& a, hipStream_t s) {
 template <typename T, int ND, int N, bool CURV>
 static hipError_t (*pick_plain(int eq, int vol, int tp))(const RhsArgs<T>&, hipStream_t) {
     if (eq == EQ_ADVECTION) {
-        if (vol == VOL_HYBRID || vol == VOL_SPLIT_NB || vol == VOL_HYBRID_NB) return nullptr;
+        if (vol == VOL_SPLIT_NB || vol == VOL_HYBRID_NB) return nullptr;
         return vol == VOL_STRONG ? &launch_plain<T, ND, N, EQ_ADVECTION, VOL_STRONG, 0, CURV>
                                  : &launch_plain<T, ND, N, EQ_ADVECTION, VOL_SPLIT, 0, CURV>;
     }
@@ -781,15 +705,6 @@ static hipError_t (*pick_plain(int eq, int vol, int tp))(const RhsArgs<T>&, hipS
             case TP_STDAVG: return &launch_plain<T, ND, N, EQ_EULER, VOL_HYBRID_NB, TP_STDAVG, false>;
             case TP_CHANDRASEKHAR: return &launch_plain<T, ND, N, EQ_EULER, VOL_HYBRID_NB, TP_CHANDRASEKHAR, false>;
             case TP_KENNEDY_GRUBER: return &launch_plain<T, ND, N, EQ_EULER, VOL_HYBRID_NB, TP_KENNEDY_GRUBER, false>;
-            default: return nullptr;
-        }
-    }
-    if (vol == VOL_HYBRID) {
-        if constexpr (CURV) return nullptr;  // subcell geometry is defined for Cartesian elements
-        switch (tp) {
-            case TP_STDAVG: return &launch_plain<T, ND, N, EQ_EULER, VOL_HYBRID, TP_STDAVG, false>;
-            case TP_CHANDRASEKHAR: return &launch_plain<T, ND, N, EQ_EULER, VOL_HYBRID, TP_CHANDRASEKHAR, false>;
-            case TP_KENNEDY_GRUBER: return &launch_plain<T, ND, N, EQ_EULER, VOL_HYBRID, TP_KENNEDY_GRUBER, false>;
             default: return nullptr;
         }
     }

@@ -24,6 +24,7 @@
 // Compile with -DFLOUHIP_ND=1|2|3.
 #include "common.hpp"
 #include "physics_plain.hpp"
+#include "stage.hpp"
 
 namespace flouhip {
 namespace split {
@@ -39,96 +40,6 @@ struct SCfg {
     static constexpr int NL = EPB * NPF;                 // lines per block and direction
 };
 
-// Line position a (bits 3..5) and b (bits 0..2) of pair `pr`, pairs (a < b) in row order,
-// ten to a 64-bit word.
-template <int N>
-struct PairTab {
-    unsigned long long w[3] = {0, 0, 0};
-    constexpr PairTab() {
-        int k = 0;
-        for (int a = 0; a < N; ++a)
-            for (int b = a + 1; b < N; ++b, ++k) w[k / 10] |= (unsigned long long)(a * 8 + b) << (6 * (k % 10));
-    }
-};
-template <int N>
-__device__ __forceinline__ int pair_ab(int pr) {
-    constexpr PairTab<N> T;
-    if (N * (N - 1) / 2 <= 10) return (int)(T.w[0] >> (6 * pr)) & 63;
-    const unsigned long long w = pr < 10 ? T.w[0] : (pr < 20 ? T.w[1] : T.w[2]);
-    return (int)(w >> (6 * (pr < 10 ? pr : (pr < 20 ? pr - 10 : pr - 20)))) & 63;
-}
-
-// Node slots in LDS: ρ, u.. and the flux's scalars: Chandrasekhar β; Kennedy-Gruber p and
-// E/ρ; StdAverage p, m.. and E.
-template <int ND, int TP>
-constexpr int slots() {
-    return TP == TP_CHANDRASEKHAR ? ND + 2 : (TP == TP_KENNEDY_GRUBER ? ND + 3 : 2 * ND + 3);
-}
-
-// Component DIR of the two-point flux between the lower (1) and higher (2) line position
-// times the metric Ja_dd (plain::twopointflux with a diagonal metric).
-template <int ND, int TP, int DIR>
-__device__ __forceinline__ void pair_flux(const double* A, const double* B, double ja, double gm1, int* err,
-                                          double* F) {
-    using T = double;
-    T f[ND + 2];
-    if constexpr (TP == TP_STDAVG) {
-        // slots: ρ, u.., p, m.., E
-        const T p1 = A[ND + 1], p2 = B[ND + 1];
-        const T* m1 = A + ND + 2;
-        const T* m2 = B + ND + 2;
-        f[0] = (m1[DIR] + m2[DIR]) / T(2);
-#pragma unroll
-        for (int c = 0; c < ND; ++c) {
-            T s = m1[c] * A[1 + DIR];
-            if (c == DIR) s = s + p1;
-            s = s + m2[c] * B[1 + DIR];
-            if (c == DIR) s = s + p2;
-            f[1 + c] = s / T(2);
-        }
-        f[ND + 1] = ((m1[ND] + p1) * A[1 + DIR] + (m2[ND] + p2) * B[1 + DIR]) / T(2);
-    } else if constexpr (TP == TP_CHANDRASEKHAR) {
-        const T rho1 = A[0], rho2 = B[0], b1 = A[ND + 1], b2 = B[ND + 1];
-        T um[ND];
-#pragma unroll
-        for (int k = 0; k < ND; ++k) um[k] = (A[1 + k] + B[1 + k]) / T(2);
-        const T rho = plain::logarithmic_mean(rho1, rho2, err);
-        const T p = xdiv(rho1 + rho2, T(2) * (b1 + b2));
-        const T beta = plain::logarithmic_mean(b1, b2, err);
-        T sq = A[1] * A[1];
-#pragma unroll
-        for (int k = 1; k < ND; ++k) sq = sq + A[1 + k] * A[1 + k];
-#pragma unroll
-        for (int k = 0; k < ND; ++k) sq = sq + B[1 + k] * B[1 + k];
-        T h = xdiv(T(1), (T(2) * beta) * gm1) - sq / T(4);
-        h = h + xdiv(p, rho);
-#pragma unroll
-        for (int k = 0; k < ND; ++k) h = h + um[k] * um[k];
-        f[0] = rho * um[DIR];
-#pragma unroll
-        for (int c = 0; c < ND; ++c) {
-            if (c == DIR) f[1 + c] = rho * (um[DIR] * um[DIR]) + p;
-            else f[1 + c] = (rho * um[c < DIR ? c : DIR]) * um[c < DIR ? DIR : c];
-        }
-        f[ND + 1] = (rho * um[DIR]) * h;
-    } else {
-        const T rho = (A[0] + B[0]) / T(2);
-        const T p = (A[ND + 1] + B[ND + 1]) / T(2);
-        const T e = (A[ND + 2] + B[ND + 2]) / T(2);
-        const T ud = (A[1 + DIR] + B[1 + DIR]) / T(2);
-        const T m = rho * ud;
-        f[0] = m;
-#pragma unroll
-        for (int c = 0; c < ND; ++c) {
-            if (c == DIR) f[1 + c] = m * ud + p;
-            else f[1 + c] = m * ((A[1 + c] + B[1 + c]) / T(2));
-        }
-        f[ND + 1] = m * e + p * ud;
-    }
-#pragma unroll
-    for (int v = 0; v < ND + 2; ++v) F[v] = f[v] * ja;
-}
-
 // One direction: the pair table, then every node's D♯ row over it in the order j = 0..N-1
 // (diagonal: the contravariant flux), then this node's face terms are left to the caller.
 template <int ND, int N, int TP, int DIR>
@@ -137,7 +48,7 @@ __device__ __forceinline__ void direction(const RhsArgs<double>& a, const double
                                           const double (&q)[ND + 2], const double (&u)[ND], double p,
                                           double (&acc)[ND + 2]) {
     using C = SCfg<ND, N>;
-    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NN = C::NN, NS = slots<ND, TP>();
+    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NN = C::NN, NS = plain::tp_slots<ND, TP>();
     const double gm1 = a.gamma - 1.0;
     __syncthreads();  // the table's memory has been read (the previous direction, or the own traces)
 #pragma unroll 1
@@ -153,7 +64,7 @@ __device__ __forceinline__ void direction(const RhsArgs<double>& a, const double
         double A[NS], B[NS], F[NV];
 #pragma unroll
         for (int c = 0; c < NS; ++c) { A[c] = pa[c * NN]; B[c] = pb[c * NN]; }
-        pair_flux<ND, TP, DIR>(A, B, sG[le2 * (ND + 1) + DIR], gm1, a.errflag, F);
+        plain::pair_flux<double, ND, TP, DIR>(A, B, sG[le2 * (ND + 1) + DIR], gm1, a.errflag, F);
 #pragma unroll
         for (int v = 0; v < NV; ++v) sPair[k * NV + v] = F[v];
     }
@@ -185,11 +96,11 @@ __device__ __forceinline__ void direction(const RhsArgs<double>& a, const double
 }
 
 template <int ND, int N, int TP>
-__global__ void __launch_bounds__((SCfg<ND, N>::TPB), (N <= 6 ? 4 : 2)) k_split(const RhsArgs<double> a) {
+__global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split(const RhsArgs<double> a) {
     using T = double;
     using C = SCfg<ND, N>;
     constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, EPB = C::EPB, TPB = C::TPB, NN = C::NN;
-    constexpr int NS = slots<ND, TP>();
+    constexpr int NS = plain::tp_slots<ND, TP>();
     constexpr int UN = NV * (NN > C::NPR ? NN : C::NPR);
     __shared__ T sS[NS * NN];          // two-point flux inputs, [slot][node]
     __shared__ T sU[UN];               // conservative states [v][node], then the pair table
@@ -237,8 +148,7 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB), (N <= 6 ? 4 : 2)) k_split(
         pn = g[fk >> 1];
         pj = g[3 * ND];
     }
-    const T* aux = (a.mode == MODE_2N && !a.first) ? a.reg
-                 : ((a.mode == MODE_SSP2 || a.mode == MODE_SSP3) ? a.ubase : nullptr);
+    const T* aux = stage_aux(a);
     T xv[NV];
     if (aux && valid) {
 #pragma unroll
@@ -262,20 +172,7 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB), (N <= 6 ? 4 : 2)) k_split(
         if (valid) {
 #pragma unroll
             for (int v = 0; v < NV; ++v) sU[v * NN + tid] = q[v];
-            sS[tid] = q[0];
-#pragma unroll
-            for (int k = 0; k < ND; ++k) sS[(1 + k) * NN + tid] = u[k];
-            if constexpr (TP == TP_CHANDRASEKHAR) {
-                sS[(ND + 1) * NN + tid] = plain::tp_scalar<T, ND, TP>(q, P, ir);
-            } else {
-                sS[(ND + 1) * NN + tid] = p;
-                if constexpr (TP == TP_KENNEDY_GRUBER) {
-                    sS[(ND + 2) * NN + tid] = plain::tp_scalar<T, ND, TP>(q, P, ir);
-                } else {
-#pragma unroll
-                    for (int c = 0; c <= ND; ++c) sS[(ND + 2 + c) * NN + tid] = q[1 + c];
-                }
-            }
+            plain::put_slots<T, ND, TP, NN>(sS + tid, q, P, ir);
         }
     }
     __syncthreads();
@@ -391,32 +288,10 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB), (N <= 6 ? 4 : 2)) k_split(
             for (int v = 0; v < NV; ++v) acc[v] = acc[v] - c * s[v * NPF];
         }
     }
-    const Recip<T> iJ(sG[le * (ND + 1) + ND]), i3(T(3));
+    const Recip<T> iJ(sG[le * (ND + 1) + ND]);
+    const StageOut<T> so(a);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        const T kv = iJ.div(acc[v]);
-        const int64_t idx = v * Nd + g0 + tid;
-        switch (a.mode) {
-            case MODE_RHS:
-                a.out[idx] = kv;
-                break;
-            case MODE_2N: {
-                const T t = a.first ? a.dt * kv : a.A * xv[v] + a.dt * kv;
-                a.reg[idx] = t;
-                a.out[idx] = q[v] + a.B * t;
-                break;
-            }
-            case MODE_SSP1:
-                a.out[idx] = q[v] + a.dt * kv;
-                break;
-            case MODE_SSP2:
-                a.out[idx] = ((T(3) * xv[v] + q[v]) + a.dt * kv) / T(4);
-                break;
-            default:
-                a.out[idx] = i3.div((xv[v] + T(2) * q[v]) + (T(2) * a.dt) * kv);
-                break;
-        }
-    }
+    for (int v = 0; v < NV; ++v) so.put(v * Nd + g0 + tid, iJ.div(acc[v]), q[v], xv[v]);
 }
 
 template <int ND, int N, int TP>

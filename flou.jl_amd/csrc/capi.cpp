@@ -4,9 +4,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -53,8 +55,10 @@ struct flou_hip_handle {
     int* d_bctype = nullptr;
     int* d_err = nullptr;
     double* d_partial = nullptr;
-    double* d_out = nullptr;
-    double* h_out = nullptr;  // pinned
+    unsigned* d_counter = nullptr;  // arrivals of the running reduction's blocks
+    HostResult* h_res = nullptr;    // pinned: result of the last reduction or flag read
+    unsigned long long seq = 0;     // number of the last call that writes h_res
+    bool uniform_dx = false;        // every d_dxe entry is alike
     // host mirrors of the boundary data
     std::vector<int> bctype;
     std::vector<double> bcstate, bcconst;
@@ -140,12 +144,12 @@ int upload_real(flou_hip_handle* h, void** dptr, const std::vector<double>& v) {
 void free_all(flou_hip_handle* h) {
     void* ptrs[] = {h->d_ops, h->d_nb, h->d_finfo, h->d_fgi, h->d_fid, h->d_egeom, h->d_fgeom,
                     h->d_dxe, h->d_jac, h->d_w, h->d_bcstate, h->d_bcconst, h->d_bctype,
-                    h->d_err, h->d_partial, h->d_out, h->d_work[0], h->d_work[1], h->d_work[2],
+                    h->d_err, h->d_partial, h->d_counter, h->d_work[0], h->d_work[1], h->d_work[2],
                     h->d_fegeom, h->d_fdsharp, h->d_ngeom, h->d_evol, h->d_eqA, h->d_fnj,
                     h->d_fwsh, h->d_fiw};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
-    if (h->h_out) (void)hipHostFree(h->h_out);
+    if (h->h_res) (void)hipHostFree(h->h_res);
 }
 
 int bytes_of(const flou_hip_handle* h) { return h->prec == FLOU_HIP_FP64 ? 8 : 4; }
@@ -332,6 +336,28 @@ int launch_stage(flou_hip_handle* h, int mode, int first, double dt, double A, d
         e = h->l32(a, h->stream);
     }
     if (e != hipSuccess) return fail(h, FLOU_HIP_EDEVICE, std::string("kernel launch: ") + hipGetErrorString(e));
+    return FLOU_HIP_OK;
+}
+
+// Output block of the handle's next reduction (or flag read).
+ReduceOut next_out(flou_hip_handle* h) {
+    return ReduceOut{h->h_res, ++h->seq, h->d_partial, h->d_counter, h->d_err};
+}
+
+// Waits until the kernel that was handed next_out() has written its result.  Its last block
+// writes to pinned memory, so the host sees the result a few microseconds before the stream
+// reports its end; after 2 ms of looking, and to learn of failures, the stream is
+// synchronised instead.
+int await_result(flou_hip_handle* h) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int k = 1;; ++k) {
+        if (__atomic_load_n(&h->h_res->seq, __ATOMIC_ACQUIRE) == h->seq) return FLOU_HIP_OK;
+        __builtin_ia32_pause();
+        if (k % 64 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
+    }
+    HIPCHECK(h, hipStreamSynchronize(h->stream));
+    if (__atomic_load_n(&h->h_res->seq, __ATOMIC_ACQUIRE) != h->seq)
+        return fail(h, FLOU_HIP_EDEVICE, "the reduction's result did not arrive");
     return FLOU_HIP_OK;
 }
 
@@ -574,6 +600,8 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
     }
 
     // reductions: Δx per element and quadrature weights (FP64)
+    h->uniform_dx = std::adjacent_find(d->elem_volume, d->elem_volume + ne, std::not_equal_to<double>()) ==
+                    d->elem_volume + ne;
     std::vector<double> dxe(ne), jac(h->curved ? 0 : ne), w(h->npe);
     for (int64_t e = 0; e < ne; ++e) {
         double dx = d->elem_volume[e] / h->npe;
@@ -781,10 +809,12 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
     if (rc) return bad(FLOU_HIP_ENOMEM, "device upload failed: " + h->err);
     if (hipMalloc((void**)&h->d_err, sizeof(int)) != hipSuccess ||
         hipMalloc((void**)&h->d_partial, reduce_max_blocks() * sizeof(double)) != hipSuccess ||
-        hipMalloc((void**)&h->d_out, 4 * sizeof(double)) != hipSuccess ||
-        hipHostMalloc((void**)&h->h_out, 4 * sizeof(double), hipHostMallocDefault) != hipSuccess)
+        hipMalloc((void**)&h->d_counter, sizeof(unsigned)) != hipSuccess ||
+        hipHostMalloc((void**)&h->h_res, sizeof(HostResult), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
         return bad(FLOU_HIP_ENOMEM, "device allocation failed");
-    if (hipMemset(h->d_err, 0, sizeof(int)) != hipSuccess) return bad(FLOU_HIP_EDEVICE, "hipMemset failed");
+    std::memset(h->h_res, 0, sizeof(HostResult));
+    if (hipMemset(h->d_err, 0, sizeof(int)) != hipSuccess || hipMemset(h->d_counter, 0, sizeof(unsigned)) != hipSuccess)
+        return bad(FLOU_HIP_EDEVICE, "hipMemset failed");
     *out = h;
     return FLOU_HIP_OK;
 }
@@ -932,18 +962,19 @@ int flou_hip_monitor(flou_hip_handle* h, const void* Q, int32_t kind, double* ou
     if (h->eq != FLOU_HIP_EULER) return fail(h, FLOU_HIP_EUNSUPPORTED, "the monitors need the Euler equations");
     if (kind != FLOU_HIP_MONITOR_KINETIC_ENERGY && kind != FLOU_HIP_MONITOR_ENTROPY)
         return fail(h, FLOU_HIP_EINVAL, "Unknown monitor");
+    const ReduceOut r = next_out(h);
     hipError_t e;
     if (h->prec == FLOU_HIP_FP64)
-        e = launch_monitor<double>((const double*)Q, h->ndofs, h->int_npe, h->nd, h->gamma, kind, h->d_jac,
-                                   h->d_w, h->d_partial, reduce_max_blocks(), h->d_out, h->d_err, h->stream);
+        e = launch_monitor<double>((const double*)Q, h->ndofs, h->int_npe, h->nd, h->gamma, kind, h->d_jac, h->d_w, r,
+                                   h->stream);
     else
-        e = launch_monitor<float>((const float*)Q, h->ndofs, h->int_npe, h->nd, h->gamma, kind, h->d_jac,
-                                  h->d_w, h->d_partial, reduce_max_blocks(), h->d_out, h->d_err, h->stream);
+        e = launch_monitor<float>((const float*)Q, h->ndofs, h->int_npe, h->nd, h->gamma, kind, h->d_jac, h->d_w, r,
+                                  h->stream);
     if (e != hipSuccess) return fail(h, FLOU_HIP_EDEVICE, hipGetErrorString(e));
-    HIPCHECK(h, hipMemcpyAsync(h->h_out, h->d_out, sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIPCHECK(h, hipStreamSynchronize(h->stream));
-    *out = h->h_out[0];
-    return flou_hip_check(h);
+    const int rc = await_result(h);
+    if (rc) return rc;
+    *out = h->h_res->value;
+    return h->h_res->flag ? flou_hip_check(h) : FLOU_HIP_OK;
 }
 
 int flou_hip_equispaced(flou_hip_handle* h, int32_t m, const double* node2eq, const void* Q, int32_t ncols,
@@ -1012,42 +1043,44 @@ int flou_hip_rk_stage(flou_hip_handle* h, int32_t scheme, int32_t stage, double 
 
 int flou_hip_max_dt(flou_hip_handle* h, const void* Q, double cfl, double* out) {
     if (!h || !Q || !out) return FLOU_HIP_EINVAL;
+    const ReduceOut r = next_out(h);
     hipError_t e;
     if (h->prec == FLOU_HIP_FP64)
-        e = launch_max_dt<double>((const double*)Q, h->ndofs, h->npe, h->nd, h->eq, h->gamma, h->anorm,
-                                  cfl, h->d_dxe, h->d_partial, h->d_out, h->d_err, h->stream);
+        e = launch_max_dt<double>((const double*)Q, h->ndofs, h->npe, h->nd, h->eq, h->gamma, h->anorm, cfl, h->d_dxe,
+                                  h->uniform_dx, r, h->stream);
     else
-        e = launch_max_dt<float>((const float*)Q, h->ndofs, h->npe, h->nd, h->eq, h->gamma, h->anorm,
-                                 cfl, h->d_dxe, h->d_partial, h->d_out, h->d_err, h->stream);
+        e = launch_max_dt<float>((const float*)Q, h->ndofs, h->npe, h->nd, h->eq, h->gamma, h->anorm, cfl, h->d_dxe,
+                                 h->uniform_dx, r, h->stream);
     if (e != hipSuccess) return fail(h, FLOU_HIP_EDEVICE, hipGetErrorString(e));
-    HIPCHECK(h, hipMemcpyAsync(h->h_out, h->d_out, sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIPCHECK(h, hipStreamSynchronize(h->stream));
-    *out = h->h_out[0];
-    return FLOU_HIP_OK;
+    const int rc = await_result(h);
+    if (!rc) *out = h->h_res->value;
+    return rc;
 }
 
 int flou_hip_integrate(flou_hip_handle* h, const void* Q, int32_t ivar, double* out) {
     if (!h || !Q || !out) return FLOU_HIP_EINVAL;
     if (ivar < 0 || ivar >= h->nv) return fail(h, FLOU_HIP_EINVAL, "ivar out of range");
+    const ReduceOut r = next_out(h);
     hipError_t e;
     if (h->prec == FLOU_HIP_FP64)
-        e = launch_integrate<double>((const double*)Q + (int64_t)ivar * h->ndofs, h->ndofs, h->int_npe,
-                                     h->d_jac, h->d_w, h->d_partial, h->d_out, h->stream);
+        e = launch_integrate<double>((const double*)Q + (int64_t)ivar * h->ndofs, h->ndofs, h->int_npe, h->d_jac,
+                                     h->d_w, r, h->stream);
     else
-        e = launch_integrate<float>((const float*)Q + (int64_t)ivar * h->ndofs, h->ndofs, h->int_npe,
-                                    h->d_jac, h->d_w, h->d_partial, h->d_out, h->stream);
+        e = launch_integrate<float>((const float*)Q + (int64_t)ivar * h->ndofs, h->ndofs, h->int_npe, h->d_jac,
+                                    h->d_w, r, h->stream);
     if (e != hipSuccess) return fail(h, FLOU_HIP_EDEVICE, hipGetErrorString(e));
-    HIPCHECK(h, hipMemcpyAsync(h->h_out, h->d_out, sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIPCHECK(h, hipStreamSynchronize(h->stream));
-    *out = h->h_out[0];
-    return FLOU_HIP_OK;
+    const int rc = await_result(h);
+    if (!rc) *out = h->h_res->value;
+    return rc;
 }
 
 int flou_hip_check(flou_hip_handle* h) {
     if (!h) return FLOU_HIP_EINVAL;
-    int flag = 0;
-    HIPCHECK(h, hipMemcpyAsync(&flag, h->d_err, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-    HIPCHECK(h, hipStreamSynchronize(h->stream));
+    const hipError_t e = launch_flag(next_out(h), h->stream);
+    if (e != hipSuccess) return fail(h, FLOU_HIP_EDEVICE, hipGetErrorString(e));
+    const int rc = await_result(h);
+    if (rc) return rc;
+    const int flag = h->h_res->flag;
     if (flag) {
         HIPCHECK(h, hipMemsetAsync(h->d_err, 0, sizeof(int), h->stream));
         HIPCHECK(h, hipStreamSynchronize(h->stream));
@@ -1059,9 +1092,11 @@ int flou_hip_check(flou_hip_handle* h) {
     return FLOU_HIP_OK;
 }
 
-int flou_hip_timeintegrate(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t nsteps,
-                           double cfl, double* t_inout) {
-    if (!h || !Q || nsteps < 0) return FLOU_HIP_EINVAL;
+namespace {
+// The time loop of flou_hip_timeintegrate: nsteps steps of dt (the CFL step at most dt), or,
+// with until, steps of at most dt until *t reaches tfinal.
+int time_loop(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t nsteps, bool until, double tfinal,
+              double cfl, double* t_inout) {
     if (scheme < FLOU_HIP_SSPRK33 || scheme > FLOU_HIP_ORK256) return fail(h, FLOU_HIP_EINVAL, "unknown scheme");
     if (!(dt > 0.0)) return fail(h, FLOU_HIP_EINVAL, "dt must be positive");
     const size_t bytes = flou_hip_state_bytes(h);
@@ -1073,13 +1108,15 @@ int flou_hip_timeintegrate(flou_hip_handle* h, int32_t scheme, void* Q, double d
     void* cur = Q;
     void* oth = h->d_work[0];
     int rc = 0;
-    for (int64_t step = 0; step < nsteps && !rc; ++step) {
-        double dts = dt;
+    for (int64_t step = 0; (until ? t < tfinal * (1 - 1e-14) : step < nsteps) && !rc; ++step) {
+        double dts = until ? std::min(dt, tfinal - t) : dt;
         if (cfl > 0.0) {
             double m;
             rc = flou_hip_max_dt(h, cur, cfl, &m);
             if (rc) break;
-            dts = std::min(m, dt);
+            // a non-physical state of the step before: the check below reports it
+            if (until && step && h->h_res->flag) break;
+            dts = std::min(m, dts);
         }
         if (scheme == FLOU_HIP_SSPRK33) {
             rc = flou_hip_rk_stage(h, scheme, 0, dts, t, Q, nullptr, nullptr, h->d_work[0]);
@@ -1097,6 +1134,20 @@ int flou_hip_timeintegrate(flou_hip_handle* h, int32_t scheme, void* Q, double d
     if (cur != Q) HIPCHECK(h, hipMemcpyAsync(Q, cur, bytes, hipMemcpyDeviceToDevice, h->stream));
     if (t_inout) *t_inout = t;
     return flou_hip_check(h);
+}
+}  // namespace
+
+int flou_hip_timeintegrate(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t nsteps,
+                           double cfl, double* t_inout) {
+    if (!h || !Q || nsteps < 0) return FLOU_HIP_EINVAL;
+    return time_loop(h, scheme, Q, dt, nsteps, false, 0.0, cfl, t_inout);
+}
+
+int flou_hip_timeintegrate_until(flou_hip_handle* h, int32_t scheme, void* Q, double dt, double tfinal, double cfl,
+                                 double* t_inout) {
+    if (!h || !Q || !t_inout) return FLOU_HIP_EINVAL;
+    if (!(*t_inout < tfinal * (1 - 1e-14))) return FLOU_HIP_OK;  // nothing to do
+    return time_loop(h, scheme, Q, dt, 0, true, tfinal, cfl, t_inout);
 }
 
 int flou_hip_rhs_vjp(flou_hip_handle* h, const void* Q, const void* dQbar, void* Qbar) {

@@ -1,17 +1,14 @@
-// Stage limiter and monitors of the Euler path (Equations/Euler.jl:541-654).
+// Stage limiter of the Euler path (Equations/Euler.jl:596-654).
 //
 // k_zhang_shu: Flou's Zhang & Shu positivity limiter.  Element means and minima are
 // sequential folds over the element's nodes (the reference's order), so the FP64 result is
 // reproducible bit for bit.
-// k_monitor: Σ Jω · s(Q) with s the kinetic energy or the mathematical entropy, FP64
-// accumulation, block partials + one finishing block (fixed tree, deterministic).
 #include "common.hpp"
 #include "reduce.hpp"
 
 namespace flouhip {
 
 static constexpr int LB = 256;  // limiter block
-static constexpr int MB = 256;  // monitor block
 
 // Elements per limiter block, the LDS stride of an element's nodes (odd: the folds' lanes,
 // one element apart, then read distinct banks) and the block's LDS values.
@@ -114,63 +111,6 @@ __global__ void __launch_bounds__(LB) k_zhang_shu(T* __restrict__ Q, int64_t ndo
     }
 }
 
-__device__ inline double mwarp_sum(double x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-    return x;
-}
-
-template <typename T>
-__global__ void __launch_bounds__(MB) k_monitor(const T* __restrict__ Q, int64_t ndofs, int wnpe, int nd,
-                                               double gamma, int kind, const double* __restrict__ jac,
-                                               const double* __restrict__ w, double* __restrict__ partial,
-                                               int* err) {
-    double s = 0.0;
-    for (int64_t i = (int64_t)blockIdx.x * MB + threadIdx.x; i < ndofs; i += (int64_t)gridDim.x * MB) {
-        double q[5];
-        for (int v = 0; v < nd + 2; ++v) q[v] = (double)Q[v * ndofs + i];
-        double m2 = q[1] * q[1];
-        for (int k = 1; k < nd; ++k) m2 = m2 + q[1 + k] * q[1 + k];
-        double val;
-        if (kind == 0) {
-            val = m2 / (2.0 * q[0]);
-        } else {
-            const double p = (gamma - 1.0) * (q[nd + 1] - m2 / (2.0 * q[0]));
-            if (p < 0.0 || q[0] < 0.0) atomicOr(err, ERR_LOG_NEG);
-            const double ent = log(p) - gamma * log(q[0]);
-            val = -(q[0] * ent) / (gamma - 1.0);
-        }
-        const int64_t k = i / wnpe;
-        s += (jac[k] * w[i - k * wnpe]) * val;
-    }
-    __shared__ double sh[MB / 64];
-    s = mwarp_sum(s);
-    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
-    if (l == 0) sh[wv] = s;
-    __syncthreads();
-    if (wv == 0) {
-        s = l < MB / 64 ? sh[l] : 0.0;
-        s = mwarp_sum(s);
-        if (l == 0) partial[blockIdx.x] = s;
-    }
-}
-
-__global__ void __launch_bounds__(MB) k_monitor_finish(const double* __restrict__ partial, int n,
-                                                      double* __restrict__ out) {
-    double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += MB) s += partial[i];
-    __shared__ double sh[MB / 64];
-    s = mwarp_sum(s);
-    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
-    if (l == 0) sh[wv] = s;
-    __syncthreads();
-    if (wv == 0) {
-        s = l < MB / 64 ? sh[l] : 0.0;
-        s = mwarp_sum(s);
-        if (l == 0) *out = s;
-    }
-}
-
 template <typename T>
 hipError_t launch_zhang_shu(T* Q, int64_t ndofs, int64_t ne, int npe, int nd, int wnpe,
                             const double* jac, const double* w, const double* vol, double minval,
@@ -187,26 +127,9 @@ hipError_t launch_zhang_shu(T* Q, int64_t ndofs, int64_t ne, int npe, int nd, in
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_monitor(const T* Q, int64_t ndofs, int wnpe, int nd, double gamma, int kind,
-                          const double* jac, const double* w, double* partial, int max_blocks,
-                          double* out, int* err, hipStream_t s) {
-    int64_t g = (ndofs + MB - 1) / MB;
-    if (g > max_blocks) g = max_blocks;
-    if (g < 1) g = 1;
-    hipLaunchKernelGGL(k_monitor<T>, dim3((int)g), dim3(MB), 0, s, Q, ndofs, wnpe, nd, gamma, kind, jac, w,
-                       partial, err);
-    hipLaunchKernelGGL(k_monitor_finish, dim3(1), dim3(MB), 0, s, partial, (int)g, out);
-    return hipGetLastError();
-}
-
 template hipError_t launch_zhang_shu<double>(double*, int64_t, int64_t, int, int, int, const double*,
                                              const double*, const double*, double, double, hipStream_t);
 template hipError_t launch_zhang_shu<float>(float*, int64_t, int64_t, int, int, int, const double*,
                                             const double*, const double*, double, double, hipStream_t);
-template hipError_t launch_monitor<double>(const double*, int64_t, int, int, double, int, const double*,
-                                           const double*, double*, int, double*, int*, hipStream_t);
-template hipError_t launch_monitor<float>(const float*, int64_t, int, int, double, int, const double*,
-                                          const double*, double*, int, double*, int*, hipStream_t);
 
 }  // namespace flouhip

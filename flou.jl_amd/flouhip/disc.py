@@ -413,10 +413,8 @@ def _timeintegrate(Q0, disc, code, tfinal, dt, cfl, t0):
             C.check(C.lib.flou_hip_timeintegrate(disc.h, code, ptr, float(rest), 1, 0.0,
                                                  ctypes.byref(t)), disc.h, "timeintegrate")
     else:
-        while t.value < float(tfinal) * (1 - 1e-14):
-            step = min(float(dt), float(tfinal) - t.value)
-            C.check(C.lib.flou_hip_timeintegrate(disc.h, code, ptr, step, 1, float(cfl),
-                                                 ctypes.byref(t)), disc.h, "timeintegrate")
+        C.check(C.lib.flou_hip_timeintegrate_until(disc.h, code, ptr, float(dt), float(tfinal), float(cfl),
+                                                   ctypes.byref(t)), disc.h, "timeintegrate")
     torch.cuda.synchronize()
     return Q0, time.perf_counter() - tic
 

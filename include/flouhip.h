@@ -212,6 +212,13 @@ int flou_hip_rk_stage(flou_hip_handle* h, int32_t scheme, int32_t stage, double 
 int flou_hip_timeintegrate(flou_hip_handle* h, int32_t scheme, void* Q, double dt,
                            int64_t nsteps, double cfl, double* t_inout);
 
+/* The CFL-controlled loop of timeintegrate up to tfinal (FlouTime.jl:34-56, 92-104), in place
+ * on Q: before every step dt_step = min(get_max_dt(Q, cfl), dt, tfinal - t), from *t_inout
+ * until t >= tfinal (1 - 1e-14); with cfl <= 0 the steps are min(dt, tfinal - t).  Returns FLOU_HIP_EDOMAIN once a
+ * step met a non-physical state; later steps are not taken. */
+int flou_hip_timeintegrate_until(flou_hip_handle* h, int32_t scheme, void* Q, double dt,
+                                 double tfinal, double cfl, double* t_inout);
+
 /* get_max_dt(Q, disc, eq, cfl) -- MultielementDiscontinuous.jl:162-178 (FP64 result). */
 int flou_hip_max_dt(flou_hip_handle* h, const void* Q, double cfl, double* out);
 

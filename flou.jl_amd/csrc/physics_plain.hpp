@@ -193,11 +193,23 @@ __device__ inline void twopointflux(const T* Q1, const T* Q2, const T* P1, const
     }
 }
 
-// Node values that pair_flux reads (slots): ρ, u.. and the flux's scalars: Chandrasekhar β; Kennedy-Gruber p and
-// E/ρ; StdAverage p, m.. and E.
+// Node values that pair_flux reads (slots), halved where the flux takes the mean of the two
+// nodes: a mean is then one addition, and scaling by powers of two commutes with every
+// rounding.  Chandrasekhar: ρ/2, u/2.., β; Kennedy-Gruber: ρ/2, u/2.., p/2, E/(2ρ);
+// StdAverage: u.., p/2, (ρu)/2.., E/2.
 template <int ND, int TP>
 constexpr int tp_slots() {
-    return TP == TP_CHANDRASEKHAR ? ND + 2 : (TP == TP_KENNEDY_GRUBER ? ND + 3 : 2 * ND + 3);
+    return TP == TP_CHANDRASEKHAR ? ND + 2 : (TP == TP_KENNEDY_GRUBER ? ND + 3 : 2 * ND + 2);
+}
+
+// Logarithmic mean of a/2 and b/2 from their ratio's F: (a + b)/(2F) with hs = (a + b)/2.
+template <typename T>
+__device__ inline T logmean_factor(T al, T ar, int* err) {
+    const T xi = xdiv(al, ar);
+    const T f = xdiv(xi - T(1), xi + T(1));
+    const T u = f * f;
+    if (u < T(0.01)) return ((T(1) + cdiv<3>(u)) + cdiv<5>(u * u)) + cdiv<7>((u * u) * u);
+    return xdiv(dlog(xi, err), T(2) * f);
 }
 
 // Component DIR of the two-point flux between the lower (1) and higher (2) line position
@@ -206,34 +218,33 @@ template <typename T, int ND, int TP, int DIR>
 __device__ __forceinline__ void pair_flux(const T* A, const T* B, T ja, T gm1, int* err, T* F) {
     T f[ND + 2];
     if constexpr (TP == TP_STDAVG) {
-        // slots: ρ, u.., p, m.., E
-        const T p1 = A[ND + 1], p2 = B[ND + 1];
-        const T* m1 = A + ND + 2;
-        const T* m2 = B + ND + 2;
-        f[0] = (m1[DIR] + m2[DIR]) / T(2);
+        const T p1 = A[ND], p2 = B[ND];
+        const T* m1 = A + ND + 1;
+        const T* m2 = B + ND + 1;
+        f[0] = m1[DIR] + m2[DIR];
 #pragma unroll
         for (int c = 0; c < ND; ++c) {
-            T s = m1[c] * A[1 + DIR];
+            T s = m1[c] * A[DIR];
             if (c == DIR) s = s + p1;
-            s = s + m2[c] * B[1 + DIR];
+            s = s + m2[c] * B[DIR];
             if (c == DIR) s = s + p2;
-            f[1 + c] = s / T(2);
+            f[1 + c] = s;
         }
-        f[ND + 1] = ((m1[ND] + p1) * A[1 + DIR] + (m2[ND] + p2) * B[1 + DIR]) / T(2);
+        f[ND + 1] = (m1[ND] + p1) * A[DIR] + (m2[ND] + p2) * B[DIR];
     } else if constexpr (TP == TP_CHANDRASEKHAR) {
-        const T rho1 = A[0], rho2 = B[0], b1 = A[ND + 1], b2 = B[ND + 1];
         T um[ND];
 #pragma unroll
-        for (int k = 0; k < ND; ++k) um[k] = (A[1 + k] + B[1 + k]) / T(2);
-        const T rho = logarithmic_mean(rho1, rho2, err);
-        const T p = xdiv(rho1 + rho2, T(2) * (b1 + b2));
-        const T beta = logarithmic_mean(b1, b2, err);
-        T sq = A[1] * A[1];
+        for (int k = 0; k < ND; ++k) um[k] = A[1 + k] + B[1 + k];
+        const T hs = A[0] + B[0], sb = A[ND + 1] + B[ND + 1];
+        const T rho = xdiv(hs, logmean_factor(A[0], B[0], err));
+        const T p = xdiv(hs, sb);
+        const T beta2 = xdiv(sb, logmean_factor(A[ND + 1], B[ND + 1], err));  // 2β̂
+        T sq = A[1] * A[1];  // (|u1|² + |u2|²)/4
 #pragma unroll
         for (int k = 1; k < ND; ++k) sq = sq + A[1 + k] * A[1 + k];
 #pragma unroll
         for (int k = 0; k < ND; ++k) sq = sq + B[1 + k] * B[1 + k];
-        T h = xdiv(T(1), (T(2) * beta) * gm1) - sq / T(4);
+        T h = xdiv(T(1), beta2 * gm1) - sq;
         h = h + xdiv(p, rho);
 #pragma unroll
         for (int k = 0; k < ND; ++k) h = h + um[k] * um[k];
@@ -245,17 +256,12 @@ __device__ __forceinline__ void pair_flux(const T* A, const T* B, T ja, T gm1, i
         }
         f[ND + 1] = (rho * um[DIR]) * h;
     } else {
-        const T rho = (A[0] + B[0]) / T(2);
-        const T p = (A[ND + 1] + B[ND + 1]) / T(2);
-        const T e = (A[ND + 2] + B[ND + 2]) / T(2);
-        const T ud = (A[1 + DIR] + B[1 + DIR]) / T(2);
+        const T rho = A[0] + B[0], p = A[ND + 1] + B[ND + 1], e = A[ND + 2] + B[ND + 2];
+        const T ud = A[1 + DIR] + B[1 + DIR];
         const T m = rho * ud;
         f[0] = m;
 #pragma unroll
-        for (int c = 0; c < ND; ++c) {
-            if (c == DIR) f[1 + c] = m * ud + p;
-            else f[1 + c] = m * ((A[1 + c] + B[1 + c]) / T(2));
-        }
+        for (int c = 0; c < ND; ++c) f[1 + c] = c == DIR ? m * ud + p : m * (A[1 + c] + B[1 + c]);
         f[ND + 1] = m * e + p * ud;
     }
 #pragma unroll
@@ -263,21 +269,27 @@ __device__ __forceinline__ void pair_flux(const T* A, const T* B, T ja, T gm1, i
 }
 
 // The slots of a node (see tp_slots) in an array of stride S; CONS false: without the
-// conservative ones of StdAverage (m.., E).
+// conservative ones of StdAverage.
 template <typename T, int ND, int TP, int S, bool CONS = true>
 __device__ __forceinline__ void put_slots(T* s, const T* q, const T* P, const Recip<T>& ir) {
-    s[0] = q[0];
+    constexpr T H = T(0.5);
+    if constexpr (TP == TP_STDAVG) {
 #pragma unroll
-    for (int k = 0; k < ND; ++k) s[(1 + k) * S] = P[1 + k];
-    if constexpr (TP == TP_CHANDRASEKHAR) {
-        s[(ND + 1) * S] = tp_scalar<T, ND, TP>(q, P, ir);
+        for (int k = 0; k < ND; ++k) s[k * S] = P[1 + k];
+        s[ND * S] = H * P[ND + 1];
+        if constexpr (CONS) {
+#pragma unroll
+            for (int c = 0; c <= ND; ++c) s[(ND + 1 + c) * S] = H * q[1 + c];
+        }
     } else {
-        s[(ND + 1) * S] = P[ND + 1];
-        if constexpr (TP == TP_KENNEDY_GRUBER) {
-            s[(ND + 2) * S] = tp_scalar<T, ND, TP>(q, P, ir);
-        } else if constexpr (CONS) {
+        s[0] = H * q[0];
 #pragma unroll
-            for (int c = 0; c <= ND; ++c) s[(ND + 2 + c) * S] = q[1 + c];
+        for (int k = 0; k < ND; ++k) s[(1 + k) * S] = H * P[1 + k];
+        if constexpr (TP == TP_CHANDRASEKHAR) {
+            s[(ND + 1) * S] = tp_scalar<T, ND, TP>(q, P, ir);
+        } else {
+            s[(ND + 1) * S] = H * P[ND + 1];
+            s[(ND + 2) * S] = H * tp_scalar<T, ND, TP>(q, P, ir);
         }
     }
 }

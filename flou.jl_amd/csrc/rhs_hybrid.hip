@@ -41,7 +41,7 @@ struct HCfg {
 // Flux input slots held beside the conservative states.
 template <int ND, int TP>
 constexpr int lds_slots() {
-    return TP == TP_STDAVG ? ND + 2 : plain::tp_slots<ND, TP>();
+    return TP == TP_STDAVG ? ND + 1 : plain::tp_slots<ND, TP>();
 }
 
 // Both sides' states (and entropy variables) of an interface of direction DIR in the
@@ -78,23 +78,32 @@ __device__ __forceinline__ void direction(const RhsArgs<T>& a, const T* sS, cons
         T A[NS], B[NS], F[NV];
 #pragma unroll
         for (int c = 0; c < NS; ++c) {  // StdAverage's conservative slots lie in sQ
-            A[c] = c < NSL ? pa[c * NN] : sQ[(pa - sS) + (1 + c - NSL) * NN];
-            B[c] = c < NSL ? pb[c * NN] : sQ[(pb - sS) + (1 + c - NSL) * NN];
+            A[c] = c < NSL ? pa[c * NN] : T(0.5) * sQ[(pa - sS) + (1 + c - NSL) * NN];
+            B[c] = c < NSL ? pb[c * NN] : T(0.5) * sQ[(pb - sS) + (1 + c - NSL) * NN];
         }
         if constexpr (DIAG) {
             plain::pair_flux<T, ND, TP, DIR>(A, B, sM[DIR * (ND + 1)], gm1, a.errflag, F);
         } else {
-            // the general form takes conservative and primitive states
+            // the general form takes conservative and primitive states (whole, not halved)
             T qa[NV], qb[NV], Pa[NV], Pb[NV];
             const T* ca = sQ + (pa - sS);
             const T* cb = sQ + (pb - sS);
+            constexpr bool SD = TP == TP_STDAVG;
+            constexpr int SC = TP == TP_KENNEDY_GRUBER ? ND + 2 : ND + 1;
+            const T sa = TP == TP_KENNEDY_GRUBER ? T(2) * A[SC] : A[SC], sb = TP == TP_KENNEDY_GRUBER ? T(2) * B[SC] : B[SC];
 #pragma unroll
             for (int v = 0; v < NV; ++v) { qa[v] = ca[v * NN]; qb[v] = cb[v * NN]; }
+            Pa[0] = qa[0];
+            Pb[0] = qb[0];
 #pragma unroll
-            for (int v = 0; v < NV; ++v) { Pa[v] = A[v]; Pb[v] = B[v]; }  // slot ND+1: p (Chandrasekhar: unread)
-            constexpr int SC = TP == TP_CHANDRASEKHAR ? ND + 1 : (TP == TP_KENNEDY_GRUBER ? ND + 2 : 0);
-            plain::twopointflux<T, ND, EQ_EULER, TP>(qa, qb, Pa, Pb, A[SC], B[SC], sM + ND * DIR, sM + ND * DIR,
-                                                     a.gamma, avel, a.errflag, F);
+            for (int k = 0; k < ND; ++k) {
+                Pa[1 + k] = SD ? A[k] : T(2) * A[1 + k];
+                Pb[1 + k] = SD ? B[k] : T(2) * B[1 + k];
+            }
+            Pa[ND + 1] = T(2) * (SD ? A[ND] : A[ND + 1]);  // p (Chandrasekhar: unread)
+            Pb[ND + 1] = T(2) * (SD ? B[ND] : B[ND + 1]);
+            plain::twopointflux<T, ND, EQ_EULER, TP>(qa, qb, Pa, Pb, sa, sb, sM + ND * DIR, sM + ND * DIR, a.gamma,
+                                                     avel, a.errflag, F);
         }
 #pragma unroll
         for (int v = 0; v < NV; ++v) sTab[k * NV + v] = F[v];

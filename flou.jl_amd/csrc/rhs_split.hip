@@ -3,21 +3,25 @@
 // kernel's arithmetic (rhs_plain.hip, reference order, every value rounded where the
 // reference rounds it) without the work that this geometry makes void.
 //
-// What bounds it: FP64 VALU issue.  k_plain<double, 3, 6, ..> spends about 4000 VALU slots
-// per node, most of them on divisions, on the two components of every flux that a diagonal
-// metric multiplies by zero, and on rotations by 0 and ±1.  Measured against it (same bits):
-// 3-D N=5, 10.5 M nodes, Chandrasekhar: 1.65 -> 0.99 ms per CK2N54 stage (0.97 -> 1.6 TB/s of
-// algorithmic bytes); 2-D N=5, 0.59 M nodes: 66 -> 47 us.  With the same results:
+// What bounds it: FP64 arithmetic, by issue (90 % of busy cycles) and by the clock the power
+// limit leaves under it (1.8 to 2.0 of 2.4 GHz).  k_plain<double, 3, 6, ..> spends about 4000
+// VALU slots per node, most of them on divisions, on the two components of every flux that a
+// diagonal metric multiplies by zero, and on rotations by 0 and ±1.  Measured against it (same
+// bits): 3-D N=5, 10.5 M nodes, Chandrasekhar: 1.65 -> 0.96 ms per CK2N54 stage; 2-D N=5, 0.59 M
+// nodes: 66 -> 43 us.  With the same results:
 //   * only the flux component along the line's direction is formed: f·n̄ has one term, the
 //     others are exact zeros.  The direction is a compile-time constant of each phase;
+//   * flux inputs are staged halved, so that means are one addition (pair_flux);
+//   * a node's own contravariant flux goes into the same table as the pairs, so that its row
+//     reads N entries without a case for the diagonal, at offsets that advance by constants
+//     (2504 -> 2186 VALU per wave at 3-D N=5 with the above, 0.99 -> 0.96 ms);
 //   * face states are read in the order (normal, transverse..) of the face frame by index,
 //     n = ±e_d, t = ±e_{d+1}, b = ±e_{d+2}: signs of the transverse axes commute with every
 //     rounding of the LxF and StdAverage fluxes, so they need not be applied;
-//   * quotients share reciprocals (exact_div.hpp), the diagonal contravariant flux reuses
-//     the staged primitives, the lift touches the end nodes only (∂g is exactly zero
-//     elsewhere);
-//   * the pair table of one direction lies over the staged conservative states, which are
-//     dead after the face fluxes; a thread keeps its own node's state in registers.
+//   * quotients share reciprocals (exact_div.hpp), the node's contravariant flux reuses its
+//     primitives, the lift touches the end nodes only (∂g is exactly zero elsewhere);
+//   * the face fluxes come last and lie over the dead table (39 KB of LDS at 3-D N=5, 4 waves
+//     per SIMD); their neighbour traces are loaded before the last direction's rows.
 // One thread per node (blocks rounded up to whole waves, the spare lanes take pairs), pairs
 // pair-major: consecutive lanes evaluate the same pair of consecutive lines, so node reads
 // and table writes are conflict-light and the pair's positions nearly uniform.
@@ -40,20 +44,31 @@ struct SCfg {
     static constexpr int NL = EPB * NPF;                 // lines per block and direction
 };
 
-// One direction: the pair table, then every node's D♯ row over it in the order j = 0..N-1
-// (diagonal: the contravariant flux), then this node's face terms are left to the caller.
-template <int ND, int N, int TP, int DIR>
-__device__ __forceinline__ void direction(const RhsArgs<double>& a, const double* sS, double* sPair, const double* sD,
+// One direction: every pair flux and every node's contravariant flux (the diagonal entry of
+// F♯) into the table, then after a barrier (before which LOADS may issue global loads) every
+// node's D♯ row over it in the order j = 0..N-1.
+template <int ND, int N, int TP, int DIR, typename LOADS>
+__device__ __forceinline__ void direction(const RhsArgs<double>& a, const double* sS, double* sTab, const double* sD,
                                           const double* sG, int nel, int tid, int le, int node, bool valid,
-                                          const double (&q)[ND + 2], const double (&u)[ND], double p,
+                                          const double (&q)[ND + 2], const double (&u)[ND], double p, LOADS loads,
                                           double (&acc)[ND + 2]) {
     using C = SCfg<ND, N>;
-    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NN = C::NN, NS = plain::tp_slots<ND, TP>();
+    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NN = C::NN, NL = C::NL, NS = plain::tp_slots<ND, TP>();
     const double gm1 = a.gamma - 1.0;
-    __syncthreads();  // the table's memory has been read (the previous direction, or the own traces)
+    int lf, ii;
+    node_line<ND, N>(node, DIR, lf, ii);
+    if (valid) {
+        // contravariant flux along DIR (plain::contravariant_flux, diagonal metric)
+        const double ja = sG[le * (ND + 1) + DIR];
+        double* t = sTab + (C::NPR + tid) * NV;
+        t[0] = q[1 + DIR] * ja;
+#pragma unroll
+        for (int c = 0; c < ND; ++c) t[1 + c] = (c == DIR ? q[1 + DIR] * u[c] + p : q[1 + DIR] * u[c]) * ja;
+        t[NV - 1] = ((q[NV - 1] + p) * u[DIR]) * ja;
+    }
 #pragma unroll 1
     for (int k = tid; k < C::NPR; k += C::TPB) {
-        const int pr = k / C::NL, l = k - pr * C::NL;
+        const int pr = k / NL, l = k - pr * NL;
         const int le2 = C::EPB == 1 ? 0 : l / NPF, f = l - le2 * NPF;
         if (le2 >= nel) continue;
         const int ab = pair_ab<N>(pr);
@@ -66,33 +81,25 @@ __device__ __forceinline__ void direction(const RhsArgs<double>& a, const double
         for (int c = 0; c < NS; ++c) { A[c] = pa[c * NN]; B[c] = pb[c * NN]; }
         plain::pair_flux<double, ND, TP, DIR>(A, B, sG[le2 * (ND + 1) + DIR], gm1, a.errflag, F);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) sPair[k * NV + v] = F[v];
+        for (int v = 0; v < NV; ++v) sTab[k * NV + v] = F[v];
     }
+    loads();
     __syncthreads();
     if (valid) {
-        int f, ii;
-        node_line<ND, N>(node, DIR, f, ii);
-        const double ja = sG[le * (ND + 1) + DIR];
-        // contravariant flux of the node along DIR (plain::contravariant_flux, diagonal metric)
-        double Fd[NV];
-        Fd[0] = q[1 + DIR] * ja;
-#pragma unroll
-        for (int c = 0; c < ND; ++c) Fd[1 + c] = (c == DIR ? q[1 + DIR] * u[c] + p : q[1 + DIR] * u[c]) * ja;
-        Fd[NV - 1] = ((q[NV - 1] + p) * u[DIR]) * ja;
-        const int l = le * NPF + f;
+        // pair (j, ii) or (ii, j) of the node's line: pair index ii - 1 at j = 0, then N - j - 2
+        // further for each j < ii and 1 further from there (the place of j = ii is skipped over)
+        const int diag = (C::NPR + tid) * NV;
+        int off = ((ii - 1) * NL + le * NPF + lf) * NV;
 #pragma unroll
         for (int j = 0; j < N; ++j) {
+            const double* t = sTab + (j == ii ? diag : off);
             const double Dij = sD[ii * N + j];
-            const int lo = j < ii ? j : ii, hi = j < ii ? ii : j;
-            const int pr = j == ii ? 0 : lo * (2 * N - lo - 1) / 2 + (hi - lo - 1);
-            const double* t = sPair + (pr * C::NL + l) * NV;
 #pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                const double F = j == ii ? Fd[v] : t[v];
-                acc[v] = acc[v] - Dij * F;
-            }
+            for (int v = 0; v < NV; ++v) acc[v] = acc[v] - Dij * t[v];
+            off += (j < ii ? N - j - 2 : 1) * (NL * NV);
         }
     }
+    __syncthreads();  // the table has been read
 }
 
 template <int ND, int N, int TP>
@@ -101,22 +108,21 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split(const RhsArgs<doub
     using C = SCfg<ND, N>;
     constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, EPB = C::EPB, TPB = C::TPB, NN = C::NN;
     constexpr int NS = plain::tp_slots<ND, TP>();
-    constexpr int UN = NV * (NN > C::NPR ? NN : C::NPR);
-    __shared__ T sS[NS * NN];          // two-point flux inputs, [slot][node]
-    __shared__ T sU[UN];               // conservative states [v][node], then the pair table
-    __shared__ T sFn[EPB * NF * NV * NPF];
+    constexpr int NFN = EPB * NF * NPF;  // face nodes of the block
+    constexpr int TAB = C::NPR + NN, FACE = NN + NFN;
+    __shared__ T sS[NS * NN];                          // two-point flux inputs, [slot][node]
+    __shared__ T sTab[NV * (TAB > FACE ? TAB : FACE)];  // pair and node fluxes of one direction, then
+                                                       // conservative states [v][node] and face fluxes
     __shared__ T sD[N * N];
-    __shared__ T sG[EPB * (ND + 1)];   // Ja_dd and J per element
+    __shared__ T sG[EPB * (ND + 1)];                   // Ja_dd and J per element
 
     const int tid = threadIdx.x;
     const int e0 = xcd_remap(blockIdx.x, gridDim.x) * EPB;
     const int64_t Nd = a.ndofs;
     const int nel = a.ne - e0 < EPB ? a.ne - e0 : EPB;
-    const int nnb = nel * NPE;         // nodes of this block
-    const T gamma = a.gamma, gm1 = a.gamma - 1.0;
+    const T gamma = a.gamma;
 
-    // ---- loads: face tables, own node, neighbour trace, epilogue operand, tables ----------
-    constexpr int NFN = EPB * NF * NPF;
+    // ---- own node, face tables, operators -----------------------------------------------
     const int fe = tid / (NF * NPF), fk = (tid - fe * (NF * NPF)) / NPF, ff = tid % NPF;
     const bool pf = tid < NFN && fe < nel;
     int pinfo = 0, pnb = -1, pfgi = 0;
@@ -126,41 +132,17 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split(const RhsArgs<doub
         pnb = a.nb[slot];
         pfgi = a.fgi[slot];
     }
-    const bool valid = tid < nnb;
+    const bool valid = tid < nel * NPE;
     const int le = tid / NPE, node = tid - le * NPE;
     const int64_t g0 = (int64_t)e0 * NPE;
     T q[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) q[v] = valid ? a.Q[v * Nd + g0 + tid] : T(1);
-    // a face node's states are read in the order ρ, normal and transverse momenta, E
-    T pext[NV];
-    if (pf && pnb >= 0) {
-        const int kp = finfo_nbpos(pinfo), dir = fk >> 1;
-        const T* Qn = a.Q + (int64_t)pnb * NPE + line_node<ND, N>(kp >> 1, ff, (kp & 1) ? N - 1 : 0);
-        pext[0] = Qn[0];
-#pragma unroll
-        for (int c = 0; c < ND; ++c) pext[1 + c] = Qn[(1 + (dir + c) % ND) * Nd];
-        pext[NV - 1] = Qn[(NV - 1) * Nd];
-    }
-    T pn = T(0), pj = T(0);
-    if (pf) {
-        const T* g = a.fgeom + (int64_t)pfgi * (3 * ND + 1);
-        pn = g[fk >> 1];
-        pj = g[3 * ND];
-    }
-    const T* aux = stage_aux(a);
-    T xv[NV];
-    if (aux && valid) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) xv[v] = aux[v * Nd + g0 + tid];
-    }
     for (int i = tid; i < N * N; i += TPB) sD[i] = a.ops[ops_Dsh(N) + i];
     for (int i = tid; i < EPB * (ND + 1); i += TPB) {
         const int e = i / (ND + 1), c = i - e * (ND + 1);
         if (e < nel) sG[i] = a.egeom[(int64_t)(e0 + e) * a.egeom_stride + (c < ND ? c * (ND + 1) : ND * ND)];
     }
-
-    // ---- staging --------------------------------------------------------------------------
     T u[ND], p;
     {
         T P[NV];
@@ -169,15 +151,54 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split(const RhsArgs<doub
 #pragma unroll
         for (int k = 0; k < ND; ++k) u[k] = P[1 + k];
         p = P[ND + 1];
-        if (valid) {
-#pragma unroll
-            for (int v = 0; v < NV; ++v) sU[v * NN + tid] = q[v];
-            plain::put_slots<T, ND, TP, NN>(sS + tid, q, P, ir);
-        }
+        if (valid) plain::put_slots<T, ND, TP, NN>(sS + tid, q, P, ir);
     }
     __syncthreads();
 
-    // ---- numerical fluxes on the element's faces -------------------------------------------
+    // ---- volume terms, direction by direction ---------------------------------------------
+    // The first face node's neighbour trace (in the order ρ, normal and transverse momenta, E)
+    // and face data and the epilogue's operand are loaded before the last direction's rows.
+    T acc[NV], pext[NV], xv[NV], pn = T(0), pj = T(0);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[v] = T(0);
+    const T* aux = stage_aux(a);
+    auto none = []() {};
+    auto prefetch = [&]() {
+        if (pf && pnb >= 0) {
+            const int kp = finfo_nbpos(pinfo), dir = fk >> 1;
+            const T* Qn = a.Q + (int64_t)pnb * NPE + line_node<ND, N>(kp >> 1, ff, (kp & 1) ? N - 1 : 0);
+            pext[0] = Qn[0];
+#pragma unroll
+            for (int c = 0; c < ND; ++c) pext[1 + c] = Qn[(1 + (dir + c) % ND) * Nd];
+            pext[NV - 1] = Qn[(NV - 1) * Nd];
+        }
+        if (pf) {
+            const T* g = a.fgeom + (int64_t)pfgi * (3 * ND + 1);
+            pn = g[fk >> 1];
+            pj = g[3 * ND];
+        }
+        if (aux && valid) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) xv[v] = aux[v * Nd + g0 + tid];
+        }
+    };
+    if constexpr (ND == 1) {
+        direction<ND, N, TP, 0>(a, sS, sTab, sD, sG, nel, tid, le, node, valid, q, u, p, prefetch, acc);
+    } else {
+        direction<ND, N, TP, 0>(a, sS, sTab, sD, sG, nel, tid, le, node, valid, q, u, p, none, acc);
+        if constexpr (ND == 3)
+            direction<ND, N, TP, 1>(a, sS, sTab, sD, sG, nel, tid, le, node, valid, q, u, p, none, acc);
+        direction<ND, N, TP, ND - 1>(a, sS, sTab, sD, sG, nel, tid, le, node, valid, q, u, p, prefetch, acc);
+    }
+
+    // ---- numerical fluxes on the element's faces --------------------------------------------
+    T* const sU = sTab;
+    T* const sFn = sTab + NV * NN;
+    if (valid) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) sU[v * NN + tid] = q[v];
+    }
+    __syncthreads();
     for (int it = tid; it < NFN; it += TPB) {
         const bool first = it == tid;
         const int le2 = it / (NF * NPF), r = it - le2 * (NF * NPF);
@@ -230,49 +251,40 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split(const RhsArgs<doub
                 if (type == BC_SLIP) ext[1] = -ext[1];
             }
         }
-        // face frame: the momentum along the master's normal ±e_dir
+        // Face frame: the momentum along the master's normal ±e_dir.  The master's and the
+        // slave's terms commute in every sum but the momentum's, and the jump only changes sign.
         own[1] = sn * own[1];
         ext[1] = sn * ext[1];
         const bool slave = finfo_side(info);
-        T Ql[NV], Qr[NV], Fn[NV];
+        const T sg = slave ? T(-1) : T(1);
+        T Fn[NV];
+        const Recip<T> iro(own[0]), irx(ext[0]);
+        const T po = plain::pressure<T, ND>(own, gamma, iro), px = plain::pressure<T, ND>(ext, gamma, irx);
+        const T uo = iro.div(own[1]), ux = irx.div(ext[1]);
+        const T mo = own[1] * uo, mx = ext[1] * ux;
+        Fn[0] = (own[1] + ext[1]) / T(2);
+        Fn[1] = ((((slave ? mx : mo) + (slave ? px : po)) + (slave ? mo : mx)) + (slave ? po : px)) / T(2);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            Ql[v] = slave ? ext[v] : own[v];
-            Qr[v] = slave ? own[v] : ext[v];
-        }
-        const Recip<T> irl(Ql[0]), irr(Qr[0]);
-        const T pl = plain::pressure<T, ND>(Ql, gamma, irl), pr = plain::pressure<T, ND>(Qr, gamma, irr);
-        const T ul = irl.div(Ql[1]), ur = irr.div(Qr[1]);
-        Fn[0] = (Ql[1] + Qr[1]) / T(2);
-        Fn[1] = (((Ql[1] * ul + pl) + Qr[1] * ur) + pr) / T(2);
-#pragma unroll
-        for (int c = 1; c < ND; ++c) Fn[1 + c] = (Ql[1 + c] * ul + Qr[1 + c] * ur) / T(2);
-        Fn[NV - 1] = ((Ql[NV - 1] + pl) * ul + (Qr[NV - 1] + pr) * ur) / T(2);
+        for (int c = 1; c < ND; ++c) Fn[1 + c] = (own[1 + c] * uo + ext[1 + c] * ux) / T(2);
+        Fn[NV - 1] = ((own[NV - 1] + po) * uo + (ext[NV - 1] + px) * ux) / T(2);
         if (a.sdiss == DISS_LXF) {
-            const T al = plain::dsqrt(irl.div(gamma * pl), a.errflag);
-            const T ar = plain::dsqrt(irr.div(gamma * pr), a.errflag);
-            const T la = fabs(ul) + al, lb = fabs(ur) + ar;
-            const T lam = (la < lb) ? lb : la;
+            const T lo = fabs(uo) + plain::dsqrt(iro.div(gamma * po), a.errflag);
+            const T lx = fabs(ux) + plain::dsqrt(irx.div(gamma * px), a.errflag);
+            // the larger speed, the master's where they do not compare
+            const T lam = sg * (slave ? ((lx < lo) ? lo : lx) : ((lo < lx) ? lx : lo));
 #pragma unroll
-            for (int v = 0; v < NV; ++v) Fn[v] = Fn[v] + ((lam * (Ql[v] - Qr[v])) / T(2)) * a.intensity;
+            for (int v = 0; v < NV; ++v) Fn[v] = Fn[v] + ((lam * (own[v] - ext[v])) / T(2)) * a.intensity;
         }
         Fn[1] = sn * Fn[1];
         T* o = sFn + ((le2 * NF + k) * NV) * NPF + f;
+        const T js = sg * jac;
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            const T x = Fn[v] * jac;
             const int vv = (v == 0 || v == NV - 1) ? v : vo[v >= 1 && v <= ND ? v - 1 : 0];
-            o[vv * NPF] = slave ? -x : x;
+            o[vv * NPF] = Fn[v] * js;
         }
     }
-
-    // ---- volume terms, direction by direction ------------------------------------------------
-    T acc[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) acc[v] = T(0);
-    direction<ND, N, TP, 0>(a, sS, sU, sD, sG, nel, tid, le, node, valid, q, u, p, acc);
-    if constexpr (ND >= 2) direction<ND, N, TP, 1>(a, sS, sU, sD, sG, nel, tid, le, node, valid, q, u, p, acc);
-    if constexpr (ND >= 3) direction<ND, N, TP, 2>(a, sS, sU, sD, sG, nel, tid, le, node, valid, q, u, p, acc);
+    __syncthreads();
     if (!valid) return;
 
     // ---- FR lift on the end nodes, mass matrix and stage epilogue -----------------------------

@@ -30,15 +30,17 @@ struct Recip {
     __device__ explicit Recip(T b_) : b(b_) {}
     __device__ T div(T a) const { return a / b; }                   // a / b
     __device__ T div2(T a) const { return a / (T(2) * b); }         // a / (2b)
+    __device__ T fin(T a) const { return a / b; }                   // a / b, b finite and not 0, a finite
 };
 
 template <>
 struct Recip<double> {
     double b, y;
     __device__ explicit Recip(double b_) : b(b_) {
+        // v_rcp_f64 is good to 2^-24; one step of third order leaves only the last rounding
         const double y0 = __builtin_amdgcn_rcp(b);
-        const double y1 = __builtin_fma(__builtin_fma(-b, y0, 1.0), y0, y0);
-        y = __builtin_fma(__builtin_fma(-b, y1, 1.0), y1, y1);
+        const double e = __builtin_fma(-b, y0, 1.0);
+        y = __builtin_fma(y0, __builtin_fma(e, e, e), y0);
     }
     __device__ static double quot(double a, double b, double y) {
         const double q = a * y;
@@ -46,6 +48,10 @@ struct Recip<double> {
     }
     __device__ double div(double a) const { return quot(a, b, y); }
     __device__ double div2(double a) const { return quot(a, 2.0 * b, 0.5 * y); }
+    __device__ double fin(double a) const {
+        const double q = a * y;
+        return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+    }
 };
 
 template <>
@@ -61,12 +67,22 @@ struct Recip<float> {
     }
     __device__ float div(float a) const { return quot(a, b, y); }
     __device__ float div2(float a) const { return quot(a, 2.0f * b, 0.5f * y); }
+    __device__ float fin(float a) const {
+        const float q = a * y;
+        return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    }
 };
 
 // a / b
 template <typename T>
 __device__ inline T xdiv(T a, T b) {
     return Recip<T>(b).div(a);
+}
+
+// a / b for finite a and b, b not 0 (elsewhere NaN, where the quotient would be infinite or 0)
+template <typename T>
+__device__ inline T fdiv(T a, T b) {
+    return Recip<T>(b).fin(a);
 }
 
 // a / C for a finite a and a small whole number C (1/C rounded at compile time)

@@ -202,14 +202,15 @@ constexpr int tp_slots() {
     return TP == TP_CHANDRASEKHAR ? ND + 2 : (TP == TP_KENNEDY_GRUBER ? ND + 3 : 2 * ND + 2);
 }
 
-// Logarithmic mean of a/2 and b/2 from their ratio's F: (a + b)/(2F) with hs = (a + b)/2.
+// F of the logarithmic mean (a + b)/(2F) (see logarithmic_mean).  Where a quotient here is not
+// finite its operands are a vacuum's or negative ones', and the flux is NaN either way.
 template <typename T>
 __device__ inline T logmean_factor(T al, T ar, int* err) {
-    const T xi = xdiv(al, ar);
-    const T f = xdiv(xi - T(1), xi + T(1));
+    const T xi = fdiv(al, ar);
+    const T f = fdiv(xi - T(1), xi + T(1));
     const T u = f * f;
     if (u < T(0.01)) return ((T(1) + cdiv<3>(u)) + cdiv<5>(u * u)) + cdiv<7>((u * u) * u);
-    return xdiv(dlog(xi, err), T(2) * f);
+    return fdiv(dlog(xi, err), T(2) * f);
 }
 
 // Component DIR of the two-point flux between the lower (1) and higher (2) line position
@@ -236,16 +237,16 @@ __device__ __forceinline__ void pair_flux(const T* A, const T* B, T ja, T gm1, i
 #pragma unroll
         for (int k = 0; k < ND; ++k) um[k] = A[1 + k] + B[1 + k];
         const T hs = A[0] + B[0], sb = A[ND + 1] + B[ND + 1];
-        const T rho = xdiv(hs, logmean_factor(A[0], B[0], err));
-        const T p = xdiv(hs, sb);
-        const T beta2 = xdiv(sb, logmean_factor(A[ND + 1], B[ND + 1], err));  // 2β̂
+        const T rho = fdiv(hs, logmean_factor(A[0], B[0], err));
+        const T p = fdiv(hs, sb);
+        const T beta2 = fdiv(sb, logmean_factor(A[ND + 1], B[ND + 1], err));  // 2β̂
         T sq = A[1] * A[1];  // (|u1|² + |u2|²)/4
 #pragma unroll
         for (int k = 1; k < ND; ++k) sq = sq + A[1 + k] * A[1 + k];
 #pragma unroll
         for (int k = 0; k < ND; ++k) sq = sq + B[1 + k] * B[1 + k];
-        T h = xdiv(T(1), beta2 * gm1) - sq;
-        h = h + xdiv(p, rho);
+        T h = fdiv(T(1), beta2 * gm1) - sq;
+        h = h + fdiv(p, rho);
 #pragma unroll
         for (int k = 0; k < ND; ++k) h = h + um[k] * um[k];
         f[0] = rho * um[DIR];

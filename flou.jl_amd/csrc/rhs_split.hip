@@ -36,7 +36,12 @@ namespace split {
 template <int ND, int N>
 struct SCfg {
     static constexpr int NPE = Cfg<ND, N>::NPE, NPF = Cfg<ND, N>::NPF, NF = 2 * ND, NV = ND + 2;
-    static constexpr int EPB = Cfg<ND, N>::EPB;
+    // Elements per block: two waves where their nodes and pairs fill whole waves (2-D N=4: 5
+    // elements of 25 nodes against 10: CFL run of 2623 elements 289 -> 259 us; more, smaller
+    // blocks wait less at barriers and spread evenly over the CUs), else the count up to 256
+    // threads that does (2-D N=5: 7; 5 elements: gradient 1360 -> 1374 us).  3-D N=5 runs one
+    // element (216 of 256 lanes; two, 432 of 448: CK2N54 step 4698 -> 5145 us).
+    static constexpr int EPB = NPE > 128 ? 1 : (ND == 2 && N == 6 ? 7 : (ND == 2 && N == 7 ? 5 : 128 / NPE));
     static constexpr int NN = EPB * NPE;                 // nodes per block
     static constexpr int TPB = ((NN + 63) / 64) * 64;    // threads per block
     static constexpr int NPAIR = N * (N - 1) / 2;

@@ -40,6 +40,8 @@ def units():
         u.append((f"vjp_fast_{name}.o", "vjp_fast.hip", ["-ffp-contract=fast", f"-DFLOUHIP_FVJP_TP={tp}"]))
     for nd in (1, 2, 3):
         u.append((f"rhs_split_{nd}d.o", "rhs_split.hip", EXACT + [f"-DFLOUHIP_ND={nd}"]))
+    for nd in (2, 3):
+        u.append((f"vjp_split_{nd}d.o", "vjp_split.hip", [f"-DFLOUHIP_ND={nd}"]))
     for prec in ("F64", "F32"):
         for nd in (1, 2, 3):
             u.append((f"rhs_hybrid_{prec.lower()}_{nd}d.o", "rhs_hybrid.hip",

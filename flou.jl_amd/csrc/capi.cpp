@@ -179,6 +179,20 @@ std::string& create_error() {
     return msg;
 }
 
+// ω_i D♯_ij antisymmetric with a vanishing diagonal, up to rounding (the SBP property on GLL
+// nodes).
+bool sbp(const flou_hip_desc* d) {
+    const int n = d->n;
+    double smax = 0.0, asym = 0.0;
+    for (int i = 0; i < n; ++i)
+        for (int j = 0; j < n; ++j) {
+            const double s = d->omega[i] * d->Dsharp[i * n + j];
+            smax = std::max(smax, std::fabs(s));
+            asym = std::max(asym, std::fabs(s + d->omega[j] * d->Dsharp[j * n + i]));
+        }
+    return asym <= 1e-14 * smax;
+}
+
 // Affine elements whose metric is diagonal and whose face frames are (±e_k, ±e_{k+1}, ±e_{k+2})
 // along the direction k of both elements of the face, zeros exact: Flou's CartesianMesh.
 bool axis_aligned(const flou_hip_desc* d) {
@@ -675,6 +689,18 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
         h->v64 = nd == 1 ? vjp_f64_1d(n, h->eq, h->vol, h->tp, h->curved, gen)
                          : (nd == 2 ? vjp_f64_2d(n, h->eq, h->vol, h->tp, h->curved, gen)
                                     : vjp_f64_3d(n, h->eq, h->vol, h->tp, h->curved, gen));
+        // split-form Euler with the StdAverage/LxF surface flux on axis-aligned affine elements,
+        // 4 or more nodes per direction: one line per thread (rhs_vjp, Chandrasekhar, 16384
+        // elements of 6x6 nodes: 55 -> 40 us, 0.5 M nodes of 8x8x8: 238 -> 72); below that lines are
+        // too short for it.  A line is a chain of n(n-1)/2 pairs: on meshes that leave CUs idle the
+        // thread per node is done sooner (7x7 nodes, 576 elements: 11.6 against 14.9 us, 6084: 34
+        // against 24; 6x6, 1296: 11.6 against 12.1, 2304: 14.5 against 12.3; 6x6x6, 125: 16.0
+        // against 17.5, 512: 22.8 against 19.3), but not StdAverage's, a sum of node terms.
+        const int64_t fill = h->tp == FLOU_HIP_TP_STDAVG || n < 6 ? 0
+                             : nd == 2 ? 256 * (n == 6 ? 6 : 12) : (n == 6 ? 256 : 0);
+        if (h->v64 && h->vol == FLOU_HIP_SPLIT && h->eq == FLOU_HIP_EULER && !gen && nd >= 2 && n >= 4 && diag &&
+            !oriented && h->gather && h->lift_end && d->nelements >= fill && sbp(d))
+            h->v64 = nd == 2 ? split_vjp_f64_2(n, h->tp) : split_vjp_f64_3(n, h->tp);
     } else {
         h->v32 = nd == 1 ? vjp_f32_1d(n, h->eq, h->vol, h->tp, h->curved, gen)
                          : (nd == 2 ? vjp_f32_2d(n, h->eq, h->vol, h->tp, h->curved, gen)

@@ -26,6 +26,27 @@ __device__ __forceinline__ int pair_ab(int pr) {
     return (int)(w >> (6 * (pr < 10 ? pr : (pr < 20 ? pr - 10 : pr - 20)))) & 63;
 }
 
+// Node arrays of a block in LDS: with PAD one value after every row of N nodes, so that lanes on
+// consecutive x-lines, N values apart, read distinct banks for even N too.
+template <int ND, int N, bool PAD>
+struct NodeLds {
+    static constexpr int RS = PAD ? N + 1 : N;               // row stride
+    static constexpr int ES = Cfg<ND, N>::NPE / N * RS;      // element stride
+    __device__ __forceinline__ static int node(int j) { return PAD ? j + j / N : j; }  // block node j
+    // first node of line f of direction DIR in an element, and the step along the line
+    template <int DIR>
+    __device__ __forceinline__ static int line(int f) {
+        if (ND == 1) return 0;
+        if (DIR == 0) return RS * f;
+        if (ND == 2) return f;
+        return f % N + RS * (DIR == 1 ? N : 1) * (f / N);
+    }
+    template <int DIR>
+    static constexpr int step() {
+        return DIR == 0 ? 1 : (DIR == 1 ? RS : RS * N);
+    }
+};
+
 // The stage epilogue's second operand: the RK register or the SSP base state, null if the
 // stage has none.
 template <typename T>

@@ -1,0 +1,602 @@
+// FP64 adjoint of the split-form Euler rhs on axis-aligned affine elements (GLL nodes,
+// Chandrasekhar, Kennedy-Gruber or StdAverage two-point flux, StdAverage or LxF(StdAverage)
+// surface flux), 2-D and 3-D, with the reverse RK stage epilogue: VjpArgs of common.hpp, the
+// products of k_vjp (vjp_plain.hip) up to rounding.
+//
+// What bounds it: FP64 arithmetic and, on small states, HBM.  k_vjp gives a thread to every
+// node; it differentiates pairs along full metric vectors and hands the partner's side over
+// through an LDS table (1859 VALU per wave of 64 nodes at 2-D N=5).  Here a thread takes a line:
+//   * each pair of the line is recomputed and differentiated once, both sides accumulated in
+//     registers; no table, and one wave runs lines of one direction, so that the direction, the
+//     LDS strides and the line frame (normal velocity first) are compile-time constants;
+//   * off the (zero) diagonal S_ij = ω_i D♯_ij is antisymmetric (SBP), so the cotangent of the
+//     pair flux F♯(i, j), -D♯_ij w_i - D♯_ji w_j, is S_ij (w_j/ω_j - w_i/ω_i);
+//   * the metric Ja_dd scales the line's result, not every pair's normal;
+//   * cotangents are those of the halved node inputs, pulled back to (ρ, m, E) once per node;
+//   * the face flux is differentiated with respect to the own trace only, by the line that
+//     ends there.
+// LDS: the node inputs and w = c·Y/J; the rows of the directions are added, one direction after
+// the other, over w.  Measured, Chandrasekhar, rhs_vjp: 2-D N=5, 0.59 M nodes: 55 -> 40 us;
+// 3-D N=5, 1.7 M nodes: 271 -> 184 us; 3-D N=7, 0.5 M nodes: 238 -> 72 us.
+// Compile with -DFLOUHIP_ND=2|3.
+#include "common.hpp"
+#include "adjoint.hpp"
+#include "stage.hpp"
+#include <type_traits>
+
+namespace flouhip {
+namespace svjp {
+
+using adj::rcp;
+
+// Elements per block: the lines of one direction fill whole waves (3-D N=6 of 7 nodes: 49 of
+// 64 lanes, N=5: 108 of 128); 2-D N=7 leaves 8 lanes for a third block per CU (Kennedy-Gruber, 4624
+// elements: 27.6 -> 18.7 us).
+template <int ND, int N>
+constexpr int epb() {
+    return ND == 2 ? (N == 8 ? 7 : 64 / N) : (N == 4 ? 4 : (N == 5 ? 5 : (N == 6 ? 3 : 1)));
+}
+
+// LDS rows are padded where lines of N nodes pile up on few banks (2-D, 16384 elements,
+// Kennedy-Gruber, rhs_vjp without and with: lines of 4 nodes 14.1 and 11.8 us, of 8 79.3 and
+// 59.2); lines of 6 nodes lose more by the block per CU that the padding costs (32.6 and 37.4).
+template <int ND, int N>
+using Nodes = NodeLds<ND, N, N == 4 || N == 8>;
+
+template <int ND, int N, int TP>
+struct LCfg {
+    static constexpr int NPE = Cfg<ND, N>::NPE, NPF = Cfg<ND, N>::NPF, NF = 2 * ND, NV = ND + 2;
+    static constexpr int EPB = epb<ND, N>();
+    static constexpr int NN = EPB * Nodes<ND, N>::ES;  // LDS nodes per block
+    static constexpr int NL = EPB * NPF;                 // lines per block and direction
+    static constexpr int WPD = (NL + 63) / 64;           // waves per direction
+    static constexpr int TPB = ND * WPD * 64;
+    static constexpr int NA = TP == TP_KENNEDY_GRUBER ? ND + 3 : ND + 2;  // node inputs = line rows
+};
+
+// F = atanh(f)/f of a logarithmic mean and dF/du at u = f² on the forward's branch
+// (Utilities.jl:34-44); a, b: the two values.  SERIES: the caller knows that u < 0.01.  Both
+// forms are evaluated and selected otherwise: a branch per pair in the unrolled line took every
+// register and spilled.
+template <bool SERIES>
+__device__ __forceinline__ void lm_factor(double u, double f, double a, double b, double& F, double& dF) {
+    F = fma(u, fma(u, fma(u, 1.0 / 7, 1.0 / 5), 1.0 / 3), 1.0);
+    dF = fma(u, fma(u, 3.0 / 7, 2.0 / 5), 1.0 / 3);
+    if constexpr (!SERIES) {
+        const double Fl = 0.5 * log(a * rcp(b)) * rcp(f);
+        const double dl = 0.5 * (rcp(1 - u) - Fl) * rcp(u);
+        F = u < 0.01 ? F : Fl;
+        dF = u < 0.01 ? dF : dl;
+    }
+}
+
+// Reverse product of component n (the first velocity) of the two-point flux for the cotangent
+// G = (ρ, n, t.., E), scaled by s, added to the cotangents gi and gj of the nodes' inputs:
+// Chandrasekhar (ρ/2, u/2.., β), Kennedy-Gruber (ρ/2, u/2.., p/2, E/(2ρ)).
+template <int ND, int TP, bool SERIES>
+__device__ __forceinline__ void pair_vjp(const double* P, const double* Q, const double* G, double s, double ig1,
+                                         double* gi, double* gj) {
+    constexpr int NV = ND + 2;
+    double ub[ND];
+#pragma unroll
+    for (int k = 0; k < ND; ++k) ub[k] = P[1 + k] + Q[1 + k];
+    const double un = ub[0];
+    double gu = G[1] * ub[0];
+#pragma unroll
+    for (int k = 1; k < ND; ++k) gu = fma(G[1 + k], ub[k], gu);
+    const double gn = G[1], ge = G[NV - 1];
+    if constexpr (TP == TP_KENNEDY_GRUBER) {
+        // f = (m, m ū + p̄ n, m ē + p̄ ū_n), m = ρ̄ ū_n: every input enters as the sum
+        const double rho = P[0] + Q[0], p = P[ND + 1] + Q[ND + 1], e = P[ND + 2] + Q[ND + 2];
+        const double m = rho * un;
+        const double mb = fma(ge, e, G[0] + gu);
+        const double unb = fma(mb, rho, ge * p);
+        double t[NV + 1];
+        t[0] = mb * un;
+#pragma unroll
+        for (int k = 0; k < ND; ++k) t[1 + k] = k == 0 ? fma(m, gn, unb) : m * G[1 + k];
+        t[ND + 1] = fma(ge, un, gn);
+        t[ND + 2] = ge * m;
+#pragma unroll
+        for (int c = 0; c < NV + 1; ++c) {
+            gi[c] = fma(s, t[c], gi[c]);
+            gj[c] = fma(s, t[c], gj[c]);
+        }
+    } else {
+        // ρ̂ = (a_i + a_j)/F_ρ, p̄ = (a_i + a_j)/(β_i + β_j), m = ρ̂ ū_n,
+        // h = (F_β/(γ-1) + F_ρ)/(β_i + β_j) + 2 v_i·v_j, f = (m, m ū + p̄ n, m h)
+        double dot = P[1] * Q[1];
+#pragma unroll
+        for (int k = 1; k < ND; ++k) dot = fma(P[1 + k], Q[1 + k], dot);
+        const double hs = P[0] + Q[0], dA = P[0] - Q[0], sb = P[ND + 1] + Q[ND + 1], db = P[ND + 1] - Q[ND + 1];
+        const double rb = rcp(sb), ihs = rcp(hs);
+        const double fr = dA * ihs, ur = fr * fr, fb = db * rb, u2 = fb * fb;
+        double Fr, dFr, Fb, dFb;
+        if (!SERIES) __builtin_amdgcn_sched_barrier(0);  // one logarithm's registers at a time
+        lm_factor<SERIES>(ur, fr, P[0], Q[0], Fr, dFr);
+        if (!SERIES) __builtin_amdgcn_sched_barrier(0);
+        lm_factor<SERIES>(u2, fb, P[ND + 1], Q[ND + 1], Fb, dFb);
+        if (!SERIES) __builtin_amdgcn_sched_barrier(0);
+        const double iFr = rcp(Fr);
+        const double rho = hs * iFr;
+        const double m = rho * un;
+        const double Xf = fma(Fb, ig1, Fr);
+        const double h = fma(rb, Xf, 2 * dot);
+        const double hb = ge * m;                     // h̄
+        const double mb = fma(ge, h, G[0] + gu);      // m̄
+        const double mbr = mb * rho;                  // of ū_n
+        const double rhob = mb * un;                  // of ρ̂
+        const double t = hb * rb;
+        double rbb = fma(hb, Xf, gn * hs);            // of 1/(β_i + β_j), through h and p̄
+        const double Frb = fma(-rhob * rho, iFr, t);  // of F_ρ, through ρ̂ and h
+        double hsb = fma(gn, rb, rhob * iFr);         // of a_i + a_j, through p̄ and ρ̂
+        const double dAb = (2 * fr) * (Frb * dFr) * ihs;
+        hsb = fma(-dAb, fr, hsb);
+        const double fbb = (2 * fb) * (t * ig1) * dFb;
+        const double dbb = fbb * rb;
+        rbb = fma(fbb, db, rbb);
+        const double sbb = -rbb * rb * rb;
+        const double dotb = 2 * hb;
+        gi[0] = fma(s, hsb + dAb, gi[0]);
+        gj[0] = fma(s, hsb - dAb, gj[0]);
+        gi[NV - 1] = fma(s, sbb + dbb, gi[NV - 1]);
+        gj[NV - 1] = fma(s, sbb - dbb, gj[NV - 1]);
+#pragma unroll
+        for (int k = 0; k < ND; ++k) {
+            const double ubb = k == 0 ? fma(m, gn, mbr) : m * G[1 + k];
+            gi[1 + k] = fma(s, fma(dotb, Q[1 + k], ubb), gi[1 + k]);
+            gj[1 + k] = fma(s, fma(dotb, P[1 + k], ubb), gj[1 + k]);
+        }
+    }
+}
+
+// One side of the face flux: its state in the face frame with what the products need.
+template <int ND>
+struct Side {
+    double ir, u[ND], uu, p, c, a;
+    __device__ __forceinline__ Side(const double* R, double gamma) {
+        ir = rcp(R[0]);
+        uu = 0;
+#pragma unroll
+        for (int k = 0; k < ND; ++k) {
+            u[k] = R[1 + k] * ir;
+            uu = fma(u[k], u[k], uu);
+        }
+        p = (gamma - 1) * fma(-0.5 * R[0], uu, R[ND + 1]);
+        c = sqrt(gamma * p * ir);
+        a = fabs(u[0]) + c;
+    }
+    // Adds to b the product of f(R)·n for the cotangent G and lb times the gradient of a.
+    __device__ __forceinline__ void add(const double* R, const double* G, double gamma, double lb, double* b) const {
+        constexpr int NV = ND + 2;
+        const double g1 = gamma - 1;
+        double unb = G[NV - 1] * (R[NV - 1] + p);
+#pragma unroll
+        for (int k = 0; k < ND; ++k) unb = fma(G[1 + k], R[1 + k], unb);
+        unb += lb * (u[0] > 0 ? 1.0 : (u[0] < 0 ? -1.0 : 0.0));
+        const double cb = lb == 0 ? 0.0 : 0.5 * lb * rcp(c);  // of c²
+        const double pg = g1 * (fma(G[NV - 1], u[0], G[1]) + cb * gamma * ir);
+        const double uir = unb * ir;
+        b[0] += -uir * u[0] + 0.5 * pg * uu - cb * c * c * ir;
+#pragma unroll
+        for (int k = 0; k < ND; ++k) b[1 + k] += fma(G[1 + k], u[0], fma(-pg, u[k], k == 0 ? G[0] + uir : 0.0));
+        b[NV - 1] += fma(G[NV - 1], u[0], pg);
+    }
+};
+
+// A wave's lines of direction DIR.  Component k of a vector in the line frame is physical
+// component (DIR + k) % ND.
+template <int ND, int N, int TP, int DIR>
+__device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const double* sP, double* sW, double* sT,
+                                           const double* sS, const double* siw, int e0, int nel, int l,
+                                           double (&acc)[N][LCfg<ND, N, TP>::NA]) {
+    using C = LCfg<ND, N, TP>;
+    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, NN = C::NN, NA = C::NA;
+    using M = Nodes<ND, N>;
+    constexpr int ST = M::template step<DIR>();
+    constexpr int GST = DIR == 0 ? 1 : (DIR == 1 ? N : N * N);  // step along the line in the state
+    const RhsArgs<double>& a = A.r;
+    const bool task = l < C::NL && l / NPF < nel;
+    const int le = task ? l / NPF : 0, f = l % NPF;
+    const int base = le * M::ES + M::template line<DIR>(f);
+    const double* eg = a.egeom + (int64_t)(e0 + le) * a.egeom_stride;
+    const double ja = eg[DIR * (ND + 1)];
+    const double gamma = a.gamma, ig1 = 1 / (gamma - 1);
+    int vo[ND];  // physical variable of line-frame momentum k
+#pragma unroll
+    for (int k = 0; k < ND; ++k) vo[k] = 1 + (DIR + k) % ND;
+
+    // ---- faces at the two line ends: cotangent of the own trace ------------------------
+    if (task) {
+#pragma unroll
+        for (int sd = 0; sd < 2; ++sd) {
+            const int slot = (e0 + le) * NF + 2 * DIR + sd;
+            const int info = a.finfo[slot], nb = a.nb[slot];
+            const double* g = a.fgeom + (int64_t)a.fgi[slot] * (3 * ND + 1);
+            const bool slave = finfo_side(info);
+            const double so = slave ? -g[DIR] : g[DIR];   // own outward normal along the axis
+            const int64_t on = (int64_t)(e0 + le) * NPE + line_node<ND, N>(DIR, f, 0) + (sd ? (N - 1) * GST : 0);
+            double o[NV], x[NV], G[NV], ob[NV], xb[NV];
+            o[0] = a.Q[on];
+            o[NV - 1] = a.Q[(NV - 1) * a.ndofs + on];
+#pragma unroll
+            for (int k = 0; k < ND; ++k) o[1 + k] = a.Q[vo[k] * a.ndofs + on];
+            // S̄ = ½·jac·(-∂g_own w_own + ∂g_nb w_nb), of (f_o + f_x)·n + λ·diss·(o - x)
+            const double h = 0.5 * g[3 * ND];
+            const double co = h * (sd ? a.ops[ops_gp(N) + N - 1] : a.ops[ops_gm(N)]);
+            const int ol = base + (sd ? (N - 1) * ST : 0);
+            G[0] = -co * sW[ol];
+            G[NV - 1] = -co * sW[(NV - 1) * NN + ol];
+#pragma unroll
+            for (int k = 0; k < ND; ++k) G[1 + k] = -co * sW[vo[k] * NN + ol];
+            int type = -1;
+            if (nb >= 0) {
+                const int kp = finfo_nbpos(info);
+                const int64_t nn = (int64_t)nb * NPE + line_node<ND, N>(DIR, f, (kp & 1) ? N - 1 : 0);
+                const double cn = h * ((kp & 1) ? a.ops[ops_gp(N) + N - 1] : a.ops[ops_gm(N)]) *
+                                  (A.c / a.egeom[(int64_t)nb * a.egeom_stride + ND * ND]);
+                x[0] = a.Q[nn];
+                x[NV - 1] = a.Q[(NV - 1) * a.ndofs + nn];
+                G[0] = fma(cn, A.Y[nn], G[0]);
+                G[NV - 1] = fma(cn, A.Y[(NV - 1) * a.ndofs + nn], G[NV - 1]);
+#pragma unroll
+                for (int k = 0; k < ND; ++k) {
+                    x[1 + k] = a.Q[vo[k] * a.ndofs + nn];
+                    G[1 + k] = fma(cn, A.Y[vo[k] * a.ndofs + nn], G[1 + k]);
+                }
+            } else {
+                const int bd = finfo_bd(info);
+                type = a.bctype[bd];
+                const double* src = type == BC_DIRICHLET ? a.bcstate + ((int64_t)a.fid[slot] * NPF + f) * NV
+                                                         : a.bcconst + bd * NV;
+                const bool given = type == BC_DIRICHLET || type == BC_INFLOW;
+                x[0] = given ? src[0] : o[0];
+                x[NV - 1] = given ? src[NV - 1] : o[NV - 1];
+#pragma unroll
+                for (int k = 0; k < ND; ++k) x[1 + k] = given ? src[vo[k]] : o[1 + k];
+                if (type == BC_SLIP) x[1] = -x[1];
+            }
+            // frame of the own outward normal
+            o[1] *= so;
+            x[1] *= so;
+            G[1] *= so;
+            const Side<ND> S(o, gamma), X(x, gamma);
+            double lo = 0, lx = 0, dl = 0;
+#pragma unroll
+            for (int v = 0; v < NV; ++v) ob[v] = xb[v] = 0;
+            if (a.sdiss == DISS_LXF) {
+                // λ's derivative goes to the side that the forward's maximum keeps, the master on ties
+                const bool mine = slave ? X.a < S.a : !(S.a < X.a);
+                const double lam = (mine ? S.a : X.a) * a.intensity;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    ob[v] = lam * G[v];
+                    xb[v] = -lam * G[v];
+                    dl = fma(o[v] - x[v], G[v], dl);
+                }
+                dl *= a.intensity;
+                lo = mine ? dl : 0;
+                lx = mine ? 0 : dl;
+            }
+            S.add(o, G, gamma, lo, ob);
+            if (type == BC_OUTFLOW || type == BC_SLIP) {  // the exterior state follows the own trace
+                X.add(x, G, gamma, lx, xb);
+                if (type == BC_SLIP) xb[1] = -xb[1];
+#pragma unroll
+                for (int v = 0; v < NV; ++v) ob[v] += xb[v];
+            }
+            ob[1] *= so;
+            double* t = sT + ((le * NF + 2 * DIR + sd) * NV) * NPF + f;
+            t[0] = ob[0];
+            t[(NV - 1) * NPF] = ob[NV - 1];
+#pragma unroll
+            for (int k = 0; k < ND; ++k) t[vo[k] * NPF] = ob[1 + k];
+        }
+    }
+
+    // ---- the line's pairs ----------------------------------------------------------------
+    auto load = [&](int p, double* P, double* W) {
+        const double* s = sP + base + p * ST;
+        const double* w = sW + base + p * ST;
+        if constexpr (TP == TP_STDAVG) {  // u.., H, |u|²
+#pragma unroll
+            for (int k = 0; k < ND; ++k) P[k] = s[(vo[k] - 1) * NN];
+            P[ND] = s[ND * NN];
+            P[ND + 1] = s[(ND + 1) * NN];
+        } else {
+            P[0] = s[0];
+#pragma unroll
+            for (int k = 0; k < ND; ++k) P[1 + k] = s[vo[k] * NN];
+#pragma unroll
+            for (int c = ND + 1; c < NA; ++c) P[c] = s[c * NN];
+        }
+        W[0] = w[0];
+#pragma unroll
+        for (int k = 0; k < ND; ++k) W[1 + k] = w[vo[k] * NN];
+        W[NV - 1] = w[(NV - 1) * NN];
+    };
+#pragma unroll
+    for (int p = 0; p < N; ++p)
+#pragma unroll
+        for (int c = 0; c < NA; ++c) acc[p][c] = 0;
+    if constexpr (TP == TP_STDAVG) {
+        // the flux is a sum of node terms: each node takes the reverse product of ½ f(Q)·n̄ for
+        // Σ_j S_ij (w_j/ω_j - w_i/ω_i)
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            double P[NA], wi[NV];
+            load(i, P, wi);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) wi[v] *= siw[i];
+#pragma unroll
+            for (int j = i + 1; j < N; ++j) {
+                const double* w = sW + base + j * ST;
+                const double s = sS[i * N + j], iw = siw[j];
+#pragma unroll
+                for (int v = 0; v < NV; ++v) {
+                    const int pv = v == 0 || v == NV - 1 ? v : vo[v >= 1 && v <= ND ? v - 1 : 0];
+                    const double g = fma(w[pv * NN], iw, -wi[v]);
+                    acc[i][v] = fma(s, g, acc[i][v]);
+                    acc[j][v] = fma(s, g, acc[j][v]);
+                }
+            }
+        }
+        const double h = 0.5 * ja;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            double P[NA], w[NV], G[NV];
+            load(i, P, w);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) G[v] = h * acc[i][v];
+            double U = G[NV - 1] * P[ND];
+#pragma unroll
+            for (int k = 0; k < ND; ++k) U = fma(G[1 + k], P[k], U);
+            const double un = P[0], pg = (gamma - 1) * fma(G[NV - 1], un, G[1]);
+            acc[i][0] = fma(-U, un, 0.5 * pg * P[ND + 1]);
+#pragma unroll
+            for (int k = 0; k < ND; ++k) acc[i][1 + k] = fma(G[1 + k], un, fma(-pg, P[k], k == 0 ? G[0] + U : 0.0));
+            acc[i][NV - 1] = fma(G[NV - 1], un, pg);
+        }
+    } else {
+        auto pairs = [&](auto series) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                double P[NA], wi[NV];
+                load(i, P, wi);
+#pragma unroll
+                for (int v = 0; v < NV; ++v) wi[v] *= siw[i];
+#pragma unroll
+                for (int j = i + 1; j < N; ++j) {
+                    double Q[NA], G[NV];
+                    load(j, Q, G);
+                    const double iw = siw[j];
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) G[v] = fma(G[v], iw, -wi[v]);
+                    pair_vjp<ND, TP, decltype(series)::value>(P, Q, G, sS[i * N + j] * ja, ig1, acc[i], acc[j]);
+                    // one pair's loads and arithmetic at a time: the registers hold the rows,
+                    // node i and one pair
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
+        if constexpr (TP == TP_CHANDRASEKHAR) {
+            // the series for every pair of the wave's lines when the spreads of ρ and β along
+            // each line allow it (u of its extreme values below 0.01), else the general form
+            double amax = sP[base], amin = amax, bmax = sP[(ND + 1) * NN + base], bmin = bmax;
+#pragma unroll
+            for (int p = 1; p < N; ++p) {
+                const double x = sP[base + p * ST], y = sP[(ND + 1) * NN + base + p * ST];
+                amax = fmax(amax, x); amin = fmin(amin, x);
+                bmax = fmax(bmax, y); bmin = fmin(bmin, y);
+            }
+            const double da = amax - amin, sa = amax + amin, db = bmax - bmin, sb = bmax + bmin;
+            const bool near = da * da < 0.01 * (1 - 1e-12) * sa * sa && db * db < 0.01 * (1 - 1e-12) * sb * sb;
+            if (__all(!task || near)) pairs(std::true_type());
+            else pairs(std::false_type());
+        } else {
+            pairs(std::true_type());
+        }
+    }
+    // (the rows are pinned here: their use below is conditional, and the pairs would sink into it)
+#pragma unroll
+    for (int p = 0; p < N; ++p)
+#pragma unroll
+        for (int c = 0; c < NA; ++c) asm volatile("" : "+v"(acc[p][c]));
+}
+
+// Adds (direction 0: writes) a line's rows to the nodes' sums, in physical component order.
+template <int ND, int N, int TP, int DIR>
+__device__ __forceinline__ void add_rows(double* sR, int nel, int l, const double (&acc)[N][LCfg<ND, N, TP>::NA]) {
+    using C = LCfg<ND, N, TP>;
+    using M = Nodes<ND, N>;
+    constexpr int ST = M::template step<DIR>();
+    if (l >= C::NL || l / C::NPF >= nel) return;
+    double* r = sR + (l / C::NPF) * M::ES + M::template line<DIR>(l % C::NPF);
+#pragma unroll
+    for (int p = 0; p < N; ++p)
+#pragma unroll
+        for (int c = 0; c < C::NA; ++c) {
+            const int pc = c >= 1 && c <= ND ? 1 + (DIR + c - 1) % ND : c;
+            double* x = r + pc * C::NN + p * ST;
+            *x = DIR == 0 ? acc[p][c] : *x + acc[p][c];
+        }
+}
+
+template <int ND, int N, int TP>
+__global__ void __launch_bounds__((LCfg<ND, N, TP>::TPB)) k_svjp(const VjpArgs<double> A) {
+    using C = LCfg<ND, N, TP>;
+    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, EPB = C::EPB, TPB = C::TPB, NN = C::NN, NA = C::NA;
+    __shared__ double sP[NA * NN];                       // node inputs
+    __shared__ double sW[(NA > NV ? NA : NV) * NN];      // w = c·Y/J, then the sums of the rows
+    __shared__ double sT[EPB * NF * NV * NPF];           // cotangents of the own traces
+    __shared__ double sS[N * N], siw[N];
+    const RhsArgs<double>& a = A.r;
+    const int tid = threadIdx.x;
+    const int e0 = xcd_remap(blockIdx.x, gridDim.x) * EPB;
+    const int64_t Nd = a.ndofs, g0 = (int64_t)e0 * NPE;
+    const int nel = a.ne - e0 < EPB ? a.ne - e0 : EPB;
+    const int nnb = nel * NPE;
+    const double gamma = a.gamma, gm1 = a.gamma - 1;
+
+    for (int i = tid; i < N * N; i += TPB) {
+        const int r = i / N, c = i - r * N;
+        const double* w = a.ops + ops_w(N);
+        const double* D = a.ops + ops_Dsh(N);
+        sS[i] = 0.5 * (w[r] * D[i] - w[c] * D[c * N + r]);
+    }
+    for (int i = tid; i < N; i += TPB) siw[i] = 1 / a.ops[ops_w(N) + i];
+    for (int j = tid; j < nnb; j += TPB) {
+        const int jj = Nodes<ND, N>::node(j);
+        double q[NV], y[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            q[v] = a.Q[v * Nd + g0 + j];
+            y[v] = A.Y[v * Nd + g0 + j];
+        }
+        const double cj = A.c / a.egeom[(int64_t)(e0 + j / NPE) * a.egeom_stride + ND * ND];
+        const double ir = rcp(q[0]);
+        double u[ND], uu = 0;
+#pragma unroll
+        for (int k = 0; k < ND; ++k) {
+            u[k] = q[1 + k] * ir;
+            uu = fma(u[k], u[k], uu);
+        }
+        const double p = gm1 * fma(-0.5 * q[0], uu, q[NV - 1]);
+        if constexpr (TP == TP_STDAVG) {
+#pragma unroll
+            for (int k = 0; k < ND; ++k) sP[k * NN + jj] = u[k];
+            sP[ND * NN + jj] = (q[NV - 1] + p) * ir;
+            sP[(ND + 1) * NN + jj] = uu;
+        } else {
+            sP[jj] = 0.5 * q[0];
+#pragma unroll
+            for (int k = 0; k < ND; ++k) sP[(1 + k) * NN + jj] = 0.5 * u[k];
+            if constexpr (TP == TP_CHANDRASEKHAR) {
+                sP[(ND + 1) * NN + jj] = 0.5 * q[0] * rcp(p);
+            } else {
+                sP[(ND + 1) * NN + jj] = 0.5 * p;
+                sP[(ND + 2) * NN + jj] = 0.5 * q[NV - 1] * ir;
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) sW[v * NN + jj] = cj * y[v];
+    }
+    __syncthreads();
+
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int dir = wave / C::WPD;
+    const int l = (wave - dir * C::WPD) * 64 + (tid & 63);
+    double acc[N][NA];
+    if (dir == 0) line_phase<ND, N, TP, 0>(A, sP, sW, sT, sS, siw, e0, nel, l, acc);
+    else if (ND == 2 || dir == 1) line_phase<ND, N, TP, 1>(A, sP, sW, sT, sS, siw, e0, nel, l, acc);
+    else line_phase<ND, N, TP, ND - 1>(A, sP, sW, sT, sS, siw, e0, nel, l, acc);
+    __syncthreads();  // w has been read
+    if (dir == 0) add_rows<ND, N, TP, 0>(sW, nel, l, acc);
+    __syncthreads();
+    if (dir == 1) add_rows<ND, N, TP, 1>(sW, nel, l, acc);
+    __syncthreads();
+    if constexpr (ND == 3) {
+        if (dir == 2) add_rows<ND, N, TP, 2>(sW, nel, l, acc);
+        __syncthreads();
+    }
+
+    // ---- per node: pullback of the inputs, face terms, epilogue ----------------------------
+    for (int j = tid; j < nnb; j += TPB) {
+        const int jj = Nodes<ND, N>::node(j);
+        double t[NA], V[NV];
+#pragma unroll
+        for (int c = 0; c < NA; ++c) t[c] = sW[c * NN + jj];
+        if constexpr (TP == TP_STDAVG) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) V[v] = t[v];
+        } else {
+            const double rho = 2 * sP[jj], ir = rcp(rho);
+            double u[ND], uu = 0, ubu = 0;
+#pragma unroll
+            for (int k = 0; k < ND; ++k) {
+                u[k] = 2 * sP[(1 + k) * NN + jj];
+                uu = fma(u[k], u[k], uu);
+            }
+            double rb, pg, eb;  // of ρ at fixed (u, p, E), (γ-1) × of p, of E at fixed ρ
+            if constexpr (TP == TP_CHANDRASEKHAR) {
+                const double b2 = 2 * sP[(ND + 1) * NN + jj];  // 1/p = 2β/ρ
+                rb = 0.5 * fma(t[NV - 1], b2 * ir, t[0]);
+                pg = -gm1 * t[NV - 1] * (0.5 * b2) * (b2 * ir);
+                eb = 0;
+            } else {
+                eb = 0.5 * t[ND + 2] * ir;
+                rb = fma(-eb, 2 * sP[(ND + 2) * NN + jj], 0.5 * t[0]);
+                pg = 0.5 * gm1 * t[ND + 1];
+            }
+#pragma unroll
+            for (int k = 0; k < ND; ++k) {
+                const double ubk = 0.5 * t[1 + k];
+                ubu = fma(ubk, u[k], ubu);
+                V[1 + k] = fma(ubk, ir, -pg * u[k]);
+            }
+            V[0] = fma(-ubu, ir, fma(0.5 * pg, uu, rb));
+            V[NV - 1] = pg + eb;
+        }
+        const int le = j / NPE, node = j - le * NPE;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            int f, pos;
+            node_line<ND, N>(node, d, f, pos);
+            if (pos == 0 || pos == N - 1) {
+                const double* F = sT + ((le * NF + 2 * d + (pos == 0 ? 0 : 1)) * NV) * NPF + f;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) V[v] += F[v * NPF];
+            }
+        }
+        double p0[NV], p1[NV], p2[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int64_t i = v * Nd + g0 + j;
+            p0[v] = A.P0 ? A.P0[i] : 0.0;
+            p1[v] = A.P1 ? A.P1[i] : 0.0;
+            p2[v] = A.P2 ? A.P2[i] : 0.0;
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int64_t i = v * Nd + g0 + j;
+            const double o = V[v] + A.a0 * p0[v] + A.a1 * p1[v];
+            if (A.o1) A.o1[i] = A.b0 * o + A.b1 * p1[v] + A.b2 * p2[v];
+            A.o0[i] = o;
+        }
+    }
+}
+
+template <int ND, int N, int TP>
+static hipError_t launch(const VjpArgs<double>& a, hipStream_t s) {
+    using C = LCfg<ND, N, TP>;
+    hipLaunchKernelGGL((k_svjp<ND, N, TP>), dim3((a.r.ne + C::EPB - 1) / C::EPB), dim3(C::TPB), 0, s, a);
+    return hipGetLastError();
+}
+
+template <int ND, int N>
+static VjpLauncherF64 pick_tp(int tp) {
+    switch (tp) {
+        case TP_STDAVG: return &launch<ND, N, TP_STDAVG>;
+        case TP_CHANDRASEKHAR: return &launch<ND, N, TP_CHANDRASEKHAR>;
+        case TP_KENNEDY_GRUBER: return &launch<ND, N, TP_KENNEDY_GRUBER>;
+        default: return nullptr;
+    }
+}
+
+}  // namespace svjp
+
+#define FLOUHIP_CAT_(a, b) a##b
+#define FLOUHIP_CAT(a, b) FLOUHIP_CAT_(a, b)
+
+VjpLauncherF64 FLOUHIP_CAT(split_vjp_f64_, FLOUHIP_ND)(int n, int tp) {
+    switch (n) {
+        case 4: return svjp::pick_tp<FLOUHIP_ND, 4>(tp);
+        case 5: return svjp::pick_tp<FLOUHIP_ND, 5>(tp);
+        case 6: return svjp::pick_tp<FLOUHIP_ND, 6>(tp);
+        case 7: return svjp::pick_tp<FLOUHIP_ND, 7>(tp);
+        case 8: return svjp::pick_tp<FLOUHIP_ND, 8>(tp);
+        default: return nullptr;
+    }
+}
+
+}  // namespace flouhip

@@ -27,6 +27,11 @@
 namespace flouhip {
 namespace hybrid {
 
+// LDS rows padded for lines of 4 and 8 nodes (MatrixDissipation, 0.6 M nodes in 2-D, 1 M in 3-D,
+// without and with: 2-D of 8 nodes 109.7 and 105.8 us, 3-D of 4 258 and 254; 2-D of 6 89.6 and 92.2).
+template <int ND, int N>
+using Nodes = NodeLds<ND, N, N == 4 || N == 8>;
+
 template <int ND, int N>
 struct HCfg {
     static constexpr int NPE = Cfg<ND, N>::NPE, NPF = Cfg<ND, N>::NPF, NF = 2 * ND, NV = ND + 2;
@@ -36,6 +41,7 @@ struct HCfg {
     static constexpr int NL = EPB * NPF;                 // lines per block and direction
     static constexpr int NPAIR = N * (N - 1) / 2;
     static constexpr int NPR = NL * NPAIR;
+    static constexpr int SN = EPB * Nodes<ND, N>::ES;  // LDS nodes per block
 };
 
 // Flux input slots held beside the conservative states.
@@ -60,9 +66,10 @@ __device__ __forceinline__ void direction(const RhsArgs<T>& a, const T* sS, cons
                                           const T* sC, const T* sw, const T* sM, int nel, int tid, int le, int node,
                                           bool valid, T (&acc)[ND + 2]) {
     using C = HCfg<ND, N>;
-    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NN = C::NN, NL = C::NL;
+    constexpr int NV = C::NV, NPF = C::NPF, SN = C::SN, NL = C::NL;
     constexpr int NS = plain::tp_slots<ND, TP>(), NSL = lds_slots<ND, TP>();
-    constexpr int ST = DIR == 0 ? 1 : (DIR == 1 ? N : N * N);
+    using M = Nodes<ND, N>;
+    constexpr int ST = M::template step<DIR>();
     const T gm1 = a.gamma - T(1);
     const T avel[3] = {T(0), T(0), T(0)};
     // pair fluxes, each once
@@ -72,14 +79,14 @@ __device__ __forceinline__ void direction(const RhsArgs<T>& a, const T* sS, cons
         const int le2 = C::EPB == 1 ? 0 : l / NPF, f = l - le2 * NPF;
         if (le2 >= nel) continue;
         const int ab = pair_ab<N>(pr);
-        const int base = le2 * NPE + line_node<ND, N>(DIR, f, 0);
+        const int base = le2 * M::ES + M::template line<DIR>(f);
         const T* pa = sS + base + (ab >> 3) * ST;
         const T* pb = sS + base + (ab & 7) * ST;
         T A[NS], B[NS], F[NV];
 #pragma unroll
         for (int c = 0; c < NS; ++c) {  // StdAverage's conservative slots lie in sQ
-            A[c] = c < NSL ? pa[c * NN] : T(0.5) * sQ[(pa - sS) + (1 + c - NSL) * NN];
-            B[c] = c < NSL ? pb[c * NN] : T(0.5) * sQ[(pb - sS) + (1 + c - NSL) * NN];
+            A[c] = c < NSL ? pa[c * SN] : T(0.5) * sQ[(pa - sS) + (1 + c - NSL) * SN];
+            B[c] = c < NSL ? pb[c * SN] : T(0.5) * sQ[(pb - sS) + (1 + c - NSL) * SN];
         }
         if constexpr (DIAG) {
             plain::pair_flux<T, ND, TP, DIR>(A, B, sM[DIR * (ND + 1)], gm1, a.errflag, F);
@@ -92,7 +99,7 @@ __device__ __forceinline__ void direction(const RhsArgs<T>& a, const T* sS, cons
             constexpr int SC = TP == TP_KENNEDY_GRUBER ? ND + 2 : ND + 1;
             const T sa = TP == TP_KENNEDY_GRUBER ? T(2) * A[SC] : A[SC], sb = TP == TP_KENNEDY_GRUBER ? T(2) * B[SC] : B[SC];
 #pragma unroll
-            for (int v = 0; v < NV; ++v) { qa[v] = ca[v * NN]; qb[v] = cb[v * NN]; }
+            for (int v = 0; v < NV; ++v) { qa[v] = ca[v * SN]; qb[v] = cb[v * SN]; }
             Pa[0] = qa[0];
             Pb[0] = qb[0];
 #pragma unroll
@@ -106,7 +113,7 @@ __device__ __forceinline__ void direction(const RhsArgs<T>& a, const T* sS, cons
                                                      avel, a.errflag, F);
         }
 #pragma unroll
-        for (int v = 0; v < NV; ++v) sTab[k * NV + v] = F[v];
+        for (int v = 0; v < NV; ++v) sTab[v * C::NPR + k] = F[v];
     }
     __syncthreads();
     // interface fluxes: at most one per thread (NL (N-1) <= NN)
@@ -120,17 +127,17 @@ __device__ __forceinline__ void direction(const RhsArgs<T>& a, const T* sS, cons
         for (int ik = s; ik < N; ++ik)
             for (int il = 0; il < s; ++il) {
                 const int pr = il * (2 * N - il - 1) / 2 + (ik - il - 1);
-                const T* t = sTab + (pr * NL + l) * NV;
+                const T* t = sTab + pr * NL + l;
                 const T c = sC[il * N + ik];
 #pragma unroll
-                for (int v = 0; v < NV; ++v) Fb[v] = Fb[v] + c * t[v];
+                for (int v = 0; v < NV; ++v) Fb[v] = Fb[v] + c * t[v * C::NPR];
             }
-        const int nr = (l / NPF) * NPE + line_node<ND, N>(DIR, l % NPF, 0) + s * ST, nl = nr - ST;
+        const int nr = (l / NPF) * M::ES + M::template line<DIR>(l % NPF) + s * ST, nl = nr - ST;
         T Ql[NV], Qr[NV], Wl[NV], Wr[NV], Rl[NV], Rr[NV], Vl[NV], Vr[NV], Fr[NV], Fv[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            Ql[v] = sQ[v * NN + nl]; Qr[v] = sQ[v * NN + nr];
-            Wl[v] = sW[v * NN + nl]; Wr[v] = sW[v * NN + nr];
+            Ql[v] = sQ[v * SN + nl]; Qr[v] = sQ[v * SN + nr];
+            Wl[v] = sW[v * SN + nl]; Wr[v] = sW[v * SN + nr];
         }
         to_frame<T, ND, DIR>(Ql, Rl);
         to_frame<T, ND, DIR>(Qr, Rr);
@@ -178,9 +185,9 @@ __global__ void __launch_bounds__((HCfg<ND, N>::TPB)) k_hybrid(const RhsArgs<T> 
     constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, EPB = C::EPB, TPB = C::TPB, NN = C::NN;
     constexpr int NS = lds_slots<ND, TP>();
     constexpr int TAB = NV * (C::NPR > N * C::NL ? C::NPR : N * C::NL);
-    __shared__ T sS[NS * NN];            // two-point flux inputs
-    __shared__ T sQ[NV * NN];            // conservative states
-    __shared__ T sW[NV * NN];            // entropy variables
+    __shared__ T sS[NS * C::SN];         // two-point flux inputs
+    __shared__ T sQ[NV * C::SN];         // conservative states
+    __shared__ T sW[NV * C::SN];         // entropy variables
     __shared__ T sTab[TAB];              // pair table of one direction, then its interface fluxes
     __shared__ T sFn[EPB * NF * NV * NPF];
     __shared__ T sC[N * N], sw[N], sM[ND * ND];
@@ -208,12 +215,13 @@ __global__ void __launch_bounds__((HCfg<ND, N>::TPB)) k_hybrid(const RhsArgs<T> 
         T P[NV], W[NV];
         const Recip<T> ir(q[0]);
         plain::cons2prim<T, ND>(q, a.gamma, P, ir);
-        plain::put_slots<T, ND, TP, NN, false>(sS + tid, q, P, ir);
+        const int j = Nodes<ND, N>::node(tid);
+        plain::put_slots<T, ND, TP, C::SN, false>(sS + j, q, P, ir);
         plain::cons2entropy<T, ND>(q, a.gamma, a.errflag, W);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
-            sQ[v * NN + tid] = q[v];
-            sW[v * NN + tid] = W[v];
+            sQ[v * C::SN + j] = q[v];
+            sW[v * C::SN + j] = W[v];
         }
     }
     __syncthreads();
@@ -227,10 +235,10 @@ __global__ void __launch_bounds__((HCfg<ND, N>::TPB)) k_hybrid(const RhsArgs<T> 
         const int slot = (e0 + le2) * NF + k;
         const int info = a.finfo[slot], nbe = a.nb[slot];
         const T* g = a.fgeom + (int64_t)a.fgi[slot] * (3 * ND + 1);
-        const int on = le2 * NPE + line_node<ND, N>(k >> 1, f, (k & 1) ? N - 1 : 0);
+        const int on = Nodes<ND, N>::node(le2 * NPE + line_node<ND, N>(k >> 1, f, (k & 1) ? N - 1 : 0));
         T own[NV], ext[NV];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) own[v] = sQ[v * NN + on];
+        for (int v = 0; v < NV; ++v) own[v] = sQ[v * C::SN + on];
         if (nbe >= 0) {
             const int kp = finfo_nbpos(info);
             const T* Qn = a.Q + (int64_t)nbe * NPE +

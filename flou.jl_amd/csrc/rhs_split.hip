@@ -33,6 +33,12 @@
 namespace flouhip {
 namespace split {
 
+// LDS rows are padded where lines of N nodes pile up on few banks (Kennedy-Gruber, 0.6 M nodes in
+// 2-D, 1 M in 3-D, without and with: 2-D lines of 4 nodes 25.8 and 22.0 us, of 6 31.7 and 26.2, of
+// 8 48.8 and 28.5; 3-D of 4 62 and 60, of 8 127 and 100); not for 2 nodes, nor 6 in 3-D (no gain).
+template <int ND, int N>
+using Nodes = NodeLds<ND, N, N == 4 || N == 8 || (ND == 2 && N == 6)>;
+
 template <int ND, int N>
 struct SCfg {
     static constexpr int NPE = Cfg<ND, N>::NPE, NPF = Cfg<ND, N>::NPF, NF = 2 * ND, NV = ND + 2;
@@ -47,6 +53,13 @@ struct SCfg {
     static constexpr int NPAIR = N * (N - 1) / 2;
     static constexpr int NPR = EPB * NPF * NPAIR;        // pairs per block and direction
     static constexpr int NL = EPB * NPF;                 // lines per block and direction
+    static constexpr int SN = EPB * Nodes<ND, N>::ES;  // LDS nodes per block
+    // The table: pair fluxes of line l at pr·NLP + l, then the nodes' own; entry k, variable v at
+    // k·KS + v·VS.  2-D (4 variables) keeps a plane per variable with an odd line count, so that
+    // neither the pairs' writes nor the rows' reads pile up on few banks.
+    static constexpr int NLP = ND == 2 ? NL | 1 : NL;
+    static constexpr int TAB = NPAIR * NLP + NN;
+    static constexpr int KS = ND == 2 ? 1 : NV, VS = ND == 2 ? TAB : 1;
 };
 
 // One direction: every pair flux and every node's contravariant flux (the diagonal entry of
@@ -58,18 +71,20 @@ __device__ __forceinline__ void direction(const RhsArgs<double>& a, const double
                                           const double (&q)[ND + 2], const double (&u)[ND], double p, LOADS loads,
                                           double (&acc)[ND + 2]) {
     using C = SCfg<ND, N>;
-    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NN = C::NN, NL = C::NL, NS = plain::tp_slots<ND, TP>();
+    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, SN = C::SN, NL = C::NL, NS = plain::tp_slots<ND, TP>();
+    constexpr int KS = C::KS, VS = C::VS, DIAG = C::NPAIR * C::NLP;
+    using M = Nodes<ND, N>;
     const double gm1 = a.gamma - 1.0;
     int lf, ii;
     node_line<ND, N>(node, DIR, lf, ii);
     if (valid) {
         // contravariant flux along DIR (plain::contravariant_flux, diagonal metric)
         const double ja = sG[le * (ND + 1) + DIR];
-        double* t = sTab + (C::NPR + tid) * NV;
+        double* t = sTab + (DIAG + tid) * KS;
         t[0] = q[1 + DIR] * ja;
 #pragma unroll
-        for (int c = 0; c < ND; ++c) t[1 + c] = (c == DIR ? q[1 + DIR] * u[c] + p : q[1 + DIR] * u[c]) * ja;
-        t[NV - 1] = ((q[NV - 1] + p) * u[DIR]) * ja;
+        for (int c = 0; c < ND; ++c) t[(1 + c) * VS] = (c == DIR ? q[1 + DIR] * u[c] + p : q[1 + DIR] * u[c]) * ja;
+        t[(NV - 1) * VS] = ((q[NV - 1] + p) * u[DIR]) * ja;
     }
 #pragma unroll 1
     for (int k = tid; k < C::NPR; k += C::TPB) {
@@ -77,31 +92,31 @@ __device__ __forceinline__ void direction(const RhsArgs<double>& a, const double
         const int le2 = C::EPB == 1 ? 0 : l / NPF, f = l - le2 * NPF;
         if (le2 >= nel) continue;
         const int ab = pair_ab<N>(pr);
-        const int base = le2 * NPE + line_node<ND, N>(DIR, f, 0);
-        constexpr int ST = DIR == 0 ? 1 : (DIR == 1 ? N : N * N);
+        const int base = le2 * M::ES + M::template line<DIR>(f);
+        constexpr int ST = M::template step<DIR>();
         const double* pa = sS + base + (ab >> 3) * ST;
         const double* pb = sS + base + (ab & 7) * ST;
         double A[NS], B[NS], F[NV];
 #pragma unroll
-        for (int c = 0; c < NS; ++c) { A[c] = pa[c * NN]; B[c] = pb[c * NN]; }
+        for (int c = 0; c < NS; ++c) { A[c] = pa[c * SN]; B[c] = pb[c * SN]; }
         plain::pair_flux<double, ND, TP, DIR>(A, B, sG[le2 * (ND + 1) + DIR], gm1, a.errflag, F);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) sTab[k * NV + v] = F[v];
+        for (int v = 0; v < NV; ++v) sTab[(pr * C::NLP + l) * KS + v * VS] = F[v];
     }
     loads();
     __syncthreads();
     if (valid) {
         // pair (j, ii) or (ii, j) of the node's line: pair index ii - 1 at j = 0, then N - j - 2
         // further for each j < ii and 1 further from there (the place of j = ii is skipped over)
-        const int diag = (C::NPR + tid) * NV;
-        int off = ((ii - 1) * NL + le * NPF + lf) * NV;
+        const int diag = (DIAG + tid) * KS;
+        int off = ((ii - 1) * C::NLP + le * NPF + lf) * KS;
 #pragma unroll
         for (int j = 0; j < N; ++j) {
             const double* t = sTab + (j == ii ? diag : off);
             const double Dij = sD[ii * N + j];
 #pragma unroll
-            for (int v = 0; v < NV; ++v) acc[v] = acc[v] - Dij * t[v];
-            off += (j < ii ? N - j - 2 : 1) * (NL * NV);
+            for (int v = 0; v < NV; ++v) acc[v] = acc[v] - Dij * t[v * VS];
+            off += (j < ii ? N - j - 2 : 1) * (C::NLP * KS);
         }
     }
     __syncthreads();  // the table has been read
@@ -114,8 +129,8 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split(const RhsArgs<doub
     constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, EPB = C::EPB, TPB = C::TPB, NN = C::NN;
     constexpr int NS = plain::tp_slots<ND, TP>();
     constexpr int NFN = EPB * NF * NPF;  // face nodes of the block
-    constexpr int TAB = C::NPR + NN, FACE = NN + NFN;
-    __shared__ T sS[NS * NN];                          // two-point flux inputs, [slot][node]
+    constexpr int TAB = C::TAB, FACE = NN + NFN;
+    __shared__ T sS[NS * C::SN];                       // two-point flux inputs, [slot][node]
     __shared__ T sTab[NV * (TAB > FACE ? TAB : FACE)];  // pair and node fluxes of one direction, then
                                                        // conservative states [v][node] and face fluxes
     __shared__ T sD[N * N];
@@ -156,7 +171,7 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split(const RhsArgs<doub
 #pragma unroll
         for (int k = 0; k < ND; ++k) u[k] = P[1 + k];
         p = P[ND + 1];
-        if (valid) plain::put_slots<T, ND, TP, NN>(sS + tid, q, P, ir);
+        if (valid) plain::put_slots<T, ND, TP, C::SN>(sS + Nodes<ND, N>::node(tid), q, P, ir);
     }
     __syncthreads();
 

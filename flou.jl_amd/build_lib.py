@@ -46,6 +46,8 @@ def units():
         for nd in (1, 2, 3):
             u.append((f"rhs_hybrid_{prec.lower()}_{nd}d.o", "rhs_hybrid.hip",
                       EXACT + [f"-DFLOUHIP_PREC_{prec}", f"-DFLOUHIP_ND={nd}"]))
+            u.append((f"rhs_strong_{prec.lower()}_{nd}d.o", "rhs_strong.hip",
+                      EXACT + [f"-DFLOUHIP_PREC_{prec}", f"-DFLOUHIP_ND={nd}"]))
             u.append((f"rhs_plain_{prec.lower()}_{nd}d.o", "rhs_plain.hip",
                       EXACT + [f"-DFLOUHIP_PREC_{prec}", f"-DFLOUHIP_ND={nd}"]))
             u.append((f"vjp_plain_{prec.lower()}_{nd}d.o", "vjp_plain.hip",

@@ -675,6 +675,16 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
                                     : plain_f32_3d(n, h->eq, kvol, h->tp, h->curved));
         if (!h->l32) return bad(FLOU_HIP_EUNSUPPORTED, "no kernel for this combination");
     }
+    // the strong form likewise, and linear advection (3-D, 5 nodes per line, 0.9 M nodes: FP32 37.8 ->
+    // 22 us, FP64 72 -> 38; advection on 256 elements 5.4 -> 5.0 us per stage)
+    if (h->vol == FLOU_HIP_STRONG && diag && !oriented && h->gather && h->lift_end &&
+        (h->eq == FLOU_HIP_ADVECTION || (h->savg == FLOU_HIP_AVG_STD && (h->sdiss == FLOU_HIP_DISS_NONE ||
+                                                                          h->sdiss == FLOU_HIP_DISS_LXF)))) {
+        if (h->prec == FLOU_HIP_FP64)
+            h->l64 = nd == 1 ? strong_f64_1(n, h->eq) : (nd == 2 ? strong_f64_2(n, h->eq) : strong_f64_3(n, h->eq));
+        else
+            h->l32 = nd == 1 ? strong_f32_1(n, h->eq) : (nd == 2 ? strong_f32_2(n, h->eq) : strong_f32_3(n, h->eq));
+    }
     // adjoint kernels: the StdAverage surface average with LxF or no dissipation has a
     // hand-written face-flux VJP; every other Euler surface flux (Chandrasekhar average,
     // Scalar and Matrix dissipation) differentiates the plain flux in dual numbers (gen)

@@ -218,6 +218,15 @@ RhsLauncherF64 split_f64_1(int n, int tp);
 RhsLauncherF64 split_f64_2(int n, int tp);
 RhsLauncherF64 split_f64_3(int n, int tp);
 
+// Strong form on axis-aligned affine elements, GLL nodes (rhs_strong.hip): Euler with the
+// StdAverage or LxF(StdAverage) surface flux, linear advection.
+RhsLauncherF64 strong_f64_1(int n, int eq);
+RhsLauncherF64 strong_f64_2(int n, int eq);
+RhsLauncherF64 strong_f64_3(int n, int eq);
+RhsLauncherF32 strong_f32_1(int n, int eq);
+RhsLauncherF32 strong_f32_2(int n, int eq);
+RhsLauncherF32 strong_f32_3(int n, int eq);
+
 typedef hipError_t (*VjpLauncherF64)(const VjpArgs<double>&, hipStream_t);
 typedef hipError_t (*VjpLauncherF32)(const VjpArgs<float>&, hipStream_t);
 // FP64 adjoint of the split form on axis-aligned affine elements (vjp_split.hip), n = 4..8.

@@ -15,9 +15,7 @@
 //   * a node's own contravariant flux goes into the same table as the pairs, so that its row
 //     reads N entries without a case for the diagonal, at offsets that advance by constants
 //     (2504 -> 2186 VALU per wave at 3-D N=5 with the above, 0.99 -> 0.96 ms);
-//   * face states are read in the order (normal, transverse..) of the face frame by index,
-//     n = ±e_d, t = ±e_{d+1}, b = ±e_{d+2}: signs of the transverse axes commute with every
-//     rounding of the LxF and StdAverage fluxes, so they need not be applied;
+//   * face states are read in the order of the face frame by index (faces.hpp);
 //   * quotients share reciprocals (exact_div.hpp), the node's contravariant flux reuses its
 //     primitives, the lift touches the end nodes only (∂g is exactly zero elsewhere);
 //   * the face fluxes come last and lie over the dead table (39 KB of LDS at 3-D N=5, 4 waves
@@ -27,6 +25,7 @@
 // and table writes are conflict-light and the pair's positions nearly uniform.
 // Compile with -DFLOUHIP_ND=1|2|3.
 #include "common.hpp"
+#include "faces.hpp"
 #include "physics_plain.hpp"
 #include "stage.hpp"
 
@@ -186,11 +185,8 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split(const RhsArgs<doub
     auto prefetch = [&]() {
         if (pf && pnb >= 0) {
             const int kp = finfo_nbpos(pinfo), dir = fk >> 1;
-            const T* Qn = a.Q + (int64_t)pnb * NPE + line_node<ND, N>(kp >> 1, ff, (kp & 1) ? N - 1 : 0);
-            pext[0] = Qn[0];
-#pragma unroll
-            for (int c = 0; c < ND; ++c) pext[1 + c] = Qn[(1 + (dir + c) % ND) * Nd];
-            pext[NV - 1] = Qn[(NV - 1) * Nd];
+            load_trace<T, ND, NV>(a.Q + (int64_t)pnb * NPE + line_node<ND, N>(kp >> 1, ff, (kp & 1) ? N - 1 : 0), Nd,
+                                  dir, pext);
         }
         if (pf) {
             const T* g = a.fgeom + (int64_t)pfgi * (3 * ND + 1);
@@ -229,13 +225,10 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split(const RhsArgs<doub
         const int info = first ? pinfo : a.finfo[slot];
         const int nbe = first ? pnb : a.nb[slot];
         const int on = le2 * NPE + line_node<ND, N>(dir, f, (k & 1) ? N - 1 : 0);
-        int vo[ND];  // physical variable of each face-frame momentum
-#pragma unroll
-        for (int c = 0; c < ND; ++c) vo[c] = 1 + (dir + c) % ND;
-        T own[NV], ext[NV];
+        T own[NV], ext[NV], Fn[NV];
         own[0] = sU[on];
 #pragma unroll
-        for (int c = 0; c < ND; ++c) own[1 + c] = sU[vo[c] * NN + on];
+        for (int c = 0; c < ND; ++c) own[1 + c] = sU[face_mom<ND>(dir, c) * NN + on];
         own[NV - 1] = sU[(NV - 1) * NN + on];
         T sn = pn, jac = pj;
         if (!first) {
@@ -249,60 +242,18 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split(const RhsArgs<doub
                 for (int v = 0; v < NV; ++v) ext[v] = pext[v];
             } else {
                 const int kp = finfo_nbpos(info);
-                const T* Qn = a.Q + (int64_t)nbe * NPE + line_node<ND, N>(kp >> 1, f, (kp & 1) ? N - 1 : 0);
-                ext[0] = Qn[0];
-#pragma unroll
-                for (int c = 0; c < ND; ++c) ext[1 + c] = Qn[vo[c] * Nd];
-                ext[NV - 1] = Qn[(NV - 1) * Nd];
+                load_trace<T, ND, NV>(a.Q + (int64_t)nbe * NPE + line_node<ND, N>(kp >> 1, f, (kp & 1) ? N - 1 : 0),
+                                      Nd, dir, ext);
             }
         } else {
-            const int bd = finfo_bd(info);
-            const int type = a.bctype[bd];
-            if (type == BC_DIRICHLET || type == BC_INFLOW) {
-                const T* src = type == BC_DIRICHLET ? a.bcstate + ((int64_t)a.fid[slot] * NPF + f) * NV
-                                                    : a.bcconst + bd * NV;
-                ext[0] = src[0];
-#pragma unroll
-                for (int c = 0; c < ND; ++c) ext[1 + c] = src[vo[c]];
-                ext[NV - 1] = src[NV - 1];
-            } else {
-#pragma unroll
-                for (int v = 0; v < NV; ++v) ext[v] = own[v];
-                if (type == BC_SLIP) ext[1] = -ext[1];
-            }
+            boundary_trace<T, ND, NPF, NV>(a, info, slot, f, dir, own, ext);
         }
-        // Face frame: the momentum along the master's normal ±e_dir.  The master's and the
-        // slave's terms commute in every sum but the momentum's, and the jump only changes sign.
-        own[1] = sn * own[1];
-        ext[1] = sn * ext[1];
-        const bool slave = finfo_side(info);
-        const T sg = slave ? T(-1) : T(1);
-        T Fn[NV];
-        const Recip<T> iro(own[0]), irx(ext[0]);
-        const T po = plain::pressure<T, ND>(own, gamma, iro), px = plain::pressure<T, ND>(ext, gamma, irx);
-        const T uo = iro.div(own[1]), ux = irx.div(ext[1]);
-        const T mo = own[1] * uo, mx = ext[1] * ux;
-        Fn[0] = (own[1] + ext[1]) / T(2);
-        Fn[1] = ((((slave ? mx : mo) + (slave ? px : po)) + (slave ? mo : mx)) + (slave ? po : px)) / T(2);
-#pragma unroll
-        for (int c = 1; c < ND; ++c) Fn[1 + c] = (own[1 + c] * uo + ext[1 + c] * ux) / T(2);
-        Fn[NV - 1] = ((own[NV - 1] + po) * uo + (ext[NV - 1] + px) * ux) / T(2);
-        if (a.sdiss == DISS_LXF) {
-            const T lo = fabs(uo) + plain::dsqrt(iro.div(gamma * po), a.errflag);
-            const T lx = fabs(ux) + plain::dsqrt(irx.div(gamma * px), a.errflag);
-            // the larger speed, the master's where they do not compare
-            const T lam = sg * (slave ? ((lx < lo) ? lo : lx) : ((lo < lx) ? lx : lo));
-#pragma unroll
-            for (int v = 0; v < NV; ++v) Fn[v] = Fn[v] + ((lam * (own[v] - ext[v])) / T(2)) * a.intensity;
-        }
-        Fn[1] = sn * Fn[1];
+        axis_flux<T, ND>(own, ext, sn, jac, finfo_side(info), a.sdiss, gamma, a.intensity, a.errflag, Fn);
         T* o = sFn + ((le2 * NF + k) * NV) * NPF + f;
-        const T js = sg * jac;
+        o[0] = Fn[0];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const int vv = (v == 0 || v == NV - 1) ? v : vo[v >= 1 && v <= ND ? v - 1 : 0];
-            o[vv * NPF] = Fn[v] * js;
-        }
+        for (int c = 0; c < ND; ++c) o[face_mom<ND>(dir, c) * NPF] = Fn[1 + c];
+        o[(NV - 1) * NPF] = Fn[NV - 1];
     }
     __syncthreads();
     if (!valid) return;

@@ -217,6 +217,9 @@ RhsLauncherF32 hybrid_f32_3(int n, int tp, bool diag);
 RhsLauncherF64 split_f64_1(int n, int tp);
 RhsLauncherF64 split_f64_2(int n, int tp);
 RhsLauncherF64 split_f64_3(int n, int tp);
+// the same on curved elements, up to rounding
+RhsLauncherF64 split_curved_f64_2(int n, int tp);
+RhsLauncherF64 split_curved_f64_3(int n, int tp);
 
 // Strong form on axis-aligned affine elements, GLL nodes (rhs_strong.hip): Euler with the
 // StdAverage or LxF(StdAverage) surface flux, linear advection.

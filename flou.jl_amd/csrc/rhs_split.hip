@@ -48,7 +48,7 @@ struct SCfg {
     // element (216 of 256 lanes; two, 432 of 448: CK2N54 step 4698 -> 5145 us).
     static constexpr int EPB = NPE > 128 ? 1 : (ND == 2 && N == 6 ? 7 : (ND == 2 && N == 7 ? 5 : 128 / NPE));
     static constexpr int NN = EPB * NPE;                 // nodes per block
-    static constexpr int TPB = ((NN + 63) / 64) * 64;    // threads per block
+    static constexpr int TPB = block_threads(NN);        // threads per block
     static constexpr int NPAIR = N * (N - 1) / 2;
     static constexpr int NPR = EPB * NPF * NPAIR;        // pairs per block and direction
     static constexpr int NL = EPB * NPF;                 // lines per block and direction
@@ -294,6 +294,383 @@ static RhsLauncherF64 pick_tp(int tp) {
     }
 }
 
+// ---- curved elements --------------------------------------------------------------------------
+//
+// The same form with a metric per node.  The general kernel forms every component of a pair's
+// flux and contracts them with the mean metric n̄, with IEEE quotients throughout, and reads
+// metrics from memory once per pair.  Here the flux along n̄ is formed directly (ρ̂ ū·n̄ first),
+// quotients by reciprocals good to an ulp and sums by fused multiply-adds, so results agree
+// with the general kernel's up to rounding; a direction's metric rows lie in LDS beside the
+// flux inputs.  Faces: the flux along n from the master's frame; every sum over the two sides
+// commutes and is rounded the same way on both, so that the sides' fluxes are opposite bit for bit.
+// What bounds it: waits between the barriers at two or three blocks per CU; HBM moves 1.6 GB a
+// stage at 11.2 M nodes, 0.34 ms at a copy's rate.  Measured, Chandrasekhar, SSPRK33 steps: 3-D N=6,
+// 11.2 M nodes: 9.1 -> 3.0 ms; N=5, 7.1 M nodes: 3.6 -> 1.8 ms.
+
+__device__ __forceinline__ double rcp(double x) {  // 1/x to about an ulp
+    const double y = __builtin_amdgcn_rcp(x), e = __builtin_fma(-x, y, 1.0);
+    return __builtin_fma(y, __builtin_fma(e, e, e), y);
+}
+
+// F of the logarithmic mean, see plain::logmean_factor; is: 1/(a + b).
+__device__ __forceinline__ double mean_factor(double a, double b, double is, int* err) {
+    const double f = (a - b) * is, u = f * f;
+    if (u < 0.01) {
+        const double s = __builtin_fma(u, 1.0 / 7, 1.0 / 5);
+        return __builtin_fma(u, __builtin_fma(u, s, 1.0 / 3), 1.0);
+    }
+    return plain::dlog(a * rcp(b), err) * rcp(2 * f);
+}
+
+// Flux input slots: plain::put_slots and, for Chandrasekhar, |u|²/4.
+template <int ND, int TP>
+constexpr int curved_slots() {
+    return plain::tp_slots<ND, TP>() + (TP == TP_CHANDRASEKHAR ? 1 : 0);
+}
+
+// Two-point flux along the mean metric n of two nodes.
+template <int ND, int TP>
+__device__ __forceinline__ void pair_flux_along(const double* A, const double* B, const double* n, double ig1, int* err,
+                                                double* F) {
+    if constexpr (TP == TP_STDAVG) {
+        double w[2], m[2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const double* X = s ? B : A;
+            w[s] = X[0] * n[0];
+            m[s] = X[ND + 1] * n[0];
+#pragma unroll
+            for (int k = 1; k < ND; ++k) {
+                w[s] = __builtin_fma(X[k], n[k], w[s]);
+                m[s] = __builtin_fma(X[ND + 1 + k], n[k], m[s]);
+            }
+        }
+        const double p = A[ND] + B[ND];
+        F[0] = m[0] + m[1];
+#pragma unroll
+        for (int c = 0; c < ND; ++c)
+            F[1 + c] = __builtin_fma(A[ND + 1 + c], w[0], __builtin_fma(B[ND + 1 + c], w[1], p * n[c]));
+        F[ND + 1] = __builtin_fma(A[2 * ND + 1] + A[ND], w[0], (B[2 * ND + 1] + B[ND]) * w[1]);
+    } else {
+        double u[ND];
+#pragma unroll
+        for (int k = 0; k < ND; ++k) u[k] = A[1 + k] + B[1 + k];
+        double un = u[0] * n[0];
+#pragma unroll
+        for (int k = 1; k < ND; ++k) un = __builtin_fma(u[k], n[k], un);
+        const double hs = A[0] + B[0];
+        double mass, p, e;
+        if constexpr (TP == TP_CHANDRASEKHAR) {
+            const double sb = A[ND + 1] + B[ND + 1];
+            const double ir = rcp(hs), ib = rcp(sb);
+            const double fr = mean_factor(A[0], B[0], ir, err), fb = mean_factor(A[ND + 1], B[ND + 1], ib, err);
+            mass = hs * rcp(fr) * un;
+            p = hs * ib;
+            // 1/(2β̂(γ-1)) + p/ρ̂ + |ū|² - (|u1|² + |u2|²)/4
+            e = __builtin_fma(fb * ib, ig1, fr * ib) - (A[ND + 2] + B[ND + 2]);
+#pragma unroll
+            for (int k = 0; k < ND; ++k) e = __builtin_fma(u[k], u[k], e);
+            F[ND + 1] = mass * e;
+        } else {
+            p = A[ND + 1] + B[ND + 1];
+            e = A[ND + 2] + B[ND + 2];
+            mass = hs * un;
+            F[ND + 1] = __builtin_fma(mass, e, p * un);
+        }
+        F[0] = mass;
+#pragma unroll
+        for (int c = 0; c < ND; ++c) F[1 + c] = __builtin_fma(mass, u[c], p * n[c]);
+    }
+}
+
+// One direction: pairs and the nodes' own fluxes into the table, then (LOADS between) the
+// nodes' D♯ rows over it.  m: the metric row of the own node.
+template <int ND, int N, int TP, int DIR, typename LOADS>
+__device__ __forceinline__ void curved_direction(const RhsArgs<double>& a, const double* sS, const double* sM, double* sTab,
+                                                 const double* sD, int nel, int tid, int le, int node, bool valid,
+                                                 const double (&q)[ND + 2], const double (&u)[ND], double p,
+                                                 const double (&m)[ND], LOADS loads, double (&acc)[ND + 2]) {
+    using C = SCfg<ND, N>;
+    constexpr int NV = C::NV, NPF = C::NPF, SN = C::SN, NL = C::NL, NS = curved_slots<ND, TP>();
+    constexpr int KS = C::KS, VS = C::VS, DIAG = C::NPAIR * C::NLP;
+    using M = Nodes<ND, N>;
+    const double ig1 = 1.0 / (a.gamma - 1.0);
+    int lf, ii;
+    node_line<ND, N>(node, DIR, lf, ii);
+    if (valid) {
+        double* t = sTab + (DIAG + tid) * KS;
+        double w = u[0] * m[0];
+#pragma unroll
+        for (int k = 1; k < ND; ++k) w = __builtin_fma(u[k], m[k], w);
+        t[0] = q[0] * w;
+#pragma unroll
+        for (int c = 0; c < ND; ++c) t[(1 + c) * VS] = __builtin_fma(q[1 + c], w, p * m[c]);
+        t[(NV - 1) * VS] = (q[NV - 1] + p) * w;
+    }
+#pragma unroll 1
+    for (int k = tid; k < C::NPR; k += C::TPB) {
+        const int pr = k / NL, l = k - pr * NL;
+        const int le2 = C::EPB == 1 ? 0 : l / NPF, f = l - le2 * NPF;
+        if (le2 >= nel) continue;
+        const int ab = pair_ab<N>(pr);
+        const int base = le2 * M::ES + M::template line<DIR>(f);
+        constexpr int ST = M::template step<DIR>();
+        const int ia = base + (ab >> 3) * ST, ib = base + (ab & 7) * ST;
+        double A[NS], B[NS], n[ND], F[NV];
+#pragma unroll
+        for (int c = 0; c < NS; ++c) { A[c] = sS[c * SN + ia]; B[c] = sS[c * SN + ib]; }
+#pragma unroll
+        for (int c = 0; c < ND; ++c) n[c] = sM[c * SN + ia] + sM[c * SN + ib];
+        pair_flux_along<ND, TP>(A, B, n, ig1, a.errflag, F);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) sTab[(pr * C::NLP + l) * KS + v * VS] = F[v];
+    }
+    loads();
+    __syncthreads();
+    if (valid) {
+        const int diag = (DIAG + tid) * KS;
+        int off = ((ii - 1) * C::NLP + le * NPF + lf) * KS;
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const double* t = sTab + (j == ii ? diag : off);
+            const double Dij = sD[ii * N + j];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) acc[v] = __builtin_fma(-Dij, t[v * VS], acc[v]);
+            off += (j < ii ? N - j - 2 : 1) * (C::NLP * KS);
+        }
+    }
+}
+
+template <int ND, int N, int TP>
+__global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split_curved(const RhsArgs<double> a) {
+    using T = double;
+    using C = SCfg<ND, N>;
+    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, EPB = C::EPB, TPB = C::TPB, NN = C::NN, SN = C::SN;
+    constexpr int NS = curved_slots<ND, TP>(), FG = 3 * ND + 1;
+    constexpr int NFN = EPB * NF * NPF;  // face nodes of the block
+    constexpr int TAB = C::TAB, FACE = NN + NFN;
+    __shared__ T sS[NS * SN];                           // two-point flux inputs, [slot][node]
+    __shared__ T sM[ND * SN];                           // half the metric row of the direction, [component][node]
+    __shared__ T sTab[NV * (TAB > FACE ? TAB : FACE)];  // as in k_split
+    __shared__ T sD[N * N];
+
+    const int tid = threadIdx.x;
+    const int e0 = xcd_remap(blockIdx.x, gridDim.x) * EPB;
+    const int64_t Nd = a.ndofs;
+    const int nel = a.ne - e0 < EPB ? a.ne - e0 : EPB;
+    const T gamma = a.gamma;
+
+    // ---- own node, face tables, operators -----------------------------------------------
+    const int fe = tid / (NF * NPF), fk = (tid - fe * (NF * NPF)) / NPF, ff = tid % NPF;
+    const bool pf = tid < NFN && fe < nel;
+    int pinfo = 0, pnb = -1, pfgi = 0;
+    if (pf) {
+        const int slot = (e0 + fe) * NF + fk;
+        pinfo = a.finfo[slot];
+        pnb = a.nb[slot];
+        pfgi = a.fgi[slot];
+    }
+    const bool valid = tid < nel * NPE;
+    const int le = tid / NPE, node = tid - le * NPE;
+    const int64_t g0 = (int64_t)e0 * NPE;
+    const int jj = Nodes<ND, N>::node(tid);
+    T q[NV], m[ND];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) q[v] = valid ? a.Q[v * Nd + g0 + tid] : T(1);
+    auto metric = [&](int dir) {  // the own node's metric row, on its way to LDS
+#pragma unroll
+        for (int c = 0; c < ND; ++c) m[c] = valid ? a.ngeom[(c + ND * dir) * Nd + g0 + tid] : T(0);
+    };
+    auto put_metric = [&]() {
+        if (valid) {
+#pragma unroll
+            for (int c = 0; c < ND; ++c) sM[c * SN + jj] = T(0.5) * m[c];
+        }
+    };
+    metric(0);
+    for (int i = tid; i < N * N; i += TPB) sD[i] = a.ops[ops_Dsh(N) + i];
+    T u[ND], p;
+    {
+        T P[NV];
+        const Recip<T> ir(q[0]);
+        plain::cons2prim<T, ND>(q, gamma, P, ir);
+#pragma unroll
+        for (int k = 0; k < ND; ++k) u[k] = P[1 + k];
+        p = P[ND + 1];
+        if (valid) {
+            plain::put_slots<T, ND, TP, SN>(sS + jj, q, P, ir);
+            if constexpr (TP == TP_CHANDRASEKHAR) {
+                T s = u[0] * u[0];
+#pragma unroll
+                for (int k = 1; k < ND; ++k) s = __builtin_fma(u[k], u[k], s);
+                sS[(NS - 1) * SN + jj] = T(0.25) * s;
+            }
+        }
+    }
+    put_metric();
+    __syncthreads();
+
+    // ---- volume terms, direction by direction ---------------------------------------------
+    T acc[NV], pext[NV], xv[NV], pg[ND + 1], J = T(1);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[v] = T(0);
+    const T* aux = stage_aux(a);
+    auto trace = [&](int info, int nbe, int f, T* ext) {
+        const int kp = finfo_nbpos(info);
+        const T* Qn = a.Q + (int64_t)nbe * NPE +
+                      line_node<ND, N>(kp >> 1, face_nb_node<ND, N>(f, info), (kp & 1) ? N - 1 : 0);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) ext[v] = Qn[v * Nd];
+    };
+    auto frame = [&](int info, int fgi, int f, T* g) {  // the master's normal, surface J
+        const T* s = a.fgeom + ((int64_t)fgi * NPF + face_master_node<ND, N>(f, info)) * FG;
+#pragma unroll
+        for (int c = 0; c < ND; ++c) g[c] = s[c];
+        g[ND] = s[3 * ND];
+    };
+    auto prefetch = [&]() {
+        if (pf && pnb >= 0) trace(pinfo, pnb, ff, pext);
+        if (pf) frame(pinfo, pfgi, ff, pg);
+        if (valid) {
+            J = a.ngeom[ND * ND * Nd + g0 + tid];
+            if (aux) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) xv[v] = aux[v * Nd + g0 + tid];
+            }
+        }
+    };
+    curved_direction<ND, N, TP, 0>(a, sS, sM, sTab, sD, nel, tid, le, node, valid, q, u, p, m, [&]() { metric(1); }, acc);
+    put_metric();
+    __syncthreads();
+    if constexpr (ND == 3) {
+        curved_direction<ND, N, TP, 1>(a, sS, sM, sTab, sD, nel, tid, le, node, valid, q, u, p, m, [&]() { metric(2); }, acc);
+        put_metric();
+        __syncthreads();
+    }
+    curved_direction<ND, N, TP, ND - 1>(a, sS, sM, sTab, sD, nel, tid, le, node, valid, q, u, p, m, prefetch, acc);
+    __syncthreads();
+
+    // ---- numerical fluxes on the element's faces --------------------------------------------
+    T* const sU = sTab;
+    T* const sFn = sTab + NV * NN;
+    if (valid) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) sU[v * NN + tid] = q[v];
+    }
+    __syncthreads();
+    for (int it = tid; it < NFN; it += TPB) {
+        const bool first = it == tid;
+        const int le2 = it / (NF * NPF), r = it - le2 * (NF * NPF);
+        const int k = r / NPF, f = r - k * NPF;
+        if (le2 >= nel) continue;
+        const int slot = (e0 + le2) * NF + k;
+        const int info = first ? pinfo : a.finfo[slot];
+        const int nbe = first ? pnb : a.nb[slot];
+        const T* own0 = sU + le2 * NPE + line_node<ND, N>(k >> 1, f, (k & 1) ? N - 1 : 0);
+        T own[NV], ext[NV], g[ND + 1];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) own[v] = own0[v * NN];
+        if (first) {
+#pragma unroll
+            for (int c = 0; c <= ND; ++c) g[c] = pg[c];
+        } else {
+            frame(info, a.fgi[slot], f, g);
+        }
+        if (nbe >= 0) {
+            if (first) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) ext[v] = pext[v];
+            } else {
+                trace(info, nbe, f, ext);
+            }
+        } else {
+            const int bd = finfo_bd(info);
+            const int type = a.bctype[bd];
+            if (type == BC_DIRICHLET || type == BC_INFLOW) {
+                const T* src = type == BC_DIRICHLET ? a.bcstate + ((int64_t)a.fid[slot] * NPF + f) * NV
+                                                    : a.bcconst + bd * NV;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) ext[v] = src[v];
+            } else {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) ext[v] = own[v];
+                if (type == BC_SLIP) {
+                    T mn = own[1] * g[0];
+#pragma unroll
+                    for (int c = 1; c < ND; ++c) mn = mn + own[1 + c] * g[c];
+#pragma unroll
+                    for (int c = 0; c < ND; ++c) ext[1 + c] = own[1 + c] - (T(2) * mn) * g[c];
+                }
+            }
+        }
+        T mo = own[1] * g[0], mx = ext[1] * g[0];
+#pragma unroll
+        for (int c = 1; c < ND; ++c) {
+            mo = mo + own[1 + c] * g[c];
+            mx = mx + ext[1 + c] * g[c];
+        }
+        const Recip<T> iro(own[0]), irx(ext[0]);
+        const T po = plain::pressure<T, ND>(own, gamma, iro), px = plain::pressure<T, ND>(ext, gamma, irx);
+        const T uo = iro.div(mo), ux = irx.div(mx);
+        const bool slave = finfo_side(info);
+        T Fn[NV];
+        Fn[0] = (mo + mx) / T(2);
+#pragma unroll
+        for (int c = 0; c < ND; ++c) Fn[1 + c] = ((own[1 + c] * uo + ext[1 + c] * ux) + (po + px) * g[c]) / T(2);
+        Fn[NV - 1] = ((own[NV - 1] + po) * uo + (ext[NV - 1] + px) * ux) / T(2);
+        const T sg = slave ? T(-1) : T(1);
+        if (a.sdiss == DISS_LXF) {
+            const T lo = fabs(uo) + plain::dsqrt(iro.div(gamma * po), a.errflag);
+            const T lx = fabs(ux) + plain::dsqrt(irx.div(gamma * px), a.errflag);
+            // the larger speed, the master's where they do not compare
+            const T lam = sg * (slave ? ((lx < lo) ? lo : lx) : ((lo < lx) ? lx : lo));
+#pragma unroll
+            for (int v = 0; v < NV; ++v) Fn[v] = Fn[v] + ((lam * (own[v] - ext[v])) / T(2)) * a.intensity;
+        }
+        T* o = sFn + ((le2 * NF + k) * NV) * NPF + f;
+        const T js = sg * g[ND];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) o[v * NPF] = Fn[v] * js;
+    }
+    __syncthreads();
+    if (!valid) return;
+
+    // ---- FR lift on the end nodes, mass matrix and stage epilogue -----------------------------
+    const T gm0 = a.ops[ops_gm(N)], gpn = a.ops[ops_gp(N) + N - 1];
+#pragma unroll
+    for (int dir = 0; dir < ND; ++dir) {
+        int f, ii;
+        node_line<ND, N>(node, dir, f, ii);
+        if (ii == 0 || ii == N - 1) {
+            const T* s = sFn + ((le * NF + 2 * dir + (ii ? 1 : 0)) * NV) * NPF + f;
+            const T c = ii ? gpn : gm0;
+#pragma unroll
+            for (int v = 0; v < NV; ++v) acc[v] = acc[v] - c * s[v * NPF];
+        }
+    }
+    const Recip<T> iJ(J);
+    const StageOut<T> so(a);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) so.put(v * Nd + g0 + tid, iJ.div(acc[v]), q[v], xv[v]);
+}
+
+template <int ND, int N, int TP>
+static hipError_t launch_curved(const RhsArgs<double>& a, hipStream_t s) {
+    using C = SCfg<ND, N>;
+    hipLaunchKernelGGL((k_split_curved<ND, N, TP>), dim3((a.ne + C::EPB - 1) / C::EPB), dim3(C::TPB), 0, s, a);
+    return hipGetLastError();
+}
+
+template <int ND, int N>
+static RhsLauncherF64 pick_curved(int tp) {
+    switch (tp) {
+        case TP_STDAVG: return &launch_curved<ND, N, TP_STDAVG>;
+        case TP_CHANDRASEKHAR: return &launch_curved<ND, N, TP_CHANDRASEKHAR>;
+        case TP_KENNEDY_GRUBER: return &launch_curved<ND, N, TP_KENNEDY_GRUBER>;
+        default: return nullptr;
+    }
+}
+
 }  // namespace split
 
 #define FLOUHIP_CAT_(a, b) a##b
@@ -311,5 +688,20 @@ RhsLauncherF64 FLOUHIP_CAT(split_f64_, FLOUHIP_ND)(int n, int tp) {
         default: return nullptr;
     }
 }
+
+#if FLOUHIP_ND > 1
+RhsLauncherF64 FLOUHIP_CAT(split_curved_f64_, FLOUHIP_ND)(int n, int tp) {
+    switch (n) {
+        case 2: return split::pick_curved<FLOUHIP_ND, 2>(tp);
+        case 3: return split::pick_curved<FLOUHIP_ND, 3>(tp);
+        case 4: return split::pick_curved<FLOUHIP_ND, 4>(tp);
+        case 5: return split::pick_curved<FLOUHIP_ND, 5>(tp);
+        case 6: return split::pick_curved<FLOUHIP_ND, 6>(tp);
+        case 7: return split::pick_curved<FLOUHIP_ND, 7>(tp);
+        case 8: return split::pick_curved<FLOUHIP_ND, 8>(tp);
+        default: return nullptr;
+    }
+}
+#endif
 
 }  // namespace flouhip

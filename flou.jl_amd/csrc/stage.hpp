@@ -26,6 +26,13 @@ __device__ __forceinline__ int pair_ab(int pr) {
     return (int)(w >> (6 * (pr < 10 ? pr : (pr < 20 ? pr - 10 : pr - 20)))) & 63;
 }
 
+// Threads of a block of n nodes: whole waves, and eight waves for five to seven.  Only one block
+// of six waves ran on a CU where two of eight do (FP64 3-D N=6: 343 nodes, 69 to 80 KB of LDS, 100 to
+// 131 registers; 5.9 waves per CU; CK2N54 step of 16.7 M nodes 14.5 -> 8.7 ms).
+constexpr int block_threads(int n) {
+    return n > 256 && n <= 512 ? 512 : (n + 63) / 64 * 64;
+}
+
 // Node arrays of a block in LDS: with PAD one value after every row of N nodes, so that lanes on
 // consecutive x-lines, N values apart, read distinct banks for even N too.
 template <int ND, int N, bool PAD>

@@ -37,7 +37,7 @@ struct HCfg {
     static constexpr int NPE = Cfg<ND, N>::NPE, NPF = Cfg<ND, N>::NPF, NF = 2 * ND, NV = ND + 2;
     static constexpr int EPB = ND == 2 ? (N == 7 ? 5 : 192 / NPE) : Cfg<ND, N>::EPB;
     static constexpr int NN = EPB * NPE;
-    static constexpr int TPB = ((NN + 63) / 64) * 64;
+    static constexpr int TPB = block_threads(NN);
     static constexpr int NL = EPB * NPF;                 // lines per block and direction
     static constexpr int NPAIR = N * (N - 1) / 2;
     static constexpr int NPR = NL * NPAIR;

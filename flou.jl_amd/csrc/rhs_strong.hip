@@ -29,7 +29,7 @@ struct TCfg {
     static constexpr int NPE = Cfg<ND, N>::NPE, NPF = Cfg<ND, N>::NPF, NF = 2 * ND;
     static constexpr int EPB = NPE >= 256 ? 1 : 256 / NPE;
     static constexpr int NN = EPB * NPE;               // nodes per block
-    static constexpr int TPB = ((NN + 63) / 64) * 64;  // threads per block
+    static constexpr int TPB = block_threads(NN);      // threads per block
     static constexpr int NFN = EPB * NF * NPF;         // face nodes per block
     static constexpr int NR = (NFN + TPB - 1) / TPB;   // face nodes per thread
 };

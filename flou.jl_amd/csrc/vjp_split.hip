@@ -50,7 +50,9 @@ struct LCfg {
     static constexpr int NN = EPB * Nodes<ND, N>::ES;  // LDS nodes per block
     static constexpr int NL = EPB * NPF;                 // lines per block and direction
     static constexpr int WPD = (NL + 63) / 64;           // waves per direction
-    static constexpr int TPB = ND * WPD * 64;
+    // a fourth wave for the node phases where the lines fill their three (3-D N=3, 2 M nodes: 157 ->
+    // 150 us, N=7: 277 -> 261; not N=6, 49 of 64 lanes: 205 -> 209)
+    static constexpr int TPB = (ND * WPD == 3 && NL % 64 == 0 ? 4 : ND * WPD) * 64;
     static constexpr int NA = TP == TP_KENNEDY_GRUBER ? ND + 3 : ND + 2;  // node inputs = line rows
 };
 
@@ -485,11 +487,11 @@ __global__ void __launch_bounds__((LCfg<ND, N, TP>::TPB)) k_svjp(const VjpArgs<d
 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int dir = wave / C::WPD;
-    const int l = (wave - dir * C::WPD) * 64 + (tid & 63);
+    const int l = dir < ND ? (wave - dir * C::WPD) * 64 + (tid & 63) : C::NL;
     double acc[N][NA];
     if (dir == 0) line_phase<ND, N, TP, 0>(A, sP, sW, sT, sS, siw, e0, nel, l, acc);
     else if (ND == 2 || dir == 1) line_phase<ND, N, TP, 1>(A, sP, sW, sT, sS, siw, e0, nel, l, acc);
-    else line_phase<ND, N, TP, ND - 1>(A, sP, sW, sT, sS, siw, e0, nel, l, acc);
+    else if (dir == ND - 1) line_phase<ND, N, TP, ND - 1>(A, sP, sW, sT, sS, siw, e0, nel, l, acc);
     __syncthreads();  // w has been read
     if (dir == 0) add_rows<ND, N, TP, 0>(sW, nel, l, acc);
     __syncthreads();

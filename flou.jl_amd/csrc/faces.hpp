@@ -17,6 +17,12 @@ __device__ __forceinline__ int face_mom(int dir, int c) {
     return 1 + (dir + c) % ND;
 }
 
+// Place in that order of the physical momentum v (1..ND).
+template <int ND>
+__device__ __forceinline__ int face_frame(int dir, int v) {
+    return 1 + (v - 1 + ND - dir) % ND;
+}
+
 // A neighbour's trace, in the order above: node n of its element nbe.
 template <typename T, int ND, int NV>
 __device__ __forceinline__ void load_trace(const T* Qn, int64_t Nd, int dir, T* ext) {

@@ -21,6 +21,7 @@
 // Measured: 2-D N=5, 2175 elements, Chandrasekhar and MatrixDissipation: 57 -> 25.5 us per stage.
 // Compile with -DFLOUHIP_PREC_F64 or -DFLOUHIP_PREC_F32 and -DFLOUHIP_ND=1|2|3.
 #include "common.hpp"
+#include "faces.hpp"
 #include "physics_plain.hpp"
 #include "stage.hpp"
 
@@ -305,8 +306,254 @@ __global__ void __launch_bounds__((HCfg<ND, N>::TPB)) k_hybrid(const RhsArgs<T> 
     for (int v = 0; v < NV; ++v) so.put(v * Nd + g0 + tid, iJ.div(acc[v]), q[v], xv[v]);
 }
 
+// ---- axis-aligned elements in 1-D and 2-D --------------------------------------------------------
+//
+// A thread group of two waves per direction: the pair tables of all directions are filled at
+// once, then one flux per thread: the N-1 interfaces of a line and its two faces (positions 0
+// and N) are items of the same kind, whose numerical fluxes (the longest chain of dependent
+// operations here) run side by side.  Small meshes, a block or two per CU, are bound by that
+// chain (2175 elements: 3 waves per CU, VALU 26 % busy): six rounds of pairs and three of
+// fluxes in k_hybrid, three and one here.  Faces read the order of their frame by index
+// (faces.hpp), neighbours' traces are loaded before the pairs.
+// Measured, N=5, Chandrasekhar and MatrixDissipation, 2175 elements: 25.6 -> 21 us per stage.
+template <int ND, int N>
+struct LCfg {
+    static constexpr int NPE = Cfg<ND, N>::NPE, NPF = Cfg<ND, N>::NPF, NF = 2 * ND, NV = ND + 2;
+    static constexpr int G = 128, TPB = ND * G;          // threads per direction and block
+    static constexpr int EPB = G / (NPF * (N + 1));      // an item per thread
+    static constexpr int NN = EPB * NPE;
+    static constexpr int NL = EPB * NPF;                 // lines per direction
+    static constexpr int NPAIR = N * (N - 1) / 2;
+    static constexpr int NPR = NL * NPAIR;
+    static constexpr int SN = EPB * Nodes<ND, N>::ES;
+    static constexpr int TAB = NV * (NPAIR > N + 1 ? NPR : (N + 1) * NL);
+};
+
+template <typename T, int ND, int N, int TP, int DIR>
+__device__ __forceinline__ void line_pairs(const T* sS, const T* sQ, T* sTab, T ja, T gm1, int* err, int nel, int i) {
+    using C = LCfg<ND, N>;
+    using M = Nodes<ND, N>;
+    constexpr int NV = C::NV, SN = C::SN, NS = plain::tp_slots<ND, TP>(), NSL = lds_slots<ND, TP>();
+    constexpr int ST = M::template step<DIR>();
+#pragma unroll 1
+    for (int k = i; k < C::NPR; k += C::G) {
+        const int pr = k / C::NL, l = k - pr * C::NL;
+        const int le = l / C::NPF, f = l - le * C::NPF;
+        if (le >= nel) continue;
+        const int ab = pair_ab<N>(pr);
+        const int base = le * M::ES + M::template line<DIR>(f);
+        const int ia = base + (ab >> 3) * ST, ib = base + (ab & 7) * ST;
+        T A[NS], B[NS], F[NV];
+#pragma unroll
+        for (int c = 0; c < NS; ++c) {  // StdAverage's conservative slots lie in sQ
+            A[c] = c < NSL ? sS[c * SN + ia] : T(0.5) * sQ[(1 + c - NSL) * SN + ia];
+            B[c] = c < NSL ? sS[c * SN + ib] : T(0.5) * sQ[(1 + c - NSL) * SN + ib];
+        }
+        plain::pair_flux<T, ND, TP, DIR>(A, B, ja, gm1, err, F);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) sTab[v * C::NPR + k] = F[v];
+    }
+}
+
+template <typename T, int ND, int N, int TP>
+__global__ void __launch_bounds__((LCfg<ND, N>::TPB)) k_hybrid_lines(const RhsArgs<T> a) {
+    using C = LCfg<ND, N>;
+    using M = Nodes<ND, N>;
+    constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, EPB = C::EPB, TPB = C::TPB, NL = C::NL, SN = C::SN;
+    __shared__ T sS[lds_slots<ND, TP>() * SN];  // two-point flux inputs
+    __shared__ T sQ[NV * SN];                   // conservative states
+    __shared__ T sW[NV * SN];                   // entropy variables
+    __shared__ T sTab[ND][C::TAB];              // pair fluxes, then the fluxes at positions 0..N
+    __shared__ T sC[N * N], sw[N];
+
+    const int tid = threadIdx.x;
+    const int e0 = xcd_remap(blockIdx.x, gridDim.x) * EPB;
+    const int64_t Nd = a.ndofs, g0 = (int64_t)e0 * NPE;
+    const int nel = a.ne - e0 < EPB ? a.ne - e0 : EPB;
+    const bool valid = tid < nel * NPE;
+    const int le = tid / NPE, node = tid - le * NPE;
+
+    // ---- the thread's item: position s of line l of its direction --------------------------
+    const int dir = ND == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / C::G), it = tid - dir * C::G;
+    const int s = it / NL, l = it - s * NL, fe = l / NPF, ff = l - fe * NPF;
+    const bool item = s <= N && fe < nel, face = item && (s == 0 || s == N);
+    int info = 0, nbe = -1, slot = 0, fgi = 0;
+    if (face) {
+        slot = (e0 + fe) * NF + 2 * dir + (s == N ? 1 : 0);
+        info = a.finfo[slot];
+        nbe = a.nb[slot];
+        fgi = a.fgi[slot];
+    }
+    T q[NV], xv[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) q[v] = valid ? a.Q[v * Nd + g0 + tid] : T(1);
+    const T* aux = stage_aux(a);
+    if (aux && valid) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) xv[v] = aux[v * Nd + g0 + tid];
+    }
+    for (int i = tid; i < N * N; i += TPB) sC[i] = (T(2) * a.ops[ops_w(N) + i / N]) * a.ops[ops_D(N) + i];
+    for (int i = tid; i < N; i += TPB) sw[i] = a.ops[ops_w(N) + i];
+    T ext[NV], sn = T(1), fj = T(1);
+    if (face) {
+        if (nbe >= 0) {
+            const int kp = finfo_nbpos(info);
+            load_trace<T, ND, NV>(a.Q + (int64_t)nbe * NPE +
+                                      line_node<ND, N>(kp >> 1, face_nb_node<ND, N>(ff, info), (kp & 1) ? N - 1 : 0),
+                                  Nd, dir, ext);
+        }
+        const T* g = a.fgeom + (int64_t)fgi * (3 * ND + 1);
+        sn = g[dir];
+        fj = g[3 * ND];
+    }
+    if (valid) {
+        T P[NV], W[NV];
+        const Recip<T> ir(q[0]);
+        plain::cons2prim<T, ND>(q, a.gamma, P, ir);
+        const int j = M::node(tid);
+        plain::put_slots<T, ND, TP, SN, false>(sS + j, q, P, ir);
+        plain::cons2entropy<T, ND>(q, a.gamma, a.errflag, W);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            sQ[v * SN + j] = q[v];
+            sW[v * SN + j] = W[v];
+        }
+    }
+    __syncthreads();
+
+    // ---- pair fluxes, each once ----------------------------------------------------------------
+    T* const tab = sTab[dir];
+    const T gm1 = a.gamma - T(1);
+    if (dir == 0) line_pairs<T, ND, N, TP, 0>(sS, sQ, tab, a.egeom[0], gm1, a.errflag, nel, it);
+    else line_pairs<T, ND, N, TP, ND - 1>(sS, sQ, tab, a.egeom[ND * ND - 1], gm1, a.errflag, nel, it);
+    __syncthreads();
+
+    // ---- the item's flux ---------------------------------------------------------------------
+    T Fx[NV];
+    if (item) {
+        const int base = fe * M::ES + (dir == 0 ? M::template line<0>(ff) : M::template line<ND - 1>(ff));
+        const int st = dir == 0 ? M::template step<0>() : M::template step<ND - 1>();
+        // lower and upper node; for a face its own node, and the sides' order is the master's
+        const int nr = base + (s < N ? s : N - 1) * st, nl = s == 0 || s == N ? nr : nr - st;
+        T Rl[NV], Rr[NV], Vl[NV], Vr[NV], Fr[NV];
+        load_trace<T, ND, NV>(sQ + nl, SN, dir, Rl);
+        load_trace<T, ND, NV>(sW + nl, SN, dir, Vl);
+        load_trace<T, ND, NV>(sQ + nr, SN, dir, Rr);
+        load_trace<T, ND, NV>(sW + nr, SN, dir, Vr);
+        const bool slave = face && finfo_side(info);
+        if (face) {
+            if (nbe < 0) boundary_trace<T, ND, NPF, NV>(a, info, slot, ff, dir, Rl, ext);
+            T W[NV];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) W[v] = T(0);
+            if (a.sdiss == DISS_MATRIX) plain::cons2entropy<T, ND>(ext, a.gamma, a.errflag, W);
+            Rl[1] = sn * Rl[1]; Rr[1] = sn * Rr[1]; ext[1] = sn * ext[1];
+            Vl[1] = sn * Vl[1]; Vr[1] = sn * Vr[1]; W[1] = sn * W[1];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                if (slave) { Rl[v] = ext[v]; Vl[v] = W[v]; }
+                else { Rr[v] = ext[v]; Vr[v] = W[v]; }
+            }
+        }
+        plain::euler_numericalflux<T, ND>(Rl, Rr, a.savg, a.sdiss, a.typo, a.intensity, a.gamma, a.errflag, Fr, Vl, Vr);
+        if (face) {
+            Fr[1] = sn * Fr[1];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const T x = Fr[v] * fj;
+                Fr[v] = slave ? -x : x;
+            }
+        } else {
+            T Fb[NV];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) Fb[v] = T(0);
+            for (int ik = s; ik < N; ++ik)
+                for (int il = 0; il < s; ++il) {
+                    const int pr = il * (2 * N - il - 1) / 2 + (ik - il - 1);
+                    const T* t = tab + pr * NL + l;
+                    const T c = sC[il * N + ik];
+#pragma unroll
+                    for (int v = 0; v < NV; ++v) Fb[v] = Fb[v] + c * t[v * C::NPR];
+                }
+            T Fv[NV], b = T(0);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) Fv[v] = Fr[v] * a.sjac[dir];
+            // the entropy production, summed over the physical variables in their order
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const int w = v == 0 || v == NV - 1 ? v : face_frame<ND>(dir, v);
+                const T x = (Vr[w] - Vl[w]) * (Fb[v] - Fv[w]);
+                b = v == 0 ? x : b + x;
+            }
+            const T dl = plain::hybrid_delta(b, a.blend, a.errflag);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const int w = v == 0 || v == NV - 1 ? v : face_frame<ND>(dir, v);
+                Fx[v] = (T(1) - dl) * Fv[w] + dl * Fb[v];
+            }
+        }
+        if (face) {
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const int w = v == 0 || v == NV - 1 ? v : face_frame<ND>(dir, v);
+                Fx[v] = Fr[w];
+            }
+        }
+    }
+    __syncthreads();  // the tables have been read
+    if (item) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) tab[(v * (N + 1) + s) * NL + l] = Fx[v];
+    }
+    __syncthreads();
+    if (!valid) return;
+
+    // ---- interface differences, FR lift, mass matrix and stage epilogue --------------------------
+    T acc[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[v] = T(0);
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        int f, ii;
+        node_line<ND, N>(node, d, f, ii);
+        const Recip<T> iw(sw[ii]);
+        const T* t = sTab[d] + ii * NL + le * NPF + f;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const T x = ii == 0 ? T(0) : t[v * (N + 1) * NL];
+            const T y = ii == N - 1 ? T(0) : t[(v * (N + 1) + 1) * NL];
+            acc[v] = acc[v] + iw.div(x - y);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        int f, ii;
+        node_line<ND, N>(node, d, f, ii);
+        const T gm = a.ops[ops_gm(N) + ii], gp = a.ops[ops_gp(N) + ii];
+        const T* t = sTab[d] + le * NPF + f;
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+            acc[v] = acc[v] - (gm * t[v * (N + 1) * NL] + gp * t[(v * (N + 1) + N) * NL]);
+    }
+    const Recip<T> iJ(a.egeom[ND * ND]);
+    const StageOut<T> so(a);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) so.put(v * Nd + g0 + tid, iJ.div(acc[v]), q[v], xv[v]);
+}
+
 template <typename T, int ND, int N, int TP, bool DIAG>
 static hipError_t launch(const RhsArgs<T>& a, hipStream_t s) {
+    // small meshes: blocks that all run at once (three per CU in FP64, six in FP32); N nodes per
+    // line, 2-D, matrix dissipation, k_hybrid and k_hybrid_lines: FP64 N=6, 540 blocks 16.9 and 12.2
+    // us, 740 23.8 and 19.8, N=5, 800 21.1 and 22.2, 4000 65 and 72
+    if constexpr (DIAG && ND <= 2) {
+        using L = LCfg<ND, N>;
+        const int nb = (a.ne + L::EPB - 1) / L::EPB;
+        if (nb <= (sizeof(T) == 8 ? 768 : 1536)) {
+            hipLaunchKernelGGL((k_hybrid_lines<T, ND, N, TP>), dim3(nb), dim3(L::TPB), 0, s, a);
+            return hipGetLastError();
+        }
+    }
     using C = HCfg<ND, N>;
     hipLaunchKernelGGL((k_hybrid<T, ND, N, TP, DIAG>), dim3((a.ne + C::EPB - 1) / C::EPB), dim3(C::TPB), 0, s, a);
     return hipGetLastError();

@@ -215,6 +215,8 @@ RhsLauncherF32 hybrid_f32_3(int n, int tp, bool diag);
 // FP64 split-form Euler kernels on axis-aligned affine elements, GLL nodes, StdAverage or
 // LxF(StdAverage) surface flux (rhs_split.hip): the plain kernels' results.
 RhsLauncherF64 split_f64_1(int n, int tp);
+// 1-D with any surface flux, null where ne elements are too many
+RhsLauncherF64 split_f64_1_small(int n, int tp, int64_t ne);
 RhsLauncherF64 split_f64_2(int n, int tp);
 RhsLauncherF64 split_f64_3(int n, int tp);
 // the same on curved elements, up to rounding

@@ -7,13 +7,13 @@
 //   * a node's primitives are formed once, for the contravariant fluxes of all directions, each
 //     of one term (the metric is diagonal), and stay in registers;
 //   * the fluxes lie in LDS in vectors of 16 bytes, so that a line's entry is one or two reads;
-//   * face tables are loaded beside the node states and the neighbours' traces before the
-//     volume sums, which hide them: two dependent global loads from start to end;
+//   * all loads come first, the face tables, then the node's state and the neighbours' traces:
+//     two dependent global loads from start to end;
 //   * faces as in faces.hpp; the lift touches the end nodes only (∂g is exactly zero elsewhere);
 //   * FP32 sums with fused multiply-adds (one rounding less per term).
-// Measured against k_plain, rhs, 0.9 M nodes, Euler, N nodes per line: 3-D N=5 FP32 37.8 -> 22 us,
-// FP64 72 -> 38; 3-D N=8 FP32 46 -> 18, FP64 130 -> 33; 2-D N=6 FP32 20.5 -> 13.3, FP64 37 -> 21.  An
-// SSPRK33 step of 7182 elements, 3-D N=5, FP32: 116 -> 64 us; ten of advection on 256 elements, 2-D
+// Measured against k_plain, rhs, 0.9 M nodes, Euler, N nodes per line: 3-D N=5 FP32 37.8 -> 20 us,
+// FP64 72 -> 36; 3-D N=8 FP32 46 -> 17, FP64 130 -> 33; 2-D N=6 FP32 20.5 -> 12.4, FP64 37 -> 20.  An
+// SSPRK33 step of 7182 elements, 3-D N=5, FP32: 116 -> 60 us; ten of advection on 256 elements, 2-D
 // N=5, FP64: 163 -> 148 us.  Blocks of 128 threads: 2-D N=6 FP32 15.8 us, FP64 26.
 // Compile with -DFLOUHIP_PREC_F64 or -DFLOUHIP_PREC_F32 and -DFLOUHIP_ND=1|2|3.
 #include "common.hpp"
@@ -63,6 +63,8 @@ struct Table {
     }
 };
 
+__device__ __forceinline__ double madd(double a, double b, double c) { return a * b + c; }
+__device__ __forceinline__ float madd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double msub(double a, double b, double c) { return a - b * c; }
 __device__ __forceinline__ float msub(float a, float b, float c) { return __builtin_fmaf(-b, c, a); }
 
@@ -90,27 +92,49 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
     const int le = tid / NPE, node = tid - le * NPE;
     const T avel[3] = {a.a0, a.a1, a.a2};
 
-    // ---- face tables, own node, element geometry, operators --------------------------------
+    // ---- loads: face tables, own node, geometry; then what depends on the tables -------------
+    // (spare lanes and boundary faces load something valid instead of branching)
     int fs[NR], info[NR], nbe[NR], fgi[NR];
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
         const int it = tid + r * TPB;
-        fs[r] = it < nel * NF * NPF ? e0 * NF + it / NPF : -1;  // face slot of face node `it`
-        if (fs[r] >= 0) {
-            info[r] = a.finfo[fs[r]];
-            nbe[r] = a.nb[fs[r]];
-            fgi[r] = a.fgi[fs[r]];
-        }
+        fs[r] = e0 * NF + (it < nel * NF * NPF ? it / NPF : 0);  // face slot of face node `it`
+        info[r] = a.finfo[fs[r]];
+        nbe[r] = a.nb[fs[r]];
+        fgi[r] = a.fgi[fs[r]];
     }
+    const int tn = valid ? tid : 0;
     T q[NV];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) q[v] = valid ? a.Q[v * Nd + g0 + tid] : T(1);
+    for (int v = 0; v < NV; ++v) q[v] = (a.Q + (v * Nd + g0))[tn];
     const T* eg = a.egeom + (int64_t)(valid ? e0 + le : e0) * a.egeom_stride;
     T ja[ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d) ja[d] = eg[d * (ND + 1)];
     const T jac = eg[ND * ND];
-    for (int i = tid; i < N * N; i += TPB) sD[i] = a.ops[ops_Ds(N) + i];
+    const T Dv = a.ops[ops_Ds(N) + (tid < N * N ? tid : 0)];
+    T own[NR][NV], ext[NR][NV], sn[NR], fj[NR], xv[NV];
+    const T* aux = stage_aux(a);
+    if (aux) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) xv[v] = (aux + (v * Nd + g0))[tn];
+    }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+        const int it = tid + r * TPB;
+        const int k = (it / NPF) % NF, f = it % NPF, dir = k >> 1;
+        const int kp = nbe[r] >= 0 ? finfo_nbpos(info[r]) : 0;
+        load_trace<T, ND, NV>(a.Q + (int64_t)(nbe[r] >= 0 ? nbe[r] : e0) * NPE +
+                                  line_node<ND, N>(kp >> 1, f, (kp & 1) ? N - 1 : 0),
+                              Nd, dir, ext[r]);
+        if constexpr (GLB) {
+            const int le2 = it < nel * NF * NPF ? it / (NF * NPF) : 0;
+            load_trace<T, ND, NV>(a.Q + g0 + le2 * NPE + line_node<ND, N>(dir, f, (k & 1) ? N - 1 : 0), Nd, dir, own[r]);
+        }
+        const T* g = a.fgeom + (int64_t)fgi[r] * (3 * ND + 1);
+        sn[r] = g[dir];
+        fj[r] = g[3 * ND];
+    }
 
     // ---- contravariant fluxes ------------------------------------------------------------
     T F[ND][NV];
@@ -120,7 +144,17 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
     } else {
         T P[NV];
         const Recip<T> ir(q[0]);
-        plain::cons2prim<T, ND>(q, a.gamma, P, ir);
+        if constexpr (sizeof(T) == 4) {
+            T m2 = T(0);
+#pragma unroll
+            for (int c = 0; c < ND; ++c) {
+                P[1 + c] = ir.fin(q[1 + c]);
+                m2 = __builtin_fmaf(q[1 + c], q[1 + c], m2);
+            }
+            P[ND + 1] = (a.gamma - T(1)) * __builtin_fmaf(T(-0.5), ir.fin(m2), q[ND + 1]);
+        } else {
+            plain::cons2prim<T, ND>(q, a.gamma, P, ir);
+        }
         const T p = P[ND + 1];
 #pragma unroll
         for (int d = 0; d < ND; ++d) {
@@ -128,7 +162,7 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
             F[d][0] = q[1 + d] * ja[d];
 #pragma unroll
             for (int c = 0; c < ND; ++c)
-                F[d][1 + c] = (c == d ? q[1 + d] * P[1 + c] + p : q[1 + d] * P[1 + c]) * ja[d];
+                F[d][1 + c] = (c == d ? madd(q[1 + d], P[1 + c], p) : q[1 + d] * P[1 + c]) * ja[d];
             F[d][NV - 1] = ((q[NV - 1] + p) * u) * ja[d];
         }
     }
@@ -141,31 +175,7 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
         }
     }
 
-    // ---- neighbours' traces, face geometry and the epilogue's operand: in flight from here -----
-    T own[NR][NV], ext[NR][NV], sn[NR], fj[NR], xv[NV];
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-        if (fs[r] >= 0) {
-            const int it = tid + r * TPB;
-            const int k = (it / NPF) % NF, f = it % NPF, dir = k >> 1;
-            if constexpr (GLB)
-                load_trace<T, ND, NV>(
-                    a.Q + g0 + it / (NF * NPF) * NPE + line_node<ND, N>(dir, f, (k & 1) ? N - 1 : 0), Nd, dir, own[r]);
-            if (nbe[r] >= 0) {
-                const int kp = finfo_nbpos(info[r]);
-                load_trace<T, ND, NV>(a.Q + (int64_t)nbe[r] * NPE + line_node<ND, N>(kp >> 1, f, (kp & 1) ? N - 1 : 0),
-                                      Nd, dir, ext[r]);
-            }
-            const T* g = a.fgeom + (int64_t)fgi[r] * (3 * ND + 1);
-            sn[r] = g[dir];
-            fj[r] = g[3 * ND];
-        }
-    }
-    const T* aux = stage_aux(a);
-    if (aux && valid) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) xv[v] = aux[v * Nd + g0 + tid];
-    }
+    if (tid < N * N) sD[tid] = Dv;
     __syncthreads();
 
     // ---- volume terms, in the reference's order ------------------------------------------------
@@ -193,8 +203,8 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
     // ---- numerical fluxes on the element's faces --------------------------------------------------
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-        if (fs[r] < 0) continue;
         const int it = tid + r * TPB;
+        if (it >= nel * NF * NPF) continue;
         const int k = (it / NPF) % NF, f = it % NPF, dir = k >> 1;
         if constexpr (!GLB)
             load_trace<T, ND, NV>(sQ + it / (NF * NPF) * NPE + line_node<ND, N>(dir, f, (k & 1) ? N - 1 : 0), NN, dir,
@@ -210,7 +220,10 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
             o[0] = Fn * (sg * fj[r]);
         } else {
             T Fn[NV];
-            axis_flux<T, ND>(own[r], ext[r], sn[r], fj[r], slave, a.sdiss, a.gamma, a.intensity, a.errflag, Fn);
+            if constexpr (sizeof(T) == 4)
+                axis_flux_f32<ND>(own[r], ext[r], sn[r], fj[r], slave, a.sdiss, a.gamma, a.intensity, a.errflag, Fn);
+            else
+                axis_flux<T, ND>(own[r], ext[r], sn[r], fj[r], slave, a.sdiss, a.gamma, a.intensity, a.errflag, Fn);
             o[0] = Fn[0];
 #pragma unroll
             for (int c = 0; c < ND; ++c) o[face_mom<ND>(dir, c) * NPF] = Fn[1 + c];
@@ -230,13 +243,13 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
             const T* s = sFn + (le * NF + 2 * d + (ii ? 1 : 0)) * (NV * NPF) + f;
             const T c = ii ? gpn : gm0;
 #pragma unroll
-            for (int v = 0; v < NV; ++v) acc[v] = acc[v] - c * s[v * NPF];
+            for (int v = 0; v < NV; ++v) acc[v] = msub(acc[v], c, s[v * NPF]);
         }
     }
     const Recip<T> iJ(jac);
     const StageOut<T> so(a);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) so.put(v * Nd + g0 + tid, iJ.div(acc[v]), q[v], xv[v]);
+    for (int v = 0; v < NV; ++v) so.put(v * Nd + g0 + tid, sizeof(T) == 4 ? iJ.fin(acc[v]) : iJ.div(acc[v]), q[v], xv[v]);
 }
 
 template <typename T, int ND, int N, int EQ>

@@ -438,170 +438,6 @@ static RhsLauncherF64 pick_tp(int tp) {
     }
 }
 
-// ---- 1-D ----------------------------------------------------------------------------------------
-//
-// Meshes of a few dozen to some ten thousand nodes: bound by the chain of dependent operations,
-// not by any rate.  Two waves take the nodes and pairs and two the faces, which read their traces from
-// memory and wait for nothing: the surface flux (any of the framework's) runs beside the pairs.
-// Measured, ORK256 steps of 20 elements, N=3, Chandrasekhar and
-// MatrixDissipation: 8.3 -> 7.3 us per stage.
-template <int N>
-struct ECfg {
-    static constexpr int G = 128, TPB = 2 * G;
-    static constexpr int NPAIR = N * (N - 1) / 2;
-    static constexpr int EPB = N == 2 ? 64 : G / NPAIR;  // a pair per thread
-    static constexpr int NN = EPB * N;
-};
-
-template <int N, int TP>
-__global__ void __launch_bounds__((ECfg<N>::TPB)) k_split_1d(const RhsArgs<double> a) {
-    using T = double;
-    using C = ECfg<N>;
-    constexpr int NV = 3, EPB = C::EPB, NN = C::NN, NS = plain::tp_slots<1, TP>(), NPAIR = C::NPAIR;
-    __shared__ T sS[NS * NN];            // two-point flux inputs
-    __shared__ T sTab[NV][EPB * NPAIR];  // pair fluxes
-    __shared__ T sFn[NV][2 * EPB];       // face fluxes
-    const int tid = threadIdx.x;
-    const int e0 = xcd_remap(blockIdx.x, gridDim.x) * EPB;
-    const int64_t Nd = a.ndofs, g0 = (int64_t)e0 * N;
-    const int nel = a.ne - e0 < EPB ? a.ne - e0 : EPB;
-    if (tid >= C::G) {
-        const int it = tid - C::G, le = it >> 1, k = it & 1;
-        const bool task = le < nel;
-        T own[NV], ext[NV], F[NV];
-        if (task) {
-            const int slot = (e0 + le) * 2 + k;
-            const int info = a.finfo[slot], nbe = a.nb[slot];
-            const T* g = a.fgeom + (int64_t)a.fgi[slot] * 4;
-            load_trace<T, 1, NV>(a.Q + (int64_t)(e0 + le) * N + (k ? N - 1 : 0), Nd, 0, own);
-            const T sn = g[0], jac = g[3];
-            if (nbe >= 0)
-                load_trace<T, 1, NV>(a.Q + (int64_t)nbe * N + ((finfo_nbpos(info) & 1) ? N - 1 : 0), Nd, 0, ext);
-            else
-                boundary_trace<T, 1, 1, NV>(a, info, slot, 0, 0, own, ext);
-            own[1] = sn * own[1];
-            ext[1] = sn * ext[1];
-            const bool slave = finfo_side(info);
-            T L[NV], R[NV];
-#pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                L[v] = slave ? ext[v] : own[v];
-                R[v] = slave ? own[v] : ext[v];
-            }
-            plain::euler_numericalflux<T, 1>(L, R, a.savg, a.sdiss, a.typo, a.intensity, a.gamma, a.errflag, F);
-            F[1] = sn * F[1];
-#pragma unroll
-            for (int v = 0; v < NV; ++v) {
-                const T x = F[v] * jac;
-                sFn[v][it] = slave ? -x : x;
-            }
-        }
-        __syncthreads();
-        __syncthreads();
-        return;
-    }
-    const bool valid = tid < nel * N;
-    const int le = tid / N, ii = tid - le * N;
-    const T ja = a.egeom[0 + (int64_t)(valid ? e0 + le : e0) * a.egeom_stride];
-    const T J = a.egeom[1 + (int64_t)(valid ? e0 + le : e0) * a.egeom_stride];
-    T q[NV], xv[NV], D[N];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) q[v] = valid ? a.Q[v * Nd + g0 + tid] : T(1);
-    const T* aux = stage_aux(a);
-    if (aux && valid) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) xv[v] = aux[v * Nd + g0 + tid];
-    }
-#pragma unroll
-    for (int j = 0; j < N; ++j) D[j] = a.ops[ops_Dsh(N) + ii * N + j];
-    const T gm0 = a.ops[ops_gm(N)], gpn = a.ops[ops_gp(N) + N - 1];
-    T own[NV];  // the node's contravariant flux
-    {
-        T P[NV];
-        const Recip<T> ir(q[0]);
-        plain::cons2prim<T, 1>(q, a.gamma, P, ir);
-        if (valid) plain::put_slots<T, 1, TP, NN>(sS + tid, q, P, ir);
-        own[0] = q[1] * ja;
-        own[1] = (q[1] * P[1] + P[2]) * ja;
-        own[2] = ((q[2] + P[2]) * P[1]) * ja;
-    }
-    __syncthreads();
-    {
-        const int pr = tid / EPB, l = tid - pr * EPB;
-        if (pr < NPAIR && l < nel) {
-            const int ab = pair_ab<N>(pr);
-            const T* sa = sS + l * N + (ab >> 3);
-            const T* sb = sS + l * N + (ab & 7);
-            T A[NS], B[NS], F[NV];
-#pragma unroll
-            for (int c = 0; c < NS; ++c) { A[c] = sa[c * NN]; B[c] = sb[c * NN]; }
-            const T jl = a.egeom[(int64_t)(e0 + l) * a.egeom_stride];
-            plain::pair_flux<T, 1, TP, 0>(A, B, jl, a.gamma - T(1), a.errflag, F);
-#pragma unroll
-            for (int v = 0; v < NV; ++v) sTab[v][tid] = F[v];
-        }
-    }
-    __syncthreads();
-    if (!valid) return;
-    T acc[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) acc[v] = T(0);
-    int off = (ii - 1) * EPB + le;  // as in direction()
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) acc[v] = acc[v] - D[j] * (j == ii ? own[v] : sTab[v][j == ii ? 0 : off]);
-        off += (j < ii ? N - j - 2 : 1) * EPB;
-    }
-    if (ii == 0 || ii == N - 1) {
-        const T c = ii ? gpn : gm0;
-#pragma unroll
-        for (int v = 0; v < NV; ++v) acc[v] = acc[v] - c * sFn[v][2 * le + (ii ? 1 : 0)];
-    }
-    const Recip<T> iJ(J);
-    const StageOut<T> so(a);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) so.put(v * Nd + g0 + tid, iJ.div(acc[v]), q[v], xv[v]);
-}
-
-template <int ND, int N, int TP>
-static hipError_t launch(const RhsArgs<double>& a, hipStream_t s) {
-    using C = SCfg<ND, N>;
-    hipLaunchKernelGGL((k_split<ND, N, TP>), dim3((a.ne + C::EPB - 1) / C::EPB), dim3(C::TPB), 0, s, a);
-    return hipGetLastError();
-}
-
-template <int N, int TP>
-static hipError_t launch_1d(const RhsArgs<double>& a, hipStream_t s) {
-    using C = ECfg<N>;
-    hipLaunchKernelGGL((k_split_1d<N, TP>), dim3((a.ne + C::EPB - 1) / C::EPB), dim3(C::TPB), 0, s, a);
-    return hipGetLastError();
-}
-
-// While all blocks run at once; of larger meshes k_split takes those with the LxF flux, the general
-// kernel the rest (Chandrasekhar and matrix dissipation, general kernel and k_split_1d: N=3, 952 blocks
-// 10.7 and 10.4 us, 2381 13.1 and 14.3; N=7, 625 10.6 and 10.3, 6250 15.3 and 29.5).
-template <int N>
-static RhsLauncherF64 pick_1d(int tp, int64_t ne) {
-    if ((ne + ECfg<N>::EPB - 1) / ECfg<N>::EPB > 1024) return nullptr;
-    switch (tp) {
-        case TP_STDAVG: return &launch_1d<N, TP_STDAVG>;
-        case TP_CHANDRASEKHAR: return &launch_1d<N, TP_CHANDRASEKHAR>;
-        case TP_KENNEDY_GRUBER: return &launch_1d<N, TP_KENNEDY_GRUBER>;
-        default: return nullptr;
-    }
-}
-
-template <int ND, int N>
-static RhsLauncherF64 pick_tp(int tp) {
-    switch (tp) {
-        case TP_STDAVG: return &launch<ND, N, TP_STDAVG>;
-        case TP_CHANDRASEKHAR: return &launch<ND, N, TP_CHANDRASEKHAR>;
-        case TP_KENNEDY_GRUBER: return &launch<ND, N, TP_KENNEDY_GRUBER>;
-        default: return nullptr;
-    }
-}
-
 // ---- curved elements --------------------------------------------------------------------------
 //
 // The same form with a metric per node.  The general kernel forms every component of a pair's
@@ -749,10 +585,8 @@ __device__ __forceinline__ void curved_direction(const RhsArgs<double>& a, const
     }
 }
 
-// (3-D N=6: 128 registers, so that two blocks of eight waves fit a CU; with 132 one block ran, 2.95 ->
-// 4.65 ms)
 template <int ND, int N, int TP>
-__global__ void __launch_bounds__((SCfg<ND, N>::TPB), (ND == 3 && N == 7 ? 4 : 1)) k_split_curved(const RhsArgs<double> a) {
+__global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split_curved(const RhsArgs<double> a) {
     using T = double;
     using C = SCfg<ND, N>;
     constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, EPB = C::EPB, TPB = C::TPB, NN = C::NN, SN = C::SN;
@@ -773,19 +607,23 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB), (ND == 3 && N == 7 ? 4 : 1
     // ---- own node, face tables, operators -----------------------------------------------
     const int fe = tid / (NF * NPF), fk = (tid - fe * (NF * NPF)) / NPF, ff = tid % NPF;
     const bool pf = tid < NFN && fe < nel;
-    const int pslot = e0 * NF + (pf ? fe * NF + fk : 0);  // (spare lanes: as in k_split)
-    const int pinfo = a.finfo[pslot], pnb = a.nb[pslot], pfgi = a.fgi[pslot];
+    int pinfo = 0, pnb = -1, pfgi = 0;
+    if (pf) {
+        const int slot = (e0 + fe) * NF + fk;
+        pinfo = a.finfo[slot];
+        pnb = a.nb[slot];
+        pfgi = a.fgi[slot];
+    }
     const bool valid = tid < nel * NPE;
-    const int tn = valid ? tid : 0;
     const int le = tid / NPE, node = tid - le * NPE;
     const int64_t g0 = (int64_t)e0 * NPE;
     const int jj = Nodes<ND, N>::node(tid);
     T q[NV], m[ND];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) q[v] = (a.Q + (v * Nd + g0))[tn];
+    for (int v = 0; v < NV; ++v) q[v] = valid ? a.Q[v * Nd + g0 + tid] : T(1);
     auto metric = [&](int dir) {  // the own node's metric row, on its way to LDS
 #pragma unroll
-        for (int c = 0; c < ND; ++c) m[c] = (a.ngeom + ((c + ND * dir) * Nd + g0))[tn];
+        for (int c = 0; c < ND; ++c) m[c] = valid ? a.ngeom[(c + ND * dir) * Nd + g0 + tid] : T(0);
     };
     auto put_metric = [&]() {
         if (valid) {
@@ -794,8 +632,7 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB), (ND == 3 && N == 7 ? 4 : 1
         }
     };
     metric(0);
-    static_assert(N * N <= TPB, "one operator entry per thread");
-    const T Dv = a.ops[ops_Dsh(N) + (tid < N * N ? tid : 0)];
+    for (int i = tid; i < N * N; i += TPB) sD[i] = a.ops[ops_Dsh(N) + i];
     T u[ND], p;
     {
         T P[NV];
@@ -815,7 +652,6 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB), (ND == 3 && N == 7 ? 4 : 1
         }
     }
     put_metric();
-    if (tid < N * N) sD[tid] = Dv;
     __syncthreads();
 
     // ---- volume terms, direction by direction ---------------------------------------------
@@ -837,12 +673,14 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB), (ND == 3 && N == 7 ? 4 : 1
         g[ND] = s[3 * ND];
     };
     auto prefetch = [&]() {
-        trace(pnb >= 0 ? pinfo : 0, pnb >= 0 ? pnb : e0, ff, pext);
-        frame(pinfo, pfgi, ff, pg);
-        J = (a.ngeom + (ND * ND * Nd + g0))[tn];
-        if (aux) {
+        if (pf && pnb >= 0) trace(pinfo, pnb, ff, pext);
+        if (pf) frame(pinfo, pfgi, ff, pg);
+        if (valid) {
+            J = a.ngeom[ND * ND * Nd + g0 + tid];
+            if (aux) {
 #pragma unroll
-            for (int v = 0; v < NV; ++v) xv[v] = (aux + (v * Nd + g0))[tn];
+                for (int v = 0; v < NV; ++v) xv[v] = aux[v * Nd + g0 + tid];
+            }
         }
     };
     curved_direction<ND, N, TP, 0>(a, sS, sM, sTab, sD, nel, tid, le, node, valid, q, u, p, m, [&]() { metric(1); }, acc);

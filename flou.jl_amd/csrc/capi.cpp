@@ -716,7 +716,14 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
                              : nd == 2 ? 256 * (n == 6 ? 6 : 12) : (n == 6 ? 256 : 0);
         if (h->v64 && h->vol == FLOU_HIP_SPLIT && h->eq == FLOU_HIP_EULER && !gen && nd >= 2 && n >= 4 && diag &&
             !oriented && h->gather && h->lift_end && d->nelements >= fill && sbp(d))
-            h->v64 = nd == 2 ? split_vjp_f64_2(n, h->tp) : split_vjp_f64_3(n, h->tp);
+            h->v64 = nd == 2 ? split_vjp_f64_2(n, h->tp, false) : split_vjp_f64_3(n, h->tp, false);
+        // and on curved elements: 3-D (600 k nodes, Chandrasekhar: 4 nodes per line 92 -> 65 us, 7 146 ->
+        // 87, 8 378 -> 131; Kennedy-Gruber at 6, where a line's wave is 56 % full, 82 -> 84), and 2-D with 4
+        // nodes or where lines fill the chip (8 nodes, 6241 elements: 50 -> 44 us, 324: 12.5 -> 17)
+        const bool cv = nd == 3 ? !(n == 6 && h->tp == FLOU_HIP_TP_KENNEDY_GRUBER) : n == 4 || d->nelements >= 4096;
+        if (h->v64 && h->vol == FLOU_HIP_SPLIT && h->eq == FLOU_HIP_EULER && !gen && n >= 4 && h->curved && h->gather &&
+            h->lift_end && cv && sbp(d))
+            h->v64 = nd == 2 ? split_vjp_f64_2(n, h->tp, true) : split_vjp_f64_3(n, h->tp, true);
     } else {
         h->v32 = nd == 1 ? vjp_f32_1d(n, h->eq, h->vol, h->tp, h->curved, gen)
                          : (nd == 2 ? vjp_f32_2d(n, h->eq, h->vol, h->tp, h->curved, gen)

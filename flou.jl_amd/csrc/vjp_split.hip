@@ -1,4 +1,4 @@
-// FP64 adjoint of the split-form Euler rhs on axis-aligned affine elements (GLL nodes,
+// FP64 adjoint of the split-form Euler rhs on axis-aligned affine and curved elements (GLL nodes,
 // Chandrasekhar, Kennedy-Gruber or StdAverage two-point flux, StdAverage or LxF(StdAverage)
 // surface flux), 2-D and 3-D, with the reverse RK stage epilogue: VjpArgs of common.hpp, the
 // products of k_vjp (vjp_plain.hip) up to rounding.
@@ -15,9 +15,12 @@
 //   * cotangents are those of the halved node inputs, pulled back to (ρ, m, E) once per node;
 //   * the face flux is differentiated with respect to the own trace only, by the line that
 //     ends there.
+// Curved elements (CURV): the pair's flux along the mean metric, which lies in LDS for all
+// directions, in physical components; normals per face node.
 // LDS: the node inputs and w = c·Y/J; the rows of the directions are added, one direction after
 // the other, over w.  Measured, Chandrasekhar, rhs_vjp: 2-D N=5, 0.59 M nodes: 55 -> 40 us;
-// 3-D N=5, 1.7 M nodes: 271 -> 184 us; 3-D N=7, 0.5 M nodes: 238 -> 72 us.
+// 3-D N=5, 1.7 M nodes: 271 -> 184 us; 3-D N=7, 0.5 M nodes: 238 -> 72 us;
+// curved 3-D N=6, 0.6 M nodes: 146 -> 87 us.
 // Compile with -DFLOUHIP_ND=2|3.
 #include "common.hpp"
 #include "adjoint.hpp"
@@ -32,8 +35,9 @@ using adj::rcp;
 // Elements per block: the lines of one direction fill whole waves (3-D N=6 of 7 nodes: 49 of
 // 64 lanes, N=5: 108 of 128); 2-D N=7 leaves 8 lanes for a third block per CU (Kennedy-Gruber, 4624
 // elements: 27.6 -> 18.7 us).
-template <int ND, int N>
+template <int ND, int N, bool CURV>
 constexpr int epb() {
+    if (CURV && ND == 3) return N == 4 ? 4 : (N == 5 ? 2 : 1);  // nine metric values per node beside them
     return ND == 2 ? (N == 8 ? 7 : 64 / N) : (N == 4 ? 4 : (N == 5 ? 5 : (N == 6 ? 3 : 1)));
 }
 
@@ -43,10 +47,10 @@ constexpr int epb() {
 template <int ND, int N>
 using Nodes = NodeLds<ND, N, N == 4 || N == 8>;
 
-template <int ND, int N, int TP>
+template <int ND, int N, int TP, bool CURV>
 struct LCfg {
     static constexpr int NPE = Cfg<ND, N>::NPE, NPF = Cfg<ND, N>::NPF, NF = 2 * ND, NV = ND + 2;
-    static constexpr int EPB = epb<ND, N>();
+    static constexpr int EPB = epb<ND, N, CURV>();
     static constexpr int NN = EPB * Nodes<ND, N>::ES;  // LDS nodes per block
     static constexpr int NL = EPB * NPF;                 // lines per block and direction
     static constexpr int WPD = (NL + 63) / 64;           // waves per direction
@@ -75,18 +79,50 @@ __device__ __forceinline__ void lm_factor(double u, double f, double a, double b
 // Reverse product of component n (the first velocity) of the two-point flux for the cotangent
 // G = (ρ, n, t.., E), scaled by s, added to the cotangents gi and gj of the nodes' inputs:
 // Chandrasekhar (ρ/2, u/2.., β), Kennedy-Gruber (ρ/2, u/2.., p/2, E/(2ρ)).
-template <int ND, int TP, bool SERIES>
-__device__ __forceinline__ void pair_vjp(const double* P, const double* Q, const double* G, double s, double ig1,
-                                         double* gi, double* gj) {
+// CURV: of the flux along n, the mean metric, instead.
+template <int ND, int TP, bool SERIES, bool CURV>
+__device__ __forceinline__ void pair_vjp(const double* P, const double* Q, const double* G, const double* n, double s,
+                                         double ig1, double* gi, double* gj) {
     constexpr int NV = ND + 2;
+    double gn = G[1];
+    if constexpr (CURV) {
+        gn = G[1] * n[0];
+#pragma unroll
+        for (int k = 1; k < ND; ++k) gn = fma(G[1 + k], n[k], gn);
+    }
+    if constexpr (TP == TP_STDAVG) {  // (u.., H, |u|²; only for CURV, see line_phase); s: with the mean's ½
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            const double* X = side ? Q : P;
+            double* g = side ? gj : gi;
+            double un = X[0] * n[0], U = G[NV - 1] * X[ND];
+#pragma unroll
+            for (int k = 0; k < ND; ++k) {
+                if (k) un = fma(X[k], n[k], un);
+                U = fma(G[1 + k], X[k], U);
+            }
+            const double g1 = 1 / ig1, pg = g1 * fma(G[NV - 1], un, gn), gU = G[0] + U;
+            g[0] = fma(s, fma(-U, un, 0.5 * pg * X[ND + 1]), g[0]);
+#pragma unroll
+            for (int k = 0; k < ND; ++k)
+                g[1 + k] = fma(s, fma(G[1 + k], un, fma(-pg, X[k], gU * n[k])), g[1 + k]);
+            g[NV - 1] = fma(s, fma(G[NV - 1], un, pg), g[NV - 1]);
+        }
+        return;
+    }
     double ub[ND];
 #pragma unroll
     for (int k = 0; k < ND; ++k) ub[k] = P[1 + k] + Q[1 + k];
-    const double un = ub[0];
+    double un = ub[0];
+    if constexpr (CURV) {
+        un = ub[0] * n[0];
+#pragma unroll
+        for (int k = 1; k < ND; ++k) un = fma(ub[k], n[k], un);
+    }
     double gu = G[1] * ub[0];
 #pragma unroll
     for (int k = 1; k < ND; ++k) gu = fma(G[1 + k], ub[k], gu);
-    const double gn = G[1], ge = G[NV - 1];
+    const double ge = G[NV - 1];
     if constexpr (TP == TP_KENNEDY_GRUBER) {
         // f = (m, m ū + p̄ n, m ē + p̄ ū_n), m = ρ̄ ū_n: every input enters as the sum
         const double rho = P[0] + Q[0], p = P[ND + 1] + Q[ND + 1], e = P[ND + 2] + Q[ND + 2];
@@ -96,7 +132,7 @@ __device__ __forceinline__ void pair_vjp(const double* P, const double* Q, const
         double t[NV + 1];
         t[0] = mb * un;
 #pragma unroll
-        for (int k = 0; k < ND; ++k) t[1 + k] = k == 0 ? fma(m, gn, unb) : m * G[1 + k];
+        for (int k = 0; k < ND; ++k) t[1 + k] = CURV ? fma(m, G[1 + k], unb * n[k]) : (k == 0 ? fma(m, gn, unb) : m * G[1 + k]);
         t[ND + 1] = fma(ge, un, gn);
         t[ND + 2] = ge * m;
 #pragma unroll
@@ -145,18 +181,19 @@ __device__ __forceinline__ void pair_vjp(const double* P, const double* Q, const
         gj[NV - 1] = fma(s, sbb - dbb, gj[NV - 1]);
 #pragma unroll
         for (int k = 0; k < ND; ++k) {
-            const double ubb = k == 0 ? fma(m, gn, mbr) : m * G[1 + k];
+            const double ubb = CURV ? fma(m, G[1 + k], mbr * n[k]) : (k == 0 ? fma(m, gn, mbr) : m * G[1 + k]);
             gi[1 + k] = fma(s, fma(dotb, Q[1 + k], ubb), gi[1 + k]);
             gj[1 + k] = fma(s, fma(dotb, P[1 + k], ubb), gj[1 + k]);
         }
     }
 }
 
-// One side of the face flux: its state in the face frame with what the products need.
-template <int ND>
+// One side of the face flux along n (CURV; else along the first axis of the state's frame): its
+// state with what the products need.
+template <int ND, bool CURV>
 struct Side {
-    double ir, u[ND], uu, p, c, a;
-    __device__ __forceinline__ Side(const double* R, double gamma) {
+    double ir, u[ND], uu, un, p, c, a;
+    __device__ __forceinline__ Side(const double* R, const double* n, double gamma) {
         ir = rcp(R[0]);
         uu = 0;
 #pragma unroll
@@ -166,33 +203,61 @@ struct Side {
         }
         p = (gamma - 1) * fma(-0.5 * R[0], uu, R[ND + 1]);
         c = sqrt(gamma * p * ir);
-        a = fabs(u[0]) + c;
+        un = u[0];
+        if constexpr (CURV) {
+            un = u[0] * n[0];
+#pragma unroll
+            for (int k = 1; k < ND; ++k) un = fma(u[k], n[k], un);
+        }
+        a = fabs(un) + c;
     }
     // Adds to b the product of f(R)·n for the cotangent G and lb times the gradient of a.
-    __device__ __forceinline__ void add(const double* R, const double* G, double gamma, double lb, double* b) const {
+    __device__ __forceinline__ void add(const double* R, const double* G, const double* n, double gamma, double lb,
+                                        double* b) const {
         constexpr int NV = ND + 2;
         const double g1 = gamma - 1;
+        double gn = G[1];
+        if constexpr (CURV) {
+            gn = G[1] * n[0];
+#pragma unroll
+            for (int k = 1; k < ND; ++k) gn = fma(G[1 + k], n[k], gn);
+        }
         double unb = G[NV - 1] * (R[NV - 1] + p);
 #pragma unroll
         for (int k = 0; k < ND; ++k) unb = fma(G[1 + k], R[1 + k], unb);
-        unb += lb * (u[0] > 0 ? 1.0 : (u[0] < 0 ? -1.0 : 0.0));
+        unb += lb * (un > 0 ? 1.0 : (un < 0 ? -1.0 : 0.0));
         const double cb = lb == 0 ? 0.0 : 0.5 * lb * rcp(c);  // of c²
-        const double pg = g1 * (fma(G[NV - 1], u[0], G[1]) + cb * gamma * ir);
+        const double pg = g1 * (fma(G[NV - 1], un, gn) + cb * gamma * ir);
         const double uir = unb * ir;
-        b[0] += -uir * u[0] + 0.5 * pg * uu - cb * c * c * ir;
+        b[0] += -uir * un + 0.5 * pg * uu - cb * c * c * ir;
 #pragma unroll
-        for (int k = 0; k < ND; ++k) b[1 + k] += fma(G[1 + k], u[0], fma(-pg, u[k], k == 0 ? G[0] + uir : 0.0));
-        b[NV - 1] += fma(G[NV - 1], u[0], pg);
+        for (int k = 0; k < ND; ++k)
+            b[1 + k] += fma(G[1 + k], un, fma(-pg, u[k], CURV ? (G[0] + uir) * n[k] : (k == 0 ? G[0] + uir : 0.0)));
+        b[NV - 1] += fma(G[NV - 1], un, pg);
     }
 };
 
+// The momentum m with its normal part reversed.
+template <int ND, bool CURV>
+__device__ __forceinline__ void mirror(double* m, const double* n) {
+    if constexpr (CURV) {
+        double mn = m[0] * n[0];
+#pragma unroll
+        for (int k = 1; k < ND; ++k) mn = fma(m[k], n[k], mn);
+#pragma unroll
+        for (int k = 0; k < ND; ++k) m[k] = fma(-2 * mn, n[k], m[k]);
+    } else {
+        m[0] = -m[0];
+    }
+}
+
 // A wave's lines of direction DIR.  Component k of a vector in the line frame is physical
-// component (DIR + k) % ND.
-template <int ND, int N, int TP, int DIR>
-__device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const double* sP, double* sW, double* sT,
-                                           const double* sS, const double* siw, int e0, int nel, int l,
-                                           double (&acc)[N][LCfg<ND, N, TP>::NA]) {
-    using C = LCfg<ND, N, TP>;
+// component (DIR + k) % ND; on curved elements (sM: half the metric rows) it is k.
+template <int ND, int N, int TP, bool CURV, int DIR>
+__device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const double* sP, const double* sM, double* sW,
+                                           double* sT, const double* sS, const double* siw, int e0, int nel, int l,
+                                           double (&acc)[N][LCfg<ND, N, TP, CURV>::NA]) {
+    using C = LCfg<ND, N, TP, CURV>;
     constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, NN = C::NN, NA = C::NA;
     using M = Nodes<ND, N>;
     constexpr int ST = M::template step<DIR>();
@@ -201,12 +266,11 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
     const bool task = l < C::NL && l / NPF < nel;
     const int le = task ? l / NPF : 0, f = l % NPF;
     const int base = le * M::ES + M::template line<DIR>(f);
-    const double* eg = a.egeom + (int64_t)(e0 + le) * a.egeom_stride;
-    const double ja = eg[DIR * (ND + 1)];
+    const double ja = CURV ? 1.0 : a.egeom[(int64_t)(e0 + le) * a.egeom_stride + DIR * (ND + 1)];
     const double gamma = a.gamma, ig1 = 1 / (gamma - 1);
     int vo[ND];  // physical variable of line-frame momentum k
 #pragma unroll
-    for (int k = 0; k < ND; ++k) vo[k] = 1 + (DIR + k) % ND;
+    for (int k = 0; k < ND; ++k) vo[k] = CURV ? 1 + k : 1 + (DIR + k) % ND;
 
     // ---- faces at the two line ends: cotangent of the own trace ------------------------
     if (task) {
@@ -214,9 +278,13 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
         for (int sd = 0; sd < 2; ++sd) {
             const int slot = (e0 + le) * NF + 2 * DIR + sd;
             const int info = a.finfo[slot], nb = a.nb[slot];
-            const double* g = a.fgeom + (int64_t)a.fgi[slot] * (3 * ND + 1);
+            const double* g = a.fgeom + ((int64_t)a.fgi[slot] * (CURV ? NPF : 1) +
+                                         (CURV ? face_master_node<ND, N>(f, info) : 0)) * (3 * ND + 1);
             const bool slave = finfo_side(info);
             const double so = slave ? -g[DIR] : g[DIR];   // own outward normal along the axis
+            double n[ND];                                 // CURV: the own outward normal
+#pragma unroll
+            for (int k = 0; k < ND; ++k) n[k] = slave ? -g[k] : g[k];
             const int64_t on = (int64_t)(e0 + le) * NPE + line_node<ND, N>(DIR, f, 0) + (sd ? (N - 1) * GST : 0);
             double o[NV], x[NV], G[NV], ob[NV], xb[NV];
             o[0] = a.Q[on];
@@ -234,9 +302,12 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
             int type = -1;
             if (nb >= 0) {
                 const int kp = finfo_nbpos(info);
-                const int64_t nn = (int64_t)nb * NPE + line_node<ND, N>(DIR, f, (kp & 1) ? N - 1 : 0);
+                const int64_t nn = (int64_t)nb * NPE +
+                                   line_node<ND, N>(CURV ? kp >> 1 : DIR, CURV ? face_nb_node<ND, N>(f, info) : f,
+                                                    (kp & 1) ? N - 1 : 0);
                 const double cn = h * ((kp & 1) ? a.ops[ops_gp(N) + N - 1] : a.ops[ops_gm(N)]) *
-                                  (A.c / a.egeom[(int64_t)nb * a.egeom_stride + ND * ND]);
+                                  (A.c / (CURV ? a.ngeom[ND * ND * a.ndofs + nn]
+                                               : a.egeom[(int64_t)nb * a.egeom_stride + ND * ND]));
                 x[0] = a.Q[nn];
                 x[NV - 1] = a.Q[(NV - 1) * a.ndofs + nn];
                 G[0] = fma(cn, A.Y[nn], G[0]);
@@ -256,13 +327,14 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
                 x[NV - 1] = given ? src[NV - 1] : o[NV - 1];
 #pragma unroll
                 for (int k = 0; k < ND; ++k) x[1 + k] = given ? src[vo[k]] : o[1 + k];
-                if (type == BC_SLIP) x[1] = -x[1];
+                if (type == BC_SLIP) mirror<ND, CURV>(x + 1, n);
             }
-            // frame of the own outward normal
-            o[1] *= so;
-            x[1] *= so;
-            G[1] *= so;
-            const Side<ND> S(o, gamma), X(x, gamma);
+            if constexpr (!CURV) {  // frame of the own outward normal
+                o[1] *= so;
+                x[1] *= so;
+                G[1] *= so;
+            }
+            const Side<ND, CURV> S(o, n, gamma), X(x, n, gamma);
             double lo = 0, lx = 0, dl = 0;
 #pragma unroll
             for (int v = 0; v < NV; ++v) ob[v] = xb[v] = 0;
@@ -280,14 +352,14 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
                 lo = mine ? dl : 0;
                 lx = mine ? 0 : dl;
             }
-            S.add(o, G, gamma, lo, ob);
+            S.add(o, G, n, gamma, lo, ob);
             if (type == BC_OUTFLOW || type == BC_SLIP) {  // the exterior state follows the own trace
-                X.add(x, G, gamma, lx, xb);
-                if (type == BC_SLIP) xb[1] = -xb[1];
+                X.add(x, G, n, gamma, lx, xb);
+                if (type == BC_SLIP) mirror<ND, CURV>(xb + 1, n);
 #pragma unroll
                 for (int v = 0; v < NV; ++v) ob[v] += xb[v];
             }
-            ob[1] *= so;
+            if constexpr (!CURV) ob[1] *= so;
             double* t = sT + ((le * NF + 2 * DIR + sd) * NV) * NPF + f;
             t[0] = ob[0];
             t[(NV - 1) * NPF] = ob[NV - 1];
@@ -297,7 +369,7 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
     }
 
     // ---- the line's pairs ----------------------------------------------------------------
-    auto load = [&](int p, double* P, double* W) {
+    auto load = [&](int base, int p, double* P, double* W) {
         const double* s = sP + base + p * ST;
         const double* w = sW + base + p * ST;
         if constexpr (TP == TP_STDAVG) {  // u.., H, |u|²
@@ -317,17 +389,22 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
         for (int k = 0; k < ND; ++k) W[1 + k] = w[vo[k] * NN];
         W[NV - 1] = w[(NV - 1) * NN];
     };
+    auto metric = [&](int base, int p, double* n) {
+        const double* s = sM + base + p * ST;
+#pragma unroll
+        for (int k = 0; k < ND; ++k) n[k] = s[(ND * DIR + k) * NN];
+    };
 #pragma unroll
     for (int p = 0; p < N; ++p)
 #pragma unroll
         for (int c = 0; c < NA; ++c) acc[p][c] = 0;
-    if constexpr (TP == TP_STDAVG) {
+    if constexpr (TP == TP_STDAVG && !CURV) {
         // the flux is a sum of node terms: each node takes the reverse product of ½ f(Q)·n̄ for
         // Σ_j S_ij (w_j/ω_j - w_i/ω_i)
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             double P[NA], wi[NV];
-            load(i, P, wi);
+            load(base, i, P, wi);
 #pragma unroll
             for (int v = 0; v < NV; ++v) wi[v] *= siw[i];
 #pragma unroll
@@ -347,7 +424,7 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             double P[NA], w[NV], G[NV];
-            load(i, P, w);
+            load(base, i, P, w);
 #pragma unroll
             for (int v = 0; v < NV; ++v) G[v] = h * acc[i][v];
             double U = G[NV - 1] * P[ND];
@@ -360,21 +437,33 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
             acc[i][NV - 1] = fma(G[NV - 1], un, pg);
         }
     } else {
-        auto pairs = [&](auto series) {
+        auto pairs = [&, base0 = base](auto series) {
+            // CURV: the address is opaque from here, so that the two forms of the pairs share no loads
+            // (their values stayed live over the whole line: 256 registers at 3-D N=6, a wave per SIMD)
+            int base = base0;
+            if constexpr (CURV && TP == TP_CHANDRASEKHAR) asm volatile("" : "+v"(base));
 #pragma unroll
             for (int i = 0; i < N; ++i) {
-                double P[NA], wi[NV];
-                load(i, P, wi);
+                double P[NA], wi[NV], ni[ND];
+                load(base, i, P, wi);
+                if constexpr (CURV) metric(base, i, ni);
 #pragma unroll
                 for (int v = 0; v < NV; ++v) wi[v] *= siw[i];
 #pragma unroll
                 for (int j = i + 1; j < N; ++j) {
-                    double Q[NA], G[NV];
-                    load(j, Q, G);
+                    double Q[NA], G[NV], n[ND];
+                    load(base, j, Q, G);
+                    if constexpr (CURV) {
+                        metric(base, j, n);
+#pragma unroll
+                        for (int k = 0; k < ND; ++k) n[k] += ni[k];
+                    }
                     const double iw = siw[j];
 #pragma unroll
                     for (int v = 0; v < NV; ++v) G[v] = fma(G[v], iw, -wi[v]);
-                    pair_vjp<ND, TP, decltype(series)::value>(P, Q, G, sS[i * N + j] * ja, ig1, acc[i], acc[j]);
+                    pair_vjp<ND, TP, decltype(series)::value, CURV>(P, Q, G, n,
+                                                                    sS[i * N + j] * (TP == TP_STDAVG ? 0.5 : ja), ig1,
+                                                                    acc[i], acc[j]);
                     // one pair's loads and arithmetic at a time: the registers hold the rows,
                     // node i and one pair
                     __builtin_amdgcn_sched_barrier(0);
@@ -407,9 +496,9 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
 }
 
 // Adds (direction 0: writes) a line's rows to the nodes' sums, in physical component order.
-template <int ND, int N, int TP, int DIR>
-__device__ __forceinline__ void add_rows(double* sR, int nel, int l, const double (&acc)[N][LCfg<ND, N, TP>::NA]) {
-    using C = LCfg<ND, N, TP>;
+template <int ND, int N, int TP, bool CURV, int DIR>
+__device__ __forceinline__ void add_rows(double* sR, int nel, int l, const double (&acc)[N][LCfg<ND, N, TP, CURV>::NA]) {
+    using C = LCfg<ND, N, TP, CURV>;
     using M = Nodes<ND, N>;
     constexpr int ST = M::template step<DIR>();
     if (l >= C::NL || l / C::NPF >= nel) return;
@@ -418,19 +507,20 @@ __device__ __forceinline__ void add_rows(double* sR, int nel, int l, const doubl
     for (int p = 0; p < N; ++p)
 #pragma unroll
         for (int c = 0; c < C::NA; ++c) {
-            const int pc = c >= 1 && c <= ND ? 1 + (DIR + c - 1) % ND : c;
+            const int pc = !CURV && c >= 1 && c <= ND ? 1 + (DIR + c - 1) % ND : c;
             double* x = r + pc * C::NN + p * ST;
             *x = DIR == 0 ? acc[p][c] : *x + acc[p][c];
         }
 }
 
-template <int ND, int N, int TP>
-__global__ void __launch_bounds__((LCfg<ND, N, TP>::TPB)) k_svjp(const VjpArgs<double> A) {
-    using C = LCfg<ND, N, TP>;
+template <int ND, int N, int TP, bool CURV>
+__global__ void __launch_bounds__((LCfg<ND, N, TP, CURV>::TPB)) k_svjp(const VjpArgs<double> A) {
+    using C = LCfg<ND, N, TP, CURV>;
     constexpr int NV = C::NV, NPE = C::NPE, NPF = C::NPF, NF = C::NF, EPB = C::EPB, TPB = C::TPB, NN = C::NN, NA = C::NA;
     __shared__ double sP[NA * NN];                       // node inputs
     __shared__ double sW[(NA > NV ? NA : NV) * NN];      // w = c·Y/J, then the sums of the rows
     __shared__ double sT[EPB * NF * NV * NPF];           // cotangents of the own traces
+    __shared__ double sM[CURV ? ND * ND * NN : 1];       // CURV: half the metric, component-major
     __shared__ double sS[N * N], siw[N];
     const RhsArgs<double>& a = A.r;
     const int tid = threadIdx.x;
@@ -455,7 +545,12 @@ __global__ void __launch_bounds__((LCfg<ND, N, TP>::TPB)) k_svjp(const VjpArgs<d
             q[v] = a.Q[v * Nd + g0 + j];
             y[v] = A.Y[v * Nd + g0 + j];
         }
-        const double cj = A.c / a.egeom[(int64_t)(e0 + j / NPE) * a.egeom_stride + ND * ND];
+        const double cj = A.c / (CURV ? a.ngeom[ND * ND * Nd + g0 + j]
+                                      : a.egeom[(int64_t)(e0 + j / NPE) * a.egeom_stride + ND * ND]);
+        if constexpr (CURV) {
+#pragma unroll
+            for (int c = 0; c < ND * ND; ++c) sM[c * NN + jj] = 0.5 * a.ngeom[c * Nd + g0 + j];
+        }
         const double ir = rcp(q[0]);
         double u[ND], uu = 0;
 #pragma unroll
@@ -489,16 +584,16 @@ __global__ void __launch_bounds__((LCfg<ND, N, TP>::TPB)) k_svjp(const VjpArgs<d
     const int dir = wave / C::WPD;
     const int l = dir < ND ? (wave - dir * C::WPD) * 64 + (tid & 63) : C::NL;
     double acc[N][NA];
-    if (dir == 0) line_phase<ND, N, TP, 0>(A, sP, sW, sT, sS, siw, e0, nel, l, acc);
-    else if (ND == 2 || dir == 1) line_phase<ND, N, TP, 1>(A, sP, sW, sT, sS, siw, e0, nel, l, acc);
-    else if (dir == ND - 1) line_phase<ND, N, TP, ND - 1>(A, sP, sW, sT, sS, siw, e0, nel, l, acc);
+    if (dir == 0) line_phase<ND, N, TP, CURV, 0>(A, sP, sM, sW, sT, sS, siw, e0, nel, l, acc);
+    else if (ND == 2 || dir == 1) line_phase<ND, N, TP, CURV, 1>(A, sP, sM, sW, sT, sS, siw, e0, nel, l, acc);
+    else if (dir == ND - 1) line_phase<ND, N, TP, CURV, ND - 1>(A, sP, sM, sW, sT, sS, siw, e0, nel, l, acc);
     __syncthreads();  // w has been read
-    if (dir == 0) add_rows<ND, N, TP, 0>(sW, nel, l, acc);
+    if (dir == 0) add_rows<ND, N, TP, CURV, 0>(sW, nel, l, acc);
     __syncthreads();
-    if (dir == 1) add_rows<ND, N, TP, 1>(sW, nel, l, acc);
+    if (dir == 1) add_rows<ND, N, TP, CURV, 1>(sW, nel, l, acc);
     __syncthreads();
     if constexpr (ND == 3) {
-        if (dir == 2) add_rows<ND, N, TP, 2>(sW, nel, l, acc);
+        if (dir == 2) add_rows<ND, N, TP, CURV, 2>(sW, nel, l, acc);
         __syncthreads();
     }
 
@@ -568,19 +663,19 @@ __global__ void __launch_bounds__((LCfg<ND, N, TP>::TPB)) k_svjp(const VjpArgs<d
     }
 }
 
-template <int ND, int N, int TP>
+template <int ND, int N, int TP, bool CURV>
 static hipError_t launch(const VjpArgs<double>& a, hipStream_t s) {
-    using C = LCfg<ND, N, TP>;
-    hipLaunchKernelGGL((k_svjp<ND, N, TP>), dim3((a.r.ne + C::EPB - 1) / C::EPB), dim3(C::TPB), 0, s, a);
+    using C = LCfg<ND, N, TP, CURV>;
+    hipLaunchKernelGGL((k_svjp<ND, N, TP, CURV>), dim3((a.r.ne + C::EPB - 1) / C::EPB), dim3(C::TPB), 0, s, a);
     return hipGetLastError();
 }
 
-template <int ND, int N>
+template <int ND, int N, bool CURV>
 static VjpLauncherF64 pick_tp(int tp) {
     switch (tp) {
-        case TP_STDAVG: return &launch<ND, N, TP_STDAVG>;
-        case TP_CHANDRASEKHAR: return &launch<ND, N, TP_CHANDRASEKHAR>;
-        case TP_KENNEDY_GRUBER: return &launch<ND, N, TP_KENNEDY_GRUBER>;
+        case TP_STDAVG: return &launch<ND, N, TP_STDAVG, CURV>;
+        case TP_CHANDRASEKHAR: return &launch<ND, N, TP_CHANDRASEKHAR, CURV>;
+        case TP_KENNEDY_GRUBER: return &launch<ND, N, TP_KENNEDY_GRUBER, CURV>;
         default: return nullptr;
     }
 }
@@ -590,13 +685,13 @@ static VjpLauncherF64 pick_tp(int tp) {
 #define FLOUHIP_CAT_(a, b) a##b
 #define FLOUHIP_CAT(a, b) FLOUHIP_CAT_(a, b)
 
-VjpLauncherF64 FLOUHIP_CAT(split_vjp_f64_, FLOUHIP_ND)(int n, int tp) {
+VjpLauncherF64 FLOUHIP_CAT(split_vjp_f64_, FLOUHIP_ND)(int n, int tp, bool curved) {
     switch (n) {
-        case 4: return svjp::pick_tp<FLOUHIP_ND, 4>(tp);
-        case 5: return svjp::pick_tp<FLOUHIP_ND, 5>(tp);
-        case 6: return svjp::pick_tp<FLOUHIP_ND, 6>(tp);
-        case 7: return svjp::pick_tp<FLOUHIP_ND, 7>(tp);
-        case 8: return svjp::pick_tp<FLOUHIP_ND, 8>(tp);
+        case 4: return curved ? svjp::pick_tp<FLOUHIP_ND, 4, true>(tp) : svjp::pick_tp<FLOUHIP_ND, 4, false>(tp);
+        case 5: return curved ? svjp::pick_tp<FLOUHIP_ND, 5, true>(tp) : svjp::pick_tp<FLOUHIP_ND, 5, false>(tp);
+        case 6: return curved ? svjp::pick_tp<FLOUHIP_ND, 6, true>(tp) : svjp::pick_tp<FLOUHIP_ND, 6, false>(tp);
+        case 7: return curved ? svjp::pick_tp<FLOUHIP_ND, 7, true>(tp) : svjp::pick_tp<FLOUHIP_ND, 7, false>(tp);
+        case 8: return curved ? svjp::pick_tp<FLOUHIP_ND, 8, true>(tp) : svjp::pick_tp<FLOUHIP_ND, 8, false>(tp);
         default: return nullptr;
     }
 }

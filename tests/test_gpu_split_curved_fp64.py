@@ -21,10 +21,11 @@ pytest.importorskip("torch")
 NEL = {2: (5, 3), 3: (3, 2, 2)}
 
 
-def build(nd, n, tp, lxf, walls):
+def build(nd, n, tp, lxf, walls, nel=None):
+    nel = nel or NEL[nd]
     b = F.LagrangeBasis("GLL", n)
     std = [None, None, F.StdQuad, F.StdHex][nd](b, F.DGSEMrec(b), nd + 2)
-    mesh = F.CartesianMesh(nd, (0.0,) * nd, (1.0,) * nd, NEL[nd])
+    mesh = F.CartesianMesh(nd, (0.0,) * nd, (1.0,) * nd, nel)
     mesh.apply_periodicBCs(*[(str(2 * k + 1), str(2 * k + 2)) for k in range(1 if walls else 0, nd)])
     mesh.apply_mapping(warp)
     bcs = {"1": F.EulerSlipBC(), "2": F.EulerOutflowBC()} if walls else {}
@@ -32,7 +33,7 @@ def build(nd, n, tp, lxf, walls):
     surf = F.LxF(F.StdAverage(), 0.8) if lxf else F.StdAverage()
     disc = F.MultielementDisc(mesh, std, eq, F.SplitDivOperator(TP[tp][0](), surf), bcs)
     J, met, ev, fr, fj = M.curved_geometry(mesh, std)
-    orc = O.OracleDisc(nd, n, list(NEL[nd]), [0.0] * nd, [1.0] * nd, [0 if walls and k == 0 else 1 for k in range(nd)],
+    orc = O.OracleDisc(nd, n, list(nel), [0.0] * nd, [1.0] * nd, [0 if walls and k == 0 else 1 for k in range(nd)],
                        O.build_ops(n, "GLL"), O.EQ_EULER, [GAMMA], O.VOL_SPLIT, TP[tp][1], O.AVG_STD,
                        O.DISS_LXF if lxf else O.DISS_NONE, 0.8 if lxf else 1.0)
     orc.set_curved(met, J, fr.reshape(-1), fj, ev)

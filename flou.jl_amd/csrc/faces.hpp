@@ -85,40 +85,4 @@ __device__ __forceinline__ void axis_flux(T* own, T* ext, T sn, T jac, bool slav
     for (int v = 0; v < NV; ++v) Fn[v] = Fn[v] * js;
 }
 
-// The same in FP32 with fused multiply-adds: each side's flux by itself, their sum (which
-// commutes) and the jump's sign as above, so that the two sides' results stay opposite bit for bit.
-template <int ND>
-__device__ __forceinline__ void axis_flux_f32(float* own, float* ext, float sn, float jac, bool slave, int sdiss, float gamma,
-                                          float intensity, int* err, float* Fn) {
-    constexpr int NV = ND + 2;
-    own[1] = sn * own[1];
-    ext[1] = sn * ext[1];
-    const float sg = slave ? -1.0f : 1.0f, js = sg * jac, hj = 0.5f * js;
-    float u[2], p[2];
-    Recip<float> r[2] = {Recip<float>(own[0]), Recip<float>(ext[0])};
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const float* Q = s ? ext : own;
-        u[s] = r[s].fin(Q[1]);
-        float m2 = Q[1] * Q[1];
-#pragma unroll
-        for (int c = 1; c < ND; ++c) m2 = __builtin_fmaf(Q[1 + c], Q[1 + c], m2);
-        p[s] = (gamma - 1.0f) * __builtin_fmaf(-0.5f, r[s].fin(m2), Q[NV - 1]);
-    }
-    Fn[0] = hj * (own[1] + ext[1]);
-    Fn[1] = hj * (__builtin_fmaf(own[1], u[0], p[0]) + __builtin_fmaf(ext[1], u[1], p[1]));
-#pragma unroll
-    for (int c = 1; c < ND; ++c) Fn[1 + c] = hj * (own[1 + c] * u[0] + ext[1 + c] * u[1]);
-    Fn[NV - 1] = hj * ((own[NV - 1] + p[0]) * u[0] + (ext[NV - 1] + p[1]) * u[1]);
-    if (sdiss == DISS_LXF) {
-        const float lo = fabsf(u[0]) + plain::dsqrt(r[0].fin(gamma * p[0]), err);
-        const float lx = fabsf(u[1]) + plain::dsqrt(r[1].fin(gamma * p[1]), err);
-        // the larger speed, the master's where they do not compare; the jump and js carry the sign
-        const float lam = (slave ? ((lx < lo) ? lo : lx) : ((lo < lx) ? lx : lo)) * (intensity * (0.5f * jac));
-#pragma unroll
-        for (int v = 0; v < NV; ++v) Fn[v] = __builtin_fmaf(lam, own[v] - ext[v], Fn[v]);
-    }
-    Fn[1] = sn * Fn[1];
-}
-
 }  // namespace flouhip

@@ -9,12 +9,13 @@
 //   * the fluxes lie in LDS in vectors of 16 bytes, so that a line's entry is one or two reads;
 //   * all loads come first, the face tables, then the node's state and the neighbours' traces:
 //     two dependent global loads from start to end;
-//   * faces as in faces.hpp; the lift touches the end nodes only (∂g is exactly zero elsewhere);
-//   * FP32 sums with fused multiply-adds (one rounding less per term).
-// Measured against k_plain, rhs, 0.9 M nodes, Euler, N nodes per line: 3-D N=5 FP32 37.8 -> 20 us,
-// FP64 72 -> 36; 3-D N=8 FP32 46 -> 17, FP64 130 -> 33; 2-D N=6 FP32 20.5 -> 12.4, FP64 37 -> 20.  An
-// SSPRK33 step of 7182 elements, 3-D N=5, FP32: 116 -> 60 us; ten of advection on 256 elements, 2-D
-// N=5, FP64: 163 -> 148 us.  Blocks of 128 threads: 2-D N=6 FP32 15.8 us, FP64 26.
+//   * faces as in faces.hpp; the lift touches the end nodes only (∂g is exactly zero elsewhere).
+// Measured against k_plain, rhs, 0.9 M nodes, Euler, N nodes per line: 3-D N=5 FP32 37.8 -> 22 us,
+// FP64 72 -> 35; 3-D N=8 FP32 46 -> 18.6, FP64 130 -> 33; 2-D N=6 FP32 20.5 -> 13.4, FP64 37 -> 20.  An
+// SSPRK33 step of 7182 elements, 3-D N=5, FP32: 116 -> 64 us; ten of advection on 256 elements, 2-D
+// N=5, FP64: 163 -> 148 us.  Blocks of 128 threads: 2-D N=6 FP32 15.8 us, FP64 26.  (FP32 with fused
+// operations: 57 us, but the 2N schemes' register, a small difference of large sums, then differs
+// from the plain kernel's in its third digit.)
 // Compile with -DFLOUHIP_PREC_F64 or -DFLOUHIP_PREC_F32 and -DFLOUHIP_ND=1|2|3.
 #include "common.hpp"
 #include "faces.hpp"
@@ -62,11 +63,6 @@ struct Table {
         for (int v = NVV * W; v < NV; ++v) x[v] = s[v * NN + j];
     }
 };
-
-__device__ __forceinline__ double madd(double a, double b, double c) { return a * b + c; }
-__device__ __forceinline__ float madd(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-__device__ __forceinline__ double msub(double a, double b, double c) { return a - b * c; }
-__device__ __forceinline__ float msub(float a, float b, float c) { return __builtin_fmaf(-b, c, a); }
 
 template <typename T, int ND, int N, int EQ>
 __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> a) {
@@ -144,17 +140,7 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
     } else {
         T P[NV];
         const Recip<T> ir(q[0]);
-        if constexpr (sizeof(T) == 4) {
-            T m2 = T(0);
-#pragma unroll
-            for (int c = 0; c < ND; ++c) {
-                P[1 + c] = ir.fin(q[1 + c]);
-                m2 = __builtin_fmaf(q[1 + c], q[1 + c], m2);
-            }
-            P[ND + 1] = (a.gamma - T(1)) * __builtin_fmaf(T(-0.5), ir.fin(m2), q[ND + 1]);
-        } else {
-            plain::cons2prim<T, ND>(q, a.gamma, P, ir);
-        }
+        plain::cons2prim<T, ND>(q, a.gamma, P, ir);
         const T p = P[ND + 1];
 #pragma unroll
         for (int d = 0; d < ND; ++d) {
@@ -162,7 +148,7 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
             F[d][0] = q[1 + d] * ja[d];
 #pragma unroll
             for (int c = 0; c < ND; ++c)
-                F[d][1 + c] = (c == d ? madd(q[1 + d], P[1 + c], p) : q[1 + d] * P[1 + c]) * ja[d];
+                F[d][1 + c] = (c == d ? q[1 + d] * P[1 + c] + p : q[1 + d] * P[1 + c]) * ja[d];
             F[d][NV - 1] = ((q[NV - 1] + p) * u) * ja[d];
         }
     }
@@ -195,7 +181,7 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
                 T x[NV];
                 Tab::get(sF[d], base + k * S[d], x);
 #pragma unroll
-                for (int v = 0; v < NV; ++v) acc[v] = msub(acc[v], Dik, x[v]);
+                for (int v = 0; v < NV; ++v) acc[v] = acc[v] - Dik * x[v];
             }
         }
     }
@@ -220,10 +206,7 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
             o[0] = Fn * (sg * fj[r]);
         } else {
             T Fn[NV];
-            if constexpr (sizeof(T) == 4)
-                axis_flux_f32<ND>(own[r], ext[r], sn[r], fj[r], slave, a.sdiss, a.gamma, a.intensity, a.errflag, Fn);
-            else
-                axis_flux<T, ND>(own[r], ext[r], sn[r], fj[r], slave, a.sdiss, a.gamma, a.intensity, a.errflag, Fn);
+            axis_flux<T, ND>(own[r], ext[r], sn[r], fj[r], slave, a.sdiss, a.gamma, a.intensity, a.errflag, Fn);
             o[0] = Fn[0];
 #pragma unroll
             for (int c = 0; c < ND; ++c) o[face_mom<ND>(dir, c) * NPF] = Fn[1 + c];
@@ -243,13 +226,13 @@ __global__ void __launch_bounds__((TCfg<ND, N>::TPB)) k_strong(const RhsArgs<T> 
             const T* s = sFn + (le * NF + 2 * d + (ii ? 1 : 0)) * (NV * NPF) + f;
             const T c = ii ? gpn : gm0;
 #pragma unroll
-            for (int v = 0; v < NV; ++v) acc[v] = msub(acc[v], c, s[v * NPF]);
+            for (int v = 0; v < NV; ++v) acc[v] = acc[v] - c * s[v * NPF];
         }
     }
     const Recip<T> iJ(jac);
     const StageOut<T> so(a);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) so.put(v * Nd + g0 + tid, sizeof(T) == 4 ? iJ.fin(acc[v]) : iJ.div(acc[v]), q[v], xv[v]);
+    for (int v = 0; v < NV; ++v) so.put(v * Nd + g0 + tid, iJ.div(acc[v]), q[v], xv[v]);
 }
 
 template <typename T, int ND, int N, int EQ>

@@ -438,10 +438,11 @@ __device__ __forceinline__ void line_phase(const VjpArgs<double>& A, const doubl
         }
     } else {
         auto pairs = [&, base0 = base](auto series) {
-            // CURV: the address is opaque from here, so that the two forms of the pairs share no loads
-            // (their values stayed live over the whole line: 256 registers at 3-D N=6, a wave per SIMD)
+            // The address is opaque from here, so that the two forms of the pairs share no loads (their
+            // values stayed live over the whole line: 256 registers and a wave per SIMD at 3-D N=7, 4096
+            // elements 257 -> 168 us; curved 3-D N=6 likewise)
             int base = base0;
-            if constexpr (CURV && TP == TP_CHANDRASEKHAR) asm volatile("" : "+v"(base));
+            if constexpr (TP == TP_CHANDRASEKHAR) asm volatile("" : "+v"(base));
 #pragma unroll
             for (int i = 0; i < N; ++i) {
                 double P[NA], wi[NV], ni[ND];
@@ -530,6 +531,30 @@ __global__ void __launch_bounds__((LCfg<ND, N, TP, CURV>::TPB)) k_svjp(const Vjp
     const int nnb = nel * NPE;
     const double gamma = a.gamma, gm1 = a.gamma - 1;
 
+    // The loads of all the thread's nodes come first (BATCH; spare threads load the block's first
+    // node): 2-D N=7, 40,000 elements, Chandrasekhar 141 -> 134 us; 3-D N=5, 4096 elements 103.5 -> 105.8,
+    // where they come node by node.
+    constexpr int NPT = (EPB * NPE + TPB - 1) / TPB;
+    constexpr bool BATCH = ND == 2 || N >= 7;
+    constexpr int NB = BATCH ? NPT : 1;
+    double q_[NB][NV], y_[NB][NV], j_[NB], m_[CURV ? NB : 1][CURV ? ND * ND : 1];
+    auto state = [&](int t, int b) {
+        const int j = tid + t * TPB < nnb ? tid + t * TPB : 0;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            q_[b][v] = (a.Q + (v * Nd + g0))[j];
+            y_[b][v] = (A.Y + (v * Nd + g0))[j];
+        }
+        j_[b] = CURV ? (a.ngeom + (ND * ND * Nd + g0))[j] : a.egeom[(int64_t)(e0 + j / NPE) * a.egeom_stride + ND * ND];
+        if constexpr (CURV) {
+#pragma unroll
+            for (int c = 0; c < ND * ND; ++c) m_[b][c] = (a.ngeom + (c * Nd + g0))[j];
+        }
+    };
+    if constexpr (BATCH) {
+#pragma unroll
+        for (int t = 0; t < NPT; ++t) state(t, t);
+    }
     for (int i = tid; i < N * N; i += TPB) {
         const int r = i / N, c = i - r * N;
         const double* w = a.ops + ops_w(N);
@@ -537,19 +562,19 @@ __global__ void __launch_bounds__((LCfg<ND, N, TP, CURV>::TPB)) k_svjp(const Vjp
         sS[i] = 0.5 * (w[r] * D[i] - w[c] * D[c * N + r]);
     }
     for (int i = tid; i < N; i += TPB) siw[i] = 1 / a.ops[ops_w(N) + i];
-    for (int j = tid; j < nnb; j += TPB) {
-        const int jj = Nodes<ND, N>::node(j);
-        double q[NV], y[NV];
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            q[v] = a.Q[v * Nd + g0 + j];
-            y[v] = A.Y[v * Nd + g0 + j];
-        }
-        const double cj = A.c / (CURV ? a.ngeom[ND * ND * Nd + g0 + j]
-                                      : a.egeom[(int64_t)(e0 + j / NPE) * a.egeom_stride + ND * ND]);
+    for (int t = 0; t < NPT; ++t) {
+        const int j = tid + t * TPB;
+        if (j >= nnb) break;
+        const int jj = Nodes<ND, N>::node(j);
+        const int b = BATCH ? t : 0;
+        if constexpr (!BATCH) state(t, 0);
+        const double* const q = q_[b];
+        const double* const y = y_[b];
+        const double cj = A.c / j_[b];
         if constexpr (CURV) {
 #pragma unroll
-            for (int c = 0; c < ND * ND; ++c) sM[c * NN + jj] = 0.5 * a.ngeom[c * Nd + g0 + j];
+            for (int c = 0; c < ND * ND; ++c) sM[c * NN + jj] = 0.5 * m_[b][c];
         }
         const double ir = rcp(q[0]);
         double u[ND], uu = 0;
@@ -597,8 +622,25 @@ __global__ void __launch_bounds__((LCfg<ND, N, TP, CURV>::TPB)) k_svjp(const Vjp
         __syncthreads();
     }
 
-    // ---- per node: pullback of the inputs, face terms, epilogue ----------------------------
-    for (int j = tid; j < nnb; j += TPB) {
+    // ---- per node: pullback of the inputs, face terms, epilogue (its operands first) ------------
+    double p_[3][NB][NV];
+    auto operands = [&](int t, int b) {
+        const int j = tid + t * TPB < nnb ? tid + t * TPB : 0;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            p_[0][b][v] = A.P0 ? (A.P0 + (v * Nd + g0))[j] : 0.0;
+            p_[1][b][v] = A.P1 ? (A.P1 + (v * Nd + g0))[j] : 0.0;
+            p_[2][b][v] = A.P2 ? (A.P2 + (v * Nd + g0))[j] : 0.0;
+        }
+    };
+    if constexpr (BATCH) {
+#pragma unroll
+        for (int t = 0; t < NPT; ++t) operands(t, t);
+    }
+#pragma unroll
+    for (int it = 0; it < NPT; ++it) {
+        const int j = tid + it * TPB;
+        if (j >= nnb) break;
         const int jj = Nodes<ND, N>::node(j);
         double t[NA], V[NV];
 #pragma unroll
@@ -645,19 +687,13 @@ __global__ void __launch_bounds__((LCfg<ND, N, TP, CURV>::TPB)) k_svjp(const Vjp
                 for (int v = 0; v < NV; ++v) V[v] += F[v * NPF];
             }
         }
-        double p0[NV], p1[NV], p2[NV];
+        const int b = BATCH ? it : 0;
+        if constexpr (!BATCH) operands(it, 0);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int64_t i = v * Nd + g0 + j;
-            p0[v] = A.P0 ? A.P0[i] : 0.0;
-            p1[v] = A.P1 ? A.P1[i] : 0.0;
-            p2[v] = A.P2 ? A.P2[i] : 0.0;
-        }
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const int64_t i = v * Nd + g0 + j;
-            const double o = V[v] + A.a0 * p0[v] + A.a1 * p1[v];
-            if (A.o1) A.o1[i] = A.b0 * o + A.b1 * p1[v] + A.b2 * p2[v];
+            const double o = V[v] + A.a0 * p_[0][b][v] + A.a1 * p_[1][b][v];
+            if (A.o1) A.o1[i] = A.b0 * o + A.b1 * p_[1][b][v] + A.b2 * p_[2][b][v];
             A.o0[i] = o;
         }
     }

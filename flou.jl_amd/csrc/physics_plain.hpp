@@ -203,7 +203,7 @@ constexpr int tp_slots() {
 }
 
 // F of the logarithmic mean (a + b)/(2F) (see logarithmic_mean).  Where a quotient here is not
-// finite its operands are a vacuum's or negative ones', and the flux is NaN either way.
+// finite an operand is 0, infinite or negative, and what the mean enters is NaN either way.
 template <typename T>
 __device__ inline T logmean_factor(T al, T ar, int* err) {
     const T xi = fdiv(al, ar);
@@ -238,7 +238,7 @@ __device__ __forceinline__ void pair_flux(const T* A, const T* B, T ja, T gm1, i
         for (int k = 0; k < ND; ++k) um[k] = A[1 + k] + B[1 + k];
         const T hs = A[0] + B[0], sb = A[ND + 1] + B[ND + 1];
         const T rho = fdiv(hs, logmean_factor(A[0], B[0], err));
-        const T p = fdiv(hs, sb);
+        const T p = xdiv(hs, sb);  // 0 where a node has no pressure (β infinite): mass and momentum are finite
         const T beta2 = fdiv(sb, logmean_factor(A[ND + 1], B[ND + 1], err));  // 2β̂
         T sq = A[1] * A[1];  // (|u1|² + |u2|²)/4
 #pragma unroll

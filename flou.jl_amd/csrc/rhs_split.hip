@@ -506,10 +506,11 @@ __device__ __forceinline__ void pair_flux_along(const double* A, const double* B
         double mass, p, e;
         if constexpr (TP == TP_CHANDRASEKHAR) {
             const double sb = A[ND + 1] + B[ND + 1];
-            const double ir = rcp(hs), ib = rcp(sb);
+            const Recip<double> isb(sb);
+            const double ir = rcp(hs), ib = isb.y;
             const double fr = mean_factor(A[0], B[0], ir, err), fb = mean_factor(A[ND + 1], B[ND + 1], ib, err);
             mass = hs * rcp(fr) * un;
-            p = hs * ib;
+            p = isb.div(hs);  // 0 where a node has no pressure, see plain::pair_flux
             // 1/(2β̂(γ-1)) + p/ρ̂ + |ū|² - (|u1|² + |u2|²)/4
             e = __builtin_fma(fb * ib, ig1, fr * ib) - (A[ND + 2] + B[ND + 2]);
 #pragma unroll

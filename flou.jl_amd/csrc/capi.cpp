@@ -1142,6 +1142,9 @@ int flou_hip_check(flou_hip_handle* h) {
 }
 
 namespace {
+// A run to tfinal is over from here on: 1e-14 of it short, whatever its sign.
+double end_time(double tfinal) { return tfinal * (tfinal < 0.0 ? 1 + 1e-14 : 1 - 1e-14); }
+
 // The time loop of flou_hip_timeintegrate: nsteps steps of dt (the CFL step at most dt), or,
 // with until, steps of at most dt until *t reaches tfinal.
 int time_loop(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t nsteps, bool until, double tfinal,
@@ -1156,8 +1159,10 @@ int time_loop(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t ns
     // work[1]); `cur` carries over from step to step and is copied back once at the end.
     void* cur = Q;
     void* oth = h->d_work[0];
+    const double end = end_time(tfinal);
+    bool stalled = false;
     int rc = 0;
-    for (int64_t step = 0; (until ? t < tfinal * (1 - 1e-14) : step < nsteps) && !rc; ++step) {
+    for (int64_t step = 0; (until ? t < end : step < nsteps) && !rc; ++step) {
         double dts = until ? std::min(dt, tfinal - t) : dt;
         if (cfl > 0.0) {
             double m;
@@ -1166,6 +1171,10 @@ int time_loop(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t ns
             // a non-physical state of the step before: the check below reports it
             if (until && step && h->h_res->flag) break;
             dts = std::min(m, dts);
+        }
+        if (until && !(t + dts > t)) {  // would never reach tfinal
+            stalled = true;
+            break;
         }
         if (scheme == FLOU_HIP_SSPRK33) {
             rc = flou_hip_rk_stage(h, scheme, 0, dts, t, Q, nullptr, nullptr, h->d_work[0]);
@@ -1182,7 +1191,9 @@ int time_loop(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t ns
     if (rc) return rc;
     if (cur != Q) HIPCHECK(h, hipMemcpyAsync(Q, cur, bytes, hipMemcpyDeviceToDevice, h->stream));
     if (t_inout) *t_inout = t;
-    return flou_hip_check(h);
+    rc = flou_hip_check(h);
+    if (!rc && stalled) return fail(h, FLOU_HIP_EDOMAIN, "the time step no longer advances the time");
+    return rc;
 }
 }  // namespace
 
@@ -1195,7 +1206,7 @@ int flou_hip_timeintegrate(flou_hip_handle* h, int32_t scheme, void* Q, double d
 int flou_hip_timeintegrate_until(flou_hip_handle* h, int32_t scheme, void* Q, double dt, double tfinal, double cfl,
                                  double* t_inout) {
     if (!h || !Q || !t_inout) return FLOU_HIP_EINVAL;
-    if (!(*t_inout < tfinal * (1 - 1e-14))) return FLOU_HIP_OK;  // nothing to do
+    if (!(*t_inout < end_time(tfinal))) return FLOU_HIP_OK;  // nothing to do
     return time_loop(h, scheme, Q, dt, 0, true, tfinal, cfl, t_inout);
 }
 

@@ -214,8 +214,9 @@ int flou_hip_timeintegrate(flou_hip_handle* h, int32_t scheme, void* Q, double d
 
 /* The CFL-controlled loop of timeintegrate up to tfinal (FlouTime.jl:34-56, 92-104), in place
  * on Q: before every step dt_step = min(get_max_dt(Q, cfl), dt, tfinal - t), from *t_inout
- * until t >= tfinal (1 - 1e-14); with cfl <= 0 the steps are min(dt, tfinal - t).  Returns FLOU_HIP_EDOMAIN once a
- * step met a non-physical state; later steps are not taken. */
+ * until t is within 1e-14 |tfinal| of tfinal; with cfl <= 0 the steps are min(dt, tfinal - t).  Returns
+ * FLOU_HIP_EDOMAIN once a step met a non-physical state (later steps are not taken), or when the step no longer
+ * advances t (an unbounded wave speed, for instance). */
 int flou_hip_timeintegrate_until(flou_hip_handle* h, int32_t scheme, void* Q, double dt,
                                  double tfinal, double cfl, double* t_inout);
 

@@ -1,0 +1,50 @@
+"""The library's loop to a final time (flou_hip_timeintegrate_until, timeintegrate(.., cfl=..)).
+
+Runs that end below zero, time steps that stop advancing the time, non-physical states met on the way,
+interrupts.  Steps of 1/64 (exact in the time's arithmetic) so that a run and its shifted copy take the same
+ones, bit for bit.
+"""
+import ctypes
+import signal
+import time
+
+import numpy as np
+import pytest
+
+import flouhip as F
+from cases import random_euler_state
+from flouhip import _capi as C
+from test_gpu_reductions import build
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def start(amp=0.01):
+    disc, eq, orc = build(2, 3, [2, 2])
+    Q = random_euler_state(orc.coords()[0], 2, seed=3, amp=amp)
+    return disc, eq, Q
+
+
+@pytest.mark.parametrize("solver", [F.SSPRK33, F.CarpenterKennedy2N54])
+@pytest.mark.parametrize("t0,tf", [(-1.0, -0.5), (-0.25, 0.25), (-0.5, 0.0)])
+def test_final_times_of_any_sign(t0, tf, solver):
+    disc, eq, Q = start()
+    a, b = disc.to_device(Q), disc.to_device(Q)
+    assert F.get_max_dt(a, disc, eq, 100.0) > 1 / 64
+    F.timeintegrate(a, disc, eq, solver(), tf, dt=1 / 64, cfl=100.0, t0=t0)
+    F.timeintegrate(b, disc, eq, solver(), tf - t0, dt=1 / 64, cfl=100.0)
+    assert torch.equal(a, b) and torch.isfinite(a).all()
+
+
+def test_step_that_no_longer_advances():
+    disc, eq, Q = start()
+    Qd = disc.to_device(Q)
+    Qd[3, 5] = float("inf")  # an unbounded wave speed: the CFL step is 0
+    with pytest.raises(F.DomainError, match="advance"):
+        F.timeintegrate(Qd, disc, eq, F.SSPRK33(), 1.0, dt=1e-2, cfl=0.2)
+    Qd = disc.to_device(Q)
+    with pytest.raises(F.DomainError, match="advance"):  # 1 + 1e-17 == 1
+        F.timeintegrate(Qd, disc, eq, F.SSPRK33(), 2.0, dt=1e-17, cfl=0.2, t0=1.0)
+    assert np.array_equal(disc.to_host(Qd), Q)
+    disc.check()

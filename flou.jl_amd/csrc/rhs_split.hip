@@ -28,6 +28,7 @@
 // Compile with -DFLOUHIP_ND=1|2|3.
 #include "common.hpp"
 #include "faces.hpp"
+#include "pair_along.hpp"
 #include "physics_plain.hpp"
 #include "stage.hpp"
 
@@ -442,91 +443,15 @@ static RhsLauncherF64 pick_tp(int tp) {
 //
 // The same form with a metric per node.  The general kernel forms every component of a pair's
 // flux and contracts them with the mean metric n̄, with IEEE quotients throughout, and reads
-// metrics from memory once per pair.  Here the flux along n̄ is formed directly (ρ̂ ū·n̄ first),
-// quotients by reciprocals good to an ulp and sums by fused multiply-adds, so results agree
-// with the general kernel's up to rounding; a direction's metric rows lie in LDS beside the
-// flux inputs.  Faces: the flux along n from the master's frame; every sum over the two sides
+// metrics from memory once per pair.  Here the flux along n̄ is formed directly (pair_along.hpp), sums
+// by fused multiply-adds, so results agree with the general kernel's up to rounding and are no
+// less exact; a direction's metric rows lie in LDS beside the flux inputs.  Eight-wave blocks run two
+// to a CU up to 128 registers: they read a node's velocities from its slots again for each direction (3-D
+// N=6, held in registers: 133, one block per CU, 84 us against 61 at 0.6 M nodes).  Faces: the flux along n from the master's frame; every sum over the two sides
 // commutes and is rounded the same way on both, so that the sides' fluxes are opposite bit for bit.
 // What bounds it: waits between the barriers at two or three blocks per CU; HBM moves 1.6 GB a
 // stage at 11.2 M nodes, 0.34 ms at a copy's rate.  Measured, Chandrasekhar, SSPRK33 steps: 3-D N=6,
 // 11.2 M nodes: 9.1 -> 3.0 ms; N=5, 7.1 M nodes: 3.6 -> 1.8 ms.
-
-__device__ __forceinline__ double rcp(double x) {  // 1/x to about an ulp
-    const double y = __builtin_amdgcn_rcp(x), e = __builtin_fma(-x, y, 1.0);
-    return __builtin_fma(y, __builtin_fma(e, e, e), y);
-}
-
-// F of the logarithmic mean, see plain::logmean_factor; is: 1/(a + b).
-__device__ __forceinline__ double mean_factor(double a, double b, double is, int* err) {
-    const double f = (a - b) * is, u = f * f;
-    if (u < 0.01) {
-        const double s = __builtin_fma(u, 1.0 / 7, 1.0 / 5);
-        return __builtin_fma(u, __builtin_fma(u, s, 1.0 / 3), 1.0);
-    }
-    return plain::dlog(a * rcp(b), err) * rcp(2 * f);
-}
-
-// Flux input slots: plain::put_slots and, for Chandrasekhar, |u|²/4.
-template <int ND, int TP>
-constexpr int curved_slots() {
-    return plain::tp_slots<ND, TP>() + (TP == TP_CHANDRASEKHAR ? 1 : 0);
-}
-
-// Two-point flux along the mean metric n of two nodes.
-template <int ND, int TP>
-__device__ __forceinline__ void pair_flux_along(const double* A, const double* B, const double* n, double ig1, int* err,
-                                                double* F) {
-    if constexpr (TP == TP_STDAVG) {
-        double w[2], m[2];
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const double* X = s ? B : A;
-            w[s] = X[0] * n[0];
-            m[s] = X[ND + 1] * n[0];
-#pragma unroll
-            for (int k = 1; k < ND; ++k) {
-                w[s] = __builtin_fma(X[k], n[k], w[s]);
-                m[s] = __builtin_fma(X[ND + 1 + k], n[k], m[s]);
-            }
-        }
-        const double p = A[ND] + B[ND];
-        F[0] = m[0] + m[1];
-#pragma unroll
-        for (int c = 0; c < ND; ++c)
-            F[1 + c] = __builtin_fma(A[ND + 1 + c], w[0], __builtin_fma(B[ND + 1 + c], w[1], p * n[c]));
-        F[ND + 1] = __builtin_fma(A[2 * ND + 1] + A[ND], w[0], (B[2 * ND + 1] + B[ND]) * w[1]);
-    } else {
-        double u[ND];
-#pragma unroll
-        for (int k = 0; k < ND; ++k) u[k] = A[1 + k] + B[1 + k];
-        double un = u[0] * n[0];
-#pragma unroll
-        for (int k = 1; k < ND; ++k) un = __builtin_fma(u[k], n[k], un);
-        const double hs = A[0] + B[0];
-        double mass, p, e;
-        if constexpr (TP == TP_CHANDRASEKHAR) {
-            const double sb = A[ND + 1] + B[ND + 1];
-            const Recip<double> isb(sb);
-            const double ir = rcp(hs), ib = isb.y;
-            const double fr = mean_factor(A[0], B[0], ir, err), fb = mean_factor(A[ND + 1], B[ND + 1], ib, err);
-            mass = hs * rcp(fr) * un;
-            p = isb.div(hs);  // 0 where a node has no pressure, see plain::pair_flux
-            // 1/(2β̂(γ-1)) + p/ρ̂ + |ū|² - (|u1|² + |u2|²)/4
-            e = __builtin_fma(fb * ib, ig1, fr * ib) - (A[ND + 2] + B[ND + 2]);
-#pragma unroll
-            for (int k = 0; k < ND; ++k) e = __builtin_fma(u[k], u[k], e);
-            F[ND + 1] = mass * e;
-        } else {
-            p = A[ND + 1] + B[ND + 1];
-            e = A[ND + 2] + B[ND + 2];
-            mass = hs * un;
-            F[ND + 1] = __builtin_fma(mass, e, p * un);
-        }
-        F[0] = mass;
-#pragma unroll
-        for (int c = 0; c < ND; ++c) F[1 + c] = __builtin_fma(mass, u[c], p * n[c]);
-    }
-}
 
 // One direction: pairs and the nodes' own fluxes into the table, then (LOADS between) the
 // nodes' D♯ rows over it.  m: the metric row of the own node.
@@ -544,10 +469,15 @@ __device__ __forceinline__ void curved_direction(const RhsArgs<double>& a, const
     node_line<ND, N>(node, DIR, lf, ii);
     if (valid) {
         double* t = sTab + (DIAG + tid) * KS;
-        double w = u[0] * m[0];
+        const double* s = sS + M::node(tid);
+        auto vel = [&](int k) { return C::TPB > 256 ? curved_velocity<TP, SN>(s, k) : u[k]; };
+        double w = vel(0) * m[0], mass = q[1] * m[0];
 #pragma unroll
-        for (int k = 1; k < ND; ++k) w = __builtin_fma(u[k], m[k], w);
-        t[0] = q[0] * w;
+        for (int k = 1; k < ND; ++k) {
+            w = __builtin_fma(vel(k), m[k], w);
+            mass = __builtin_fma(q[1 + k], m[k], mass);
+        }
+        t[0] = mass;
 #pragma unroll
         for (int c = 0; c < ND; ++c) t[(1 + c) * VS] = __builtin_fma(q[1 + c], w, p * m[c]);
         t[(NV - 1) * VS] = (q[NV - 1] + p) * w;
@@ -642,15 +572,7 @@ __global__ void __launch_bounds__((SCfg<ND, N>::TPB)) k_split_curved(const RhsAr
 #pragma unroll
         for (int k = 0; k < ND; ++k) u[k] = P[1 + k];
         p = P[ND + 1];
-        if (valid) {
-            plain::put_slots<T, ND, TP, SN>(sS + jj, q, P, ir);
-            if constexpr (TP == TP_CHANDRASEKHAR) {
-                T s = u[0] * u[0];
-#pragma unroll
-                for (int k = 1; k < ND; ++k) s = __builtin_fma(u[k], u[k], s);
-                sS[(NS - 1) * SN + jj] = T(0.25) * s;
-            }
-        }
+        if (valid) curved_node<ND, TP, SN>(sS + jj, q, P, ir);
     }
     put_metric();
     __syncthreads();

@@ -375,6 +375,13 @@ int await_result(flou_hip_handle* h) {
     return FLOU_HIP_OK;
 }
 
+// The domain-error flag as of the stream's work so far, to h_res.
+int read_flag(flou_hip_handle* h) {
+    const hipError_t e = launch_flag(next_out(h), h->stream);
+    if (e != hipSuccess) return fail(h, FLOU_HIP_EDEVICE, hipGetErrorString(e));
+    return await_result(h);
+}
+
 bool overlaps(const void* a, const void* b, size_t bytes) {
     const char* x = (const char*)a;
     const char* y = (const char*)b;
@@ -1125,9 +1132,7 @@ int flou_hip_integrate(flou_hip_handle* h, const void* Q, int32_t ivar, double* 
 
 int flou_hip_check(flou_hip_handle* h) {
     if (!h) return FLOU_HIP_EINVAL;
-    const hipError_t e = launch_flag(next_out(h), h->stream);
-    if (e != hipSuccess) return fail(h, FLOU_HIP_EDEVICE, hipGetErrorString(e));
-    const int rc = await_result(h);
+    const int rc = read_flag(h);
     if (rc) return rc;
     const int flag = h->h_res->flag;
     if (flag) {
@@ -1168,10 +1173,13 @@ int time_loop(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t ns
             double m;
             rc = flou_hip_max_dt(h, cur, cfl, &m);
             if (rc) break;
-            // a non-physical state of the step before: the check below reports it
-            if (until && step && h->h_res->flag) break;
             dts = std::min(m, dts);
+        } else if (until && step) {
+            rc = read_flag(h);
+            if (rc) break;
         }
+        // a non-physical state of the step before (get_max_dt brings the flag too): the check below reports it
+        if (until && step && h->h_res->flag) break;
         if (until && !(t + dts > t)) {  // would never reach tfinal
             stalled = true;
             break;

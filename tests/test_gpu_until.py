@@ -48,3 +48,15 @@ def test_step_that_no_longer_advances():
         F.timeintegrate(Qd, disc, eq, F.SSPRK33(), 2.0, dt=1e-17, cfl=0.2, t0=1.0)
     assert np.array_equal(disc.to_host(Qd), Q)
     disc.check()
+
+
+@pytest.mark.parametrize("cfl", [0.0, 0.2])
+def test_no_step_after_a_non_physical_state(cfl):
+    """The step that meets the state is the last: t stays where it ended."""
+    disc, eq, Q = start()
+    Q[7, 3] = -1.0  # negative pressure
+    Qd = disc.to_device(Q)
+    t = ctypes.c_double(0.0)
+    rc = C.lib.flou_hip_timeintegrate_until(disc.h, C.SSPRK33, disc._dptr(Qd), 1e-4, 1.0, cfl, ctypes.byref(t))
+    assert rc == C.EDOMAIN and 0 < t.value <= 1e-4
+    disc.check()

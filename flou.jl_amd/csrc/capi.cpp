@@ -1151,9 +1151,9 @@ namespace {
 double end_time(double tfinal) { return tfinal * (tfinal < 0.0 ? 1 + 1e-14 : 1 - 1e-14); }
 
 // The time loop of flou_hip_timeintegrate: nsteps steps of dt (the CFL step at most dt), or,
-// with until, steps of at most dt until *t reaches tfinal.
+// with until, steps of at most dt until *t reaches tfinal or `seconds` of wall time have passed.
 int time_loop(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t nsteps, bool until, double tfinal,
-              double cfl, double* t_inout) {
+              double cfl, double seconds, double* t_inout) {
     if (scheme < FLOU_HIP_SSPRK33 || scheme > FLOU_HIP_ORK256) return fail(h, FLOU_HIP_EINVAL, "unknown scheme");
     if (!(dt > 0.0)) return fail(h, FLOU_HIP_EINVAL, "dt must be positive");
     const size_t bytes = flou_hip_state_bytes(h);
@@ -1165,6 +1165,7 @@ int time_loop(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t ns
     void* cur = Q;
     void* oth = h->d_work[0];
     const double end = end_time(tfinal);
+    const auto t0 = std::chrono::steady_clock::now();
     bool stalled = false;
     int rc = 0;
     for (int64_t step = 0; (until ? t < end : step < nsteps) && !rc; ++step) {
@@ -1195,6 +1196,9 @@ int time_loop(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t ns
             }
         }
         t += dts;
+        // (where the state is back in Q, so that a slice costs no copy)
+        if (until && cur == Q && std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() >= seconds)
+            break;
     }
     if (rc) return rc;
     if (cur != Q) HIPCHECK(h, hipMemcpyAsync(Q, cur, bytes, hipMemcpyDeviceToDevice, h->stream));
@@ -1208,14 +1212,19 @@ int time_loop(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t ns
 int flou_hip_timeintegrate(flou_hip_handle* h, int32_t scheme, void* Q, double dt, int64_t nsteps,
                            double cfl, double* t_inout) {
     if (!h || !Q || nsteps < 0) return FLOU_HIP_EINVAL;
-    return time_loop(h, scheme, Q, dt, nsteps, false, 0.0, cfl, t_inout);
+    return time_loop(h, scheme, Q, dt, nsteps, false, 0.0, cfl, 0.0, t_inout);
 }
 
 int flou_hip_timeintegrate_until(flou_hip_handle* h, int32_t scheme, void* Q, double dt, double tfinal, double cfl,
                                  double* t_inout) {
+    return flou_hip_timeintegrate_slice(h, scheme, Q, dt, tfinal, cfl, INFINITY, t_inout);
+}
+
+int flou_hip_timeintegrate_slice(flou_hip_handle* h, int32_t scheme, void* Q, double dt, double tfinal, double cfl,
+                                 double seconds, double* t_inout) {
     if (!h || !Q || !t_inout) return FLOU_HIP_EINVAL;
     if (!(*t_inout < end_time(tfinal))) return FLOU_HIP_OK;  // nothing to do
-    return time_loop(h, scheme, Q, dt, 0, true, tfinal, cfl, t_inout);
+    return time_loop(h, scheme, Q, dt, 0, true, tfinal, cfl, seconds, t_inout);
 }
 
 int flou_hip_rhs_vjp(flou_hip_handle* h, const void* Q, const void* dQbar, void* Qbar) {

@@ -75,6 +75,8 @@ SYMBOLS = {
                                          ctypes.c_double, _vp, _vp, _vp, _vp]),
     "flou_hip_timeintegrate_until": (ctypes.c_int, [_vp, ctypes.c_int32, _vp, ctypes.c_double, ctypes.c_double,
                                                     ctypes.c_double, ctypes.POINTER(ctypes.c_double)]),
+    "flou_hip_timeintegrate_slice": (ctypes.c_int, [_vp, ctypes.c_int32, _vp, ctypes.c_double, ctypes.c_double,
+                                                    ctypes.c_double, ctypes.c_double, ctypes.POINTER(ctypes.c_double)]),
     "flou_hip_timeintegrate": (ctypes.c_int, [_vp, ctypes.c_int32, _vp, ctypes.c_double,
                                               ctypes.c_int64, ctypes.c_double, _d]),
     "flou_hip_max_dt": (ctypes.c_int, [_vp, _vp, ctypes.c_double, _d]),

@@ -354,6 +354,9 @@ def make_callback_list(*callbacks):
     return callbacks[0] if len(callbacks) == 1 else list(callbacks)
 
 
+_SLICE = 0.05  # seconds of a CFL-controlled run per library call
+
+
 def timeintegrate(Q0, disc, equation, solver, tfinal, dt, cfl=None, t0=0.0, callback=None):
     """timeintegrate(Q0, disc, equation, solver, tf; dt, adaptive=false) -- FlouTime.jl:34-56.
 
@@ -413,8 +416,11 @@ def _timeintegrate(Q0, disc, code, tfinal, dt, cfl, t0):
             C.check(C.lib.flou_hip_timeintegrate(disc.h, code, ptr, float(rest), 1, 0.0,
                                                  ctypes.byref(t)), disc.h, "timeintegrate")
     else:
-        C.check(C.lib.flou_hip_timeintegrate_until(disc.h, code, ptr, float(dt), float(tfinal), float(cfl),
-                                                   ctypes.byref(t)), disc.h, "timeintegrate")
+        before = -np.inf
+        while t.value > before:  # in slices, between which Python handles signals (Ctrl-C)
+            before = t.value
+            C.check(C.lib.flou_hip_timeintegrate_slice(disc.h, code, ptr, float(dt), float(tfinal), float(cfl), _SLICE,
+                                                       ctypes.byref(t)), disc.h, "timeintegrate")
     torch.cuda.synchronize()
     return Q0, time.perf_counter() - tic
 

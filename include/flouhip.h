@@ -220,6 +220,12 @@ int flou_hip_timeintegrate(flou_hip_handle* h, int32_t scheme, void* Q, double d
 int flou_hip_timeintegrate_until(flou_hip_handle* h, int32_t scheme, void* Q, double dt,
                                  double tfinal, double cfl, double* t_inout);
 
+/* A slice of flou_hip_timeintegrate_until: the same steps, but returns FLOU_HIP_OK with *t_inout short of
+ * tfinal after a step (two for the 2N schemes) by whose end `seconds` of wall time have passed.  Called again from there
+ * until it no longer moves t, it gives a host that must stay responsive (signals, a user interface) the same run. */
+int flou_hip_timeintegrate_slice(flou_hip_handle* h, int32_t scheme, void* Q, double dt, double tfinal, double cfl,
+                                 double seconds, double* t_inout);
+
 /* get_max_dt(Q, disc, eq, cfl) -- MultielementDiscontinuous.jl:162-178 (FP64 result). */
 int flou_hip_max_dt(flou_hip_handle* h, const void* Q, double cfl, double* out);
 

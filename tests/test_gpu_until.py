@@ -60,3 +60,44 @@ def test_no_step_after_a_non_physical_state(cfl):
     rc = C.lib.flou_hip_timeintegrate_until(disc.h, C.SSPRK33, disc._dptr(Qd), 1e-4, 1.0, cfl, ctypes.byref(t))
     assert rc == C.EDOMAIN and 0 < t.value <= 1e-4
     disc.check()
+
+
+class Alarm(Exception):
+    pass
+
+
+def test_a_run_can_be_interrupted():
+    """A signal ends a run of many steps soon, and leaves a state between two steps."""
+    disc, eq, Q = start()
+    Qd = disc.to_device(Q)
+
+    def ring(*_):
+        raise Alarm
+
+    old = signal.signal(signal.SIGALRM, ring)
+    signal.setitimer(signal.ITIMER_REAL, 0.5)
+    tic = time.perf_counter()
+    try:
+        with pytest.raises(Alarm):
+            # 200,000 steps, some seconds
+            F.timeintegrate(Qd, disc, eq, F.CarpenterKennedy2N54(), 0.2, dt=1e-6, cfl=0.2)
+    finally:
+        signal.setitimer(signal.ITIMER_REAL, 0)
+        signal.signal(signal.SIGALRM, old)
+    assert time.perf_counter() - tic < 2.0
+    assert torch.isfinite(Qd).all() and F.get_max_dt(Qd, disc, eq, 0.2) > 1e-6
+
+
+@pytest.mark.parametrize("scheme", [C.SSPRK33, C.CK2N54])
+def test_slices_take_the_same_steps(scheme):
+    disc, eq, Q = start(0.1)
+    a, b = disc.to_device(Q), disc.to_device(Q)
+    tf, dt = 7.3e-3, 1e-3
+    ta, tb = ctypes.c_double(0.0), ctypes.c_double(0.0)
+    assert C.lib.flou_hip_timeintegrate_until(disc.h, scheme, disc._dptr(a), dt, tf, 0.1, ctypes.byref(ta)) == C.OK
+    calls, before = 0, -1.0
+    while tb.value > before:
+        before = tb.value
+        assert C.lib.flou_hip_timeintegrate_slice(disc.h, scheme, disc._dptr(b), dt, tf, 0.1, 0.0, ctypes.byref(tb)) == C.OK
+        calls += 1
+    assert calls > 3 and ta.value == tb.value and torch.equal(a, b)

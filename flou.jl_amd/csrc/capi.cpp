@@ -1135,6 +1135,7 @@ int flou_hip_check(flou_hip_handle* h) {
     const int rc = read_flag(h);
     if (rc) return rc;
     const int flag = h->h_res->flag;
+    HIPCHECK(h, hipStreamSynchronize(h->stream));  // the word in h_res arrives before the stream reports its end
     if (flag) {
         HIPCHECK(h, hipMemsetAsync(h->d_err, 0, sizeof(int), h->stream));
         HIPCHECK(h, hipStreamSynchronize(h->stream));

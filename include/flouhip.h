@@ -207,7 +207,7 @@ int flou_hip_rk_stage(flou_hip_handle* h, int32_t scheme, int32_t stage, double 
 /* Full fixed-dt time integration of nsteps steps in place on Q, with handle-owned work
  * buffers (timeintegrate(Q0, disc, eq, solver, tf; dt, adaptive=false), FlouTime.jl:34-56).
  * If cfl > 0, dt is recomputed before every step as min(get_max_dt(Q, cfl), dt) (the
- * get_cfl_callback pattern, FlouTime.jl:92-104) and `dt` acts as Δtmax.
+ * get_cfl_callback pattern, FlouTime.jl:92-104) and `dt` acts as Δtmax.  Synchronises the stream.
  * Returns FLOU_HIP_EDOMAIN if a non-physical state was met ("Simulation crashed!"). */
 int flou_hip_timeintegrate(flou_hip_handle* h, int32_t scheme, void* Q, double dt,
                            int64_t nsteps, double cfl, double* t_inout);
@@ -226,7 +226,10 @@ int flou_hip_timeintegrate_until(flou_hip_handle* h, int32_t scheme, void* Q, do
 int flou_hip_timeintegrate_slice(flou_hip_handle* h, int32_t scheme, void* Q, double dt, double tfinal, double cfl,
                                  double seconds, double* t_inout);
 
-/* get_max_dt(Q, disc, eq, cfl) -- MultielementDiscontinuous.jl:162-178 (FP64 result). */
+/* get_max_dt(Q, disc, eq, cfl) -- MultielementDiscontinuous.jl:162-178 (FP64 result).
+ * flou_hip_max_dt, flou_hip_integrate and flou_hip_monitor return once their result has arrived in host
+ * memory: all earlier work of the handle's stream is complete then, though the stream itself may
+ * report its end some microseconds later (flou_hip_check and flou_hip_synchronize wait for that). */
 int flou_hip_max_dt(flou_hip_handle* h, const void* Q, double cfl, double* out);
 
 /* integrate(Q, disc, ivar) -- MultielementDiscontinuous.jl:148-160 (FP64 result); ivar
@@ -271,7 +274,7 @@ int flou_hip_monitor(flou_hip_handle* h, const void* Q, int32_t kind, double* ou
 int flou_hip_equispaced(flou_hip_handle* h, int32_t m, const double* node2eq, const void* Q,
                         int32_t ncols, void* Qe);
 
-/* Synchronises, returns FLOU_HIP_EDOMAIN if a kernel met a non-physical state since the
+/* Synchronises the stream, returns FLOU_HIP_EDOMAIN if a kernel met a non-physical state since the
  * last call (sqrt or log of a negative number in the reference), and clears the flag. */
 int flou_hip_check(flou_hip_handle* h);
 

@@ -72,6 +72,8 @@ struct flou_hip_handle {
     RhsLauncherF32 l32 = nullptr;
     VjpLauncherF64 v64 = nullptr;
     VjpLauncherF32 v32 = nullptr;
+    const char* rhs_name = "k_plain";  // kernels behind l64/l32 and v64/v32
+    const char* vjp_name = "k_vjp";
     std::string vjp_why;  // why the adjoint is unavailable for this handle
     // FP32 fast path (2-D/3-D split form on axis-aligned affine or curved elements)
     FastLauncher lfast = nullptr;
@@ -664,6 +666,18 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
             h->l32 = nd == 1 ? hybrid_f32_1(n, h->tp, diag)
                              : (nd == 2 ? hybrid_f32_2(n, h->tp, diag) : hybrid_f32_3(n, h->tp, diag));
         if (!h->l64 && !h->l32) return bad(FLOU_HIP_EUNSUPPORTED, "no kernel for this combination");
+        h->rhs_name = "k_hybrid";
+        RhsLauncherF64 f64 = nullptr;
+        RhsLauncherF32 f32 = nullptr;
+        if (diag && nd < 3 && h->prec == FLOU_HIP_FP64)
+            f64 = nd == 1 ? hybrid_lines_f64_1(n, h->tp, ne) : hybrid_lines_f64_2(n, h->tp, ne);
+        else if (diag && nd < 3)
+            f32 = nd == 1 ? hybrid_lines_f32_1(n, h->tp, ne) : hybrid_lines_f32_2(n, h->tp, ne);
+        if (f64 || f32) {
+            h->l64 = f64;
+            h->l32 = f32;
+            h->rhs_name = "k_hybrid_lines";
+        }
     } else if (h->prec == FLOU_HIP_FP64) {
         h->l64 = nd == 1 ? plain_f64_1d(n, h->eq, kvol, h->tp, h->curved)
                          : (nd == 2 ? plain_f64_2d(n, h->eq, kvol, h->tp, h->curved)
@@ -675,13 +689,20 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
         const bool lxf = h->savg == FLOU_HIP_AVG_STD &&
                          (h->sdiss == FLOU_HIP_DISS_NONE || h->sdiss == FLOU_HIP_DISS_LXF);
         if (kvol == VOL_SPLIT && h->eq == FLOU_HIP_EULER && lxf && diag && !oriented && h->gather &&
-            h->lift_end)
+            h->lift_end) {
             h->l64 = nd == 1 ? split_f64_1(n, h->tp) : (nd == 2 ? split_f64_2(n, h->tp) : split_f64_3(n, h->tp));
+            h->rhs_name = "k_split";
+        }
         // and on curved elements (3-D N=6, 11.2 M nodes: 3.0 -> 1.0 ms per stage)
-        else if (kvol == VOL_SPLIT && h->eq == FLOU_HIP_EULER && lxf && h->curved && h->gather && h->lift_end)
+        else if (kvol == VOL_SPLIT && h->eq == FLOU_HIP_EULER && lxf && h->curved && h->gather && h->lift_end) {
             h->l64 = nd == 2 ? split_curved_f64_2(n, h->tp) : split_curved_f64_3(n, h->tp);
+            h->rhs_name = "k_split_curved";
+        }
         if (kvol == VOL_SPLIT && h->eq == FLOU_HIP_EULER && nd == 1 && diag && h->gather && h->lift_end)
-            if (const RhsLauncherF64 f = split_f64_1_small(n, h->tp, d->nelements)) h->l64 = f;
+            if (const RhsLauncherF64 f = split_f64_1_small(n, h->tp, ne)) {
+                h->l64 = f;
+                h->rhs_name = "k_split_1d";
+            }
     } else {
         h->l32 = nd == 1 ? plain_f32_1d(n, h->eq, kvol, h->tp, h->curved)
                          : (nd == 2 ? plain_f32_2d(n, h->eq, kvol, h->tp, h->curved)
@@ -693,6 +714,7 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
     if (h->vol == FLOU_HIP_STRONG && diag && !oriented && h->gather && h->lift_end &&
         (h->eq == FLOU_HIP_ADVECTION || (h->savg == FLOU_HIP_AVG_STD && (h->sdiss == FLOU_HIP_DISS_NONE ||
                                                                           h->sdiss == FLOU_HIP_DISS_LXF)))) {
+        h->rhs_name = "k_strong";
         if (h->prec == FLOU_HIP_FP64)
             h->l64 = nd == 1 ? strong_f64_1(n, h->eq) : (nd == 2 ? strong_f64_2(n, h->eq) : strong_f64_3(n, h->eq));
         else
@@ -722,15 +744,19 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
         const int64_t fill = h->tp == FLOU_HIP_TP_STDAVG || n < 6 ? 0
                              : nd == 2 ? 256 * (n == 6 ? 6 : 12) : (n == 6 ? 256 : 0);
         if (h->v64 && h->vol == FLOU_HIP_SPLIT && h->eq == FLOU_HIP_EULER && !gen && nd >= 2 && n >= 4 && diag &&
-            !oriented && h->gather && h->lift_end && d->nelements >= fill && sbp(d))
+            !oriented && h->gather && h->lift_end && ne >= fill && sbp(d)) {
             h->v64 = nd == 2 ? split_vjp_f64_2(n, h->tp, false) : split_vjp_f64_3(n, h->tp, false);
+            h->vjp_name = "k_svjp";
+        }
         // and on curved elements: 3-D (600 k nodes, Chandrasekhar: 4 nodes per line 92 -> 65 us, 7 146 ->
         // 87, 8 378 -> 131; Kennedy-Gruber at 6, where a line's wave is 56 % full, 82 -> 84), and 2-D with 4
         // nodes or where lines fill the chip (8 nodes, 6241 elements: 50 -> 44 us, 324: 12.5 -> 17)
-        const bool cv = nd == 3 ? !(n == 6 && h->tp == FLOU_HIP_TP_KENNEDY_GRUBER) : n == 4 || d->nelements >= 4096;
+        const bool cv = nd == 3 ? !(n == 6 && h->tp == FLOU_HIP_TP_KENNEDY_GRUBER) : n == 4 || ne >= 4096;
         if (h->v64 && h->vol == FLOU_HIP_SPLIT && h->eq == FLOU_HIP_EULER && !gen && n >= 4 && h->curved && h->gather &&
-            h->lift_end && cv && sbp(d))
+            h->lift_end && cv && sbp(d)) {
             h->v64 = nd == 2 ? split_vjp_f64_2(n, h->tp, true) : split_vjp_f64_3(n, h->tp, true);
+            h->vjp_name = "k_svjp";
+        }
     } else {
         h->v32 = nd == 1 ? vjp_f32_1d(n, h->eq, h->vol, h->tp, h->curved, gen)
                          : (nd == 2 ? vjp_f32_2d(n, h->eq, h->vol, h->tp, h->curved, gen)
@@ -882,6 +908,13 @@ int flou_hip_destroy(flou_hip_handle* h) {
     free_all(h);
     delete h;
     return FLOU_HIP_OK;
+}
+
+const char* flou_hip_kernel_name(const flou_hip_handle* h, int32_t which) {
+    if (!h || which < 0 || which > 1) return nullptr;
+    if (which == 0) return h->lfast && !h->force_plain ? (h->curved ? "k_fastc" : "k_fast") : h->rhs_name;
+    if (!h->v64 && !h->v32) return "";
+    return h->vfast && !h->force_plain ? "k_fvjp" : h->vjp_name;
 }
 
 int flou_hip_set_stream(flou_hip_handle* h, void* stream) {

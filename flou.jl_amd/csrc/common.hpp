@@ -211,6 +211,11 @@ RhsLauncherF64 hybrid_f64_3(int n, int tp, bool diag);
 RhsLauncherF32 hybrid_f32_1(int n, int tp, bool diag);
 RhsLauncherF32 hybrid_f32_2(int n, int tp, bool diag);
 RhsLauncherF32 hybrid_f32_3(int n, int tp, bool diag);
+// its kernel for small axis-aligned meshes, null where ne elements are too many
+RhsLauncherF64 hybrid_lines_f64_1(int n, int tp, int64_t ne);
+RhsLauncherF64 hybrid_lines_f64_2(int n, int tp, int64_t ne);
+RhsLauncherF32 hybrid_lines_f32_1(int n, int tp, int64_t ne);
+RhsLauncherF32 hybrid_lines_f32_2(int n, int tp, int64_t ne);
 
 // FP64 split-form Euler kernels on axis-aligned affine elements, GLL nodes, StdAverage or
 // LxF(StdAverage) surface flux (rhs_split.hip): the plain kernels' results.

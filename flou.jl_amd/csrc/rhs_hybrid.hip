@@ -543,19 +543,15 @@ __global__ void __launch_bounds__((LCfg<ND, N>::TPB)) k_hybrid_lines(const RhsAr
 
 template <typename T, int ND, int N, int TP, bool DIAG>
 static hipError_t launch(const RhsArgs<T>& a, hipStream_t s) {
-    // small meshes: blocks that all run at once (three per CU in FP64, six in FP32); N nodes per
-    // line, 2-D, matrix dissipation, k_hybrid and k_hybrid_lines: FP64 N=6, 540 blocks 16.9 and 12.2
-    // us, 740 23.8 and 19.8, N=5, 800 21.1 and 22.2, 4000 65 and 72
-    if constexpr (DIAG && ND <= 2) {
-        using L = LCfg<ND, N>;
-        const int nb = (a.ne + L::EPB - 1) / L::EPB;
-        if (nb <= (sizeof(T) == 8 ? 768 : 1536)) {
-            hipLaunchKernelGGL((k_hybrid_lines<T, ND, N, TP>), dim3(nb), dim3(L::TPB), 0, s, a);
-            return hipGetLastError();
-        }
-    }
     using C = HCfg<ND, N>;
     hipLaunchKernelGGL((k_hybrid<T, ND, N, TP, DIAG>), dim3((a.ne + C::EPB - 1) / C::EPB), dim3(C::TPB), 0, s, a);
+    return hipGetLastError();
+}
+
+template <typename T, int ND, int N, int TP>
+static hipError_t launch_lines(const RhsArgs<T>& a, hipStream_t s) {
+    using C = LCfg<ND, N>;
+    hipLaunchKernelGGL((k_hybrid_lines<T, ND, N, TP>), dim3((a.ne + C::EPB - 1) / C::EPB), dim3(C::TPB), 0, s, a);
     return hipGetLastError();
 }
 
@@ -565,6 +561,21 @@ static hipError_t (*pick_tp(int tp))(const RhsArgs<T>&, hipStream_t) {
         case TP_STDAVG: return &launch<T, ND, N, TP_STDAVG, DIAG>;
         case TP_CHANDRASEKHAR: return &launch<T, ND, N, TP_CHANDRASEKHAR, DIAG>;
         case TP_KENNEDY_GRUBER: return &launch<T, ND, N, TP_KENNEDY_GRUBER, DIAG>;
+        default: return nullptr;
+    }
+}
+
+// k_hybrid_lines where ne elements are few, else null: blocks that all run at once (three per CU in
+// FP64, six in FP32); N nodes per line, 2-D, matrix dissipation, k_hybrid and k_hybrid_lines: FP64 N=6, 540
+// blocks 16.9 and 12.2 us, 740 23.8 and 19.8, N=5, 800 21.1 and 22.2, 4000 65 and 72
+template <typename T, int ND, int N>
+static hipError_t (*pick_lines(int tp, int64_t ne))(const RhsArgs<T>&, hipStream_t) {
+    const int64_t nb = (ne + LCfg<ND, N>::EPB - 1) / LCfg<ND, N>::EPB;
+    if (nb > (sizeof(T) == 8 ? 768 : 1536)) return nullptr;
+    switch (tp) {
+        case TP_STDAVG: return &launch_lines<T, ND, N, TP_STDAVG>;
+        case TP_CHANDRASEKHAR: return &launch_lines<T, ND, N, TP_CHANDRASEKHAR>;
+        case TP_KENNEDY_GRUBER: return &launch_lines<T, ND, N, TP_KENNEDY_GRUBER>;
         default: return nullptr;
     }
 }
@@ -594,15 +605,31 @@ static hipError_t (*pick_n(int n, int tp))(const RhsArgs<T>&, hipStream_t) {
 #else
 #error "define FLOUHIP_PREC_F64 or FLOUHIP_PREC_F32"
 #endif
-#define FLOUHIP_CAT_(p, d) hybrid_##p##_##d
-#define FLOUHIP_CAT(p, d) FLOUHIP_CAT_(p, d)
+#define FLOUHIP_CAT_(k, p, d) k##p##_##d
+#define FLOUHIP_CAT(k, p, d) FLOUHIP_CAT_(k, p, d)
 
-hipError_t (*FLOUHIP_CAT(FLOUHIP_PTAG, FLOUHIP_ND)(int n, int tp, bool diag))(const RhsArgs<FLOUHIP_SCALAR>&,
-                                                                              hipStream_t) {
+hipError_t (*FLOUHIP_CAT(hybrid_, FLOUHIP_PTAG, FLOUHIP_ND)(int n, int tp, bool diag))(const RhsArgs<FLOUHIP_SCALAR>&,
+                                                                                       hipStream_t) {
 #if FLOUHIP_ND > 1
     if (!diag) return hybrid::pick_n<FLOUHIP_SCALAR, FLOUHIP_ND, false>(n, tp);
 #endif
     return hybrid::pick_n<FLOUHIP_SCALAR, FLOUHIP_ND, true>(n, tp);
 }
+
+#if FLOUHIP_ND < 3
+hipError_t (*FLOUHIP_CAT(hybrid_lines_, FLOUHIP_PTAG, FLOUHIP_ND)(int n, int tp, int64_t ne))(
+    const RhsArgs<FLOUHIP_SCALAR>&, hipStream_t) {
+    switch (n) {
+        case 2: return hybrid::pick_lines<FLOUHIP_SCALAR, FLOUHIP_ND, 2>(tp, ne);
+        case 3: return hybrid::pick_lines<FLOUHIP_SCALAR, FLOUHIP_ND, 3>(tp, ne);
+        case 4: return hybrid::pick_lines<FLOUHIP_SCALAR, FLOUHIP_ND, 4>(tp, ne);
+        case 5: return hybrid::pick_lines<FLOUHIP_SCALAR, FLOUHIP_ND, 5>(tp, ne);
+        case 6: return hybrid::pick_lines<FLOUHIP_SCALAR, FLOUHIP_ND, 6>(tp, ne);
+        case 7: return hybrid::pick_lines<FLOUHIP_SCALAR, FLOUHIP_ND, 7>(tp, ne);
+        case 8: return hybrid::pick_lines<FLOUHIP_SCALAR, FLOUHIP_ND, 8>(tp, ne);
+        default: return nullptr;
+    }
+}
+#endif
 
 }  // namespace flouhip

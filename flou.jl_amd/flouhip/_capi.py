@@ -61,6 +61,7 @@ SYMBOLS = {
     "flou_hip_last_error": (ctypes.c_char_p, [_vp]),
     "flou_hip_create_error": (ctypes.c_char_p, []),
     "flou_hip_set_option": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int32]),
+    "flou_hip_kernel_name": (ctypes.c_char_p, [_vp, ctypes.c_int32]),
     "flou_hip_set_stream": (ctypes.c_int, [_vp, _vp]),
     "flou_hip_set_bc": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int32, _d]),
     "flou_hip_ndofs": (ctypes.c_int64, [_vp]),

@@ -147,6 +147,10 @@ class MultielementDisc:
         """True when this (FP32) discretisation's adjoint runs the fast fused kernel."""
         return C.lib.flou_hip_set_option(self.h, 3, 0) == 1
 
+    def kernel_name(self, adjoint=False):
+        """Name of the kernel that runs this discretisation's rhs and stages, or their adjoint."""
+        return C.lib.flou_hip_kernel_name(self.h, int(adjoint)).decode()
+
     def _set_bcs(self, bcs):
         mesh = self.mesh
         for name, bc in bcs.items():

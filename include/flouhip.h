@@ -169,6 +169,11 @@ const char* flou_hip_create_error(void);
  *     fast rhs), else 0. */
 int flou_hip_set_option(flou_hip_handle* h, int32_t which, int32_t value);
 
+/* Name of the kernel that runs the handle's rhs and RK stages (which = 0) or their adjoint (1; "" where
+ * it has none), e.g. "k_split": chosen by equation, form, geometry, precision and mesh size.  NULL
+ * for another `which`. */
+const char* flou_hip_kernel_name(const flou_hip_handle* h, int32_t which);
+
 /* Stream the handle launches on (hipStream_t; NULL = default stream). */
 int flou_hip_set_stream(flou_hip_handle* h, void* stream);
 

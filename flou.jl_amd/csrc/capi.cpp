@@ -699,7 +699,7 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
             h->rhs_name = "k_split_curved";
         }
         if (kvol == VOL_SPLIT && h->eq == FLOU_HIP_EULER && nd == 1 && diag && h->gather && h->lift_end)
-            if (const RhsLauncherF64 f = split_f64_1_small(n, h->tp, ne)) {
+            if (const RhsLauncherF64 f = split_f64_1_small(n, h->tp, ne, lxf && !oriented)) {
                 h->l64 = f;
                 h->rhs_name = "k_split_1d";
             }
@@ -738,20 +738,26 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
         // 4 or more nodes per direction: one line per thread (rhs_vjp, Chandrasekhar, 16384
         // elements of 6x6 nodes: 55 -> 40 us, 0.5 M nodes of 8x8x8: 238 -> 72); below that lines are
         // too short for it.  A line is a chain of n(n-1)/2 pairs: on meshes that leave CUs idle the
-        // thread per node is done sooner (7x7 nodes, 576 elements: 11.6 against 14.9 us, 6084: 34
-        // against 24; 6x6, 1296: 11.6 against 12.1, 2304: 14.5 against 12.3; 6x6x6, 125: 16.0
-        // against 17.5, 512: 22.8 against 19.3), but not StdAverage's, a sum of node terms.
-        const int64_t fill = h->tp == FLOU_HIP_TP_STDAVG || n < 6 ? 0
-                             : nd == 2 ? 256 * (n == 6 ? 6 : 12) : (n == 6 ? 256 : 0);
+        // thread per node is done sooner, but not StdAverage's, a sum of node terms.  Its times over the
+        // line's in 2-D, Chandrasekhar and Kennedy-Gruber: 4 nodes 1.07 to 1.14 at every size; 5: 0.92 and 1.00 at
+        // 4624 elements, 1.13 and 1.18 at 5184; 6: 0.86 and 1.00 at 3025, 1.07 and 1.17 at 3844; 7: 0.77 and 0.81 at
+        // 1024, 1.06 and 0.95 at 3025, 1.23 at 3844; 8: 0.77 and 0.79 at 1024, 0.90 and 1.03 at 3025, 1.07 and 1.15
+        // at 3844 (all above 1 from there).  3-D, 6 nodes: 0.91 and 0.98 at 216, 1.23 and 1.30 at 343; other
+        // node counts 1.04 and more from 8 elements.
+        const int64_t many = n == 5 ? 5120 : 3584;
+        const int64_t fill = h->tp == FLOU_HIP_TP_STDAVG || n == 4 ? 0 : nd == 2 ? many : (n == 6 ? 256 : 0);
         if (h->v64 && h->vol == FLOU_HIP_SPLIT && h->eq == FLOU_HIP_EULER && !gen && nd >= 2 && n >= 4 && diag &&
             !oriented && h->gather && h->lift_end && ne >= fill && sbp(d)) {
             h->v64 = nd == 2 ? split_vjp_f64_2(n, h->tp, false) : split_vjp_f64_3(n, h->tp, false);
             h->vjp_name = "k_svjp";
         }
         // and on curved elements: 3-D (600 k nodes, Chandrasekhar: 4 nodes per line 92 -> 65 us, 7 146 ->
-        // 87, 8 378 -> 131; Kennedy-Gruber at 6, where a line's wave is 56 % full, 82 -> 84), and 2-D with 4
-        // nodes or where lines fill the chip (8 nodes, 6241 elements: 50 -> 44 us, 324: 12.5 -> 17)
-        const bool cv = nd == 3 ? !(n == 6 && h->tp == FLOU_HIP_TP_KENNEDY_GRUBER) : n == 4 || ne >= 4096;
+        // 87, 8 378 -> 131; 1.04 and more from one element up, Kennedy-Gruber with 6 nodes 0.98 to 1.12); 2-D with 4
+        // nodes (1.03 to 1.09) or, as above, on many elements (5 nodes 0.88 at 4096, 1.07 at 5184; 6: 0.85
+        // at 3025, 1.07 at 3844; 7: 1.06 and 1.23).  Not in 2-D: 8 nodes, and Kennedy-Gruber with 5 and 7, 0.82 to
+        // 1.2 without a trend up to 25,600 elements.
+        const bool cv = nd == 3 || n == 4 ||
+                        (ne >= many && n < 8 && (n == 6 || h->tp != FLOU_HIP_TP_KENNEDY_GRUBER));
         if (h->v64 && h->vol == FLOU_HIP_SPLIT && h->eq == FLOU_HIP_EULER && !gen && n >= 4 && h->curved && h->gather &&
             h->lift_end && cv && sbp(d)) {
             h->v64 = nd == 2 ? split_vjp_f64_2(n, h->tp, true) : split_vjp_f64_3(n, h->tp, true);

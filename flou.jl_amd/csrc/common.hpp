@@ -211,7 +211,7 @@ RhsLauncherF64 hybrid_f64_3(int n, int tp, bool diag);
 RhsLauncherF32 hybrid_f32_1(int n, int tp, bool diag);
 RhsLauncherF32 hybrid_f32_2(int n, int tp, bool diag);
 RhsLauncherF32 hybrid_f32_3(int n, int tp, bool diag);
-// its kernel for small axis-aligned meshes, null where ne elements are too many
+// its kernel for small axis-aligned meshes, null where the other is as fast for ne elements
 RhsLauncherF64 hybrid_lines_f64_1(int n, int tp, int64_t ne);
 RhsLauncherF64 hybrid_lines_f64_2(int n, int tp, int64_t ne);
 RhsLauncherF32 hybrid_lines_f32_1(int n, int tp, int64_t ne);
@@ -220,8 +220,8 @@ RhsLauncherF32 hybrid_lines_f32_2(int n, int tp, int64_t ne);
 // FP64 split-form Euler kernels on axis-aligned affine elements, GLL nodes, StdAverage or
 // LxF(StdAverage) surface flux (rhs_split.hip): the plain kernels' results.
 RhsLauncherF64 split_f64_1(int n, int tp);
-// 1-D with any surface flux, null where ne elements are too many
-RhsLauncherF64 split_f64_1_small(int n, int tp, int64_t ne);
+// 1-D with any surface flux (lxf: one that split_f64_1 takes too), null where another kernel is as fast
+RhsLauncherF64 split_f64_1_small(int n, int tp, int64_t ne, bool lxf);
 RhsLauncherF64 split_f64_2(int n, int tp);
 RhsLauncherF64 split_f64_3(int n, int tp);
 // the same on curved elements, up to rounding

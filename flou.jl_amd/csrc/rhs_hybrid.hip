@@ -565,13 +565,18 @@ static hipError_t (*pick_tp(int tp))(const RhsArgs<T>&, hipStream_t) {
     }
 }
 
-// k_hybrid_lines where ne elements are few, else null: blocks that all run at once (three per CU in
-// FP64, six in FP32); N nodes per line, 2-D, matrix dissipation, k_hybrid and k_hybrid_lines: FP64 N=6, 540
-// blocks 16.9 and 12.2 us, 740 23.8 and 19.8, N=5, 800 21.1 and 22.2, 4000 65 and 72
+// k_hybrid_lines on small meshes, else null: blocks that all run at once, three per CU in FP64, four
+// in FP32.  k_hybrid over it, all node counts, matrix dissipation and LxF, at 256, 512 and 768 blocks: 2-D FP64 1.2 to
+// 1.7, 1.0 to 1.5 and 1.04 to 1.5 (1024: 0.78 to 1.23); 2-D FP32 1.2 to 1.6, 1.2 to 1.5, 1.1 to 1.5, and at 1024
+// 1.01 to 1.36 (1536: 0.95 to 1.2); 1-D FP32 1.04 to 1.2 at 256, 1.0 to 1.1 at 1024.  1-D FP64: 1.02 to 1.3 up to one
+// block per CU; above that 0.88 to 1.02 while k_hybrid, whose blocks hold twice the elements and more, still has one
+// per CU, then 0.99 to 1.3.
 template <typename T, int ND, int N>
 static hipError_t (*pick_lines(int tp, int64_t ne))(const RhsArgs<T>&, hipStream_t) {
+    constexpr int CUS = 256;
     const int64_t nb = (ne + LCfg<ND, N>::EPB - 1) / LCfg<ND, N>::EPB;
-    if (nb > (sizeof(T) == 8 ? 768 : 1536)) return nullptr;
+    if (nb > (sizeof(T) == 8 ? 3 : 4) * CUS) return nullptr;
+    if (ND == 1 && sizeof(T) == 8 && nb > CUS && (ne + HCfg<ND, N>::EPB - 1) / HCfg<ND, N>::EPB <= CUS) return nullptr;
     switch (tp) {
         case TP_STDAVG: return &launch_lines<T, ND, N, TP_STDAVG>;
         case TP_CHANDRASEKHAR: return &launch_lines<T, ND, N, TP_CHANDRASEKHAR>;

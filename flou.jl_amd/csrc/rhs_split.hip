@@ -415,12 +415,15 @@ static hipError_t launch_1d(const RhsArgs<double>& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// While all blocks run at once; of larger meshes k_split takes those with the LxF flux, the general
-// kernel the rest (Chandrasekhar and matrix dissipation, general kernel and k_split_1d: N=3, 952 blocks
-// 10.7 and 10.4 us, 2381 13.1 and 14.3; N=7, 625 10.6 and 10.3, 6250 15.3 and 29.5).
+// While all blocks run at once.  Against the general kernel (lxf false: the other surface fluxes) that is
+// up to 1024 blocks at every node count (512 to 1024 blocks, N nodes per line: 1.0 to 1.2 times as fast at 2 and
+// 3, 1.1 to 1.4 from 4; N=8, 6250 blocks 15.3 us against 29.5).  k_split, which LxF and StdAverage have instead,
+// does without the second half of the block: 5 nodes and more up to 768 blocks (1.0 to 1.3; 8 nodes and StdAverage,
+// 896 blocks 5.16 us against 5.37); 2 and 3 nodes 0.88 to 1.0 from 128 blocks, 4 nodes 0.91 to 1.08.
 template <int N>
-static RhsLauncherF64 pick_1d(int tp, int64_t ne) {
-    if ((ne + ECfg<N>::EPB - 1) / ECfg<N>::EPB > 1024) return nullptr;
+static RhsLauncherF64 pick_1d(int tp, int64_t ne, bool lxf) {
+    const int64_t nb = (ne + ECfg<N>::EPB - 1) / ECfg<N>::EPB;
+    if (lxf ? N < 5 || nb > 768 : nb > 1024) return nullptr;
     switch (tp) {
         case TP_STDAVG: return &launch_1d<N, TP_STDAVG>;
         case TP_CHANDRASEKHAR: return &launch_1d<N, TP_CHANDRASEKHAR>;
@@ -757,15 +760,15 @@ RhsLauncherF64 FLOUHIP_CAT(split_f64_, FLOUHIP_ND)(int n, int tp) {
 }
 
 #if FLOUHIP_ND == 1
-RhsLauncherF64 split_f64_1_small(int n, int tp, int64_t ne) {
+RhsLauncherF64 split_f64_1_small(int n, int tp, int64_t ne, bool lxf) {
     switch (n) {
-        case 2: return split::pick_1d<2>(tp, ne);
-        case 3: return split::pick_1d<3>(tp, ne);
-        case 4: return split::pick_1d<4>(tp, ne);
-        case 5: return split::pick_1d<5>(tp, ne);
-        case 6: return split::pick_1d<6>(tp, ne);
-        case 7: return split::pick_1d<7>(tp, ne);
-        case 8: return split::pick_1d<8>(tp, ne);
+        case 2: return split::pick_1d<2>(tp, ne, lxf);
+        case 3: return split::pick_1d<3>(tp, ne, lxf);
+        case 4: return split::pick_1d<4>(tp, ne, lxf);
+        case 5: return split::pick_1d<5>(tp, ne, lxf);
+        case 6: return split::pick_1d<6>(tp, ne, lxf);
+        case 7: return split::pick_1d<7>(tp, ne, lxf);
+        case 8: return split::pick_1d<8>(tp, ne, lxf);
         default: return nullptr;
     }
 }

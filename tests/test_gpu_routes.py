@@ -54,3 +54,53 @@ def test_plain_option():
     d = disc(3, 6, [2, 2, 2], F.SplitDivOperator(CH, LXF), "fp32")
     d.set_option(1, 1)
     assert (d.kernel_name(), d.kernel_name(adjoint=True)) == ("k_plain", "k_vjp")
+
+
+SPLIT_CH, SPLIT_KG, SPLIT_STD = (F.SplitDivOperator(tp, LXF) for tp in (CH, KG, STD))
+HYBRID = F.HybridDivOperator(CH, MATRIX, 1.0)
+
+
+# the last mesh of each size rule's range, and the first beyond it
+@pytest.mark.parametrize("inside,outside,args,nel_in,nel_out", [
+    ("k_split_1d", "k_split", (1, 5, SPLIT_CH), [768 * 12], [768 * 12 + 1]),
+    ("k_split_1d", "k_split", (1, 8, SPLIT_STD), [768 * 4], [768 * 4 + 1]),
+    ("k_split_1d", "k_plain", (1, 8, F.SplitDivOperator(CH, MATRIX)), [1024 * 4], [1024 * 4 + 1]),
+    ("k_split_1d", "k_plain", (1, 2, F.SplitDivOperator(KG, MATRIX)), [1024 * 64], [1024 * 64 + 1]),
+    ("k_hybrid_lines", "k_hybrid", (2, 6, HYBRID), [48, 48], [48, 49]),
+    ("k_hybrid_lines", "k_hybrid", (2, 6, HYBRID, "fp32"), [64, 48], [64, 49]),
+    ("k_hybrid_lines", "k_hybrid", (1, 5, HYBRID), [256 * 21], [256 * 21 + 1]),
+    ("k_hybrid_lines", "k_hybrid", (1, 5, HYBRID), [256 * 51 + 1], [256 * 51]),
+    ("k_hybrid_lines", "k_hybrid", (1, 5, HYBRID), [768 * 21], [768 * 21 + 1]),
+    ("k_hybrid_lines", "k_hybrid", (1, 5, HYBRID, "fp32"), [1024 * 21], [1024 * 21 + 1]),
+], ids=lambda x: None if isinstance(x, tuple) else str(x).replace(" ", ""))
+def test_size_rules_of_the_rhs(inside, outside, args, nel_in, nel_out):
+    nd, n, op, *precision = args
+    assert disc(nd, n, nel_in, op, *precision).kernel_name() == inside
+    assert disc(nd, n, nel_out, op, *precision).kernel_name() == outside
+
+
+# meshes that take the line adjoint, and ones too small for it (or None)
+@pytest.mark.parametrize("args,nel,small", [
+    ((2, 4, SPLIT_CH, False), [1, 2], None),
+    ((2, 5, SPLIT_CH, False), [80, 64], [79, 64]),
+    ((2, 6, SPLIT_KG, False), [64, 56], [63, 56]),
+    ((2, 8, SPLIT_CH, False), [64, 56], [63, 56]),
+    ((2, 8, SPLIT_STD, False), [3, 3], None),
+    ((3, 6, SPLIT_CH, False), [8, 8, 4], [17, 5, 3]),
+    ((3, 7, SPLIT_KG, False), [1, 2, 2], None),
+    ((2, 4, SPLIT_STD, True), [2, 2], None),
+    ((2, 5, SPLIT_CH, True), [80, 64], [79, 64]),
+    ((2, 6, SPLIT_KG, True), [64, 56], [63, 56]),
+    ((2, 7, SPLIT_STD, True), [64, 56], [63, 56]),
+    ((3, 6, SPLIT_KG, True), [1, 2, 2], None),
+], ids=lambda x: f"{x[0]}d-n{x[1]}" if isinstance(x, tuple) else str(x).replace(" ", ""))
+def test_size_rules_of_the_adjoint(args, nel, small):
+    nd, n, op, curved = args
+    assert disc(nd, n, nel, op, curved=curved).kernel_name(adjoint=True) == "k_svjp"
+    if small:
+        assert disc(nd, n, small, op, curved=curved).kernel_name(adjoint=True) == "k_vjp"
+
+
+@pytest.mark.parametrize("n,op", [(5, SPLIT_KG), (7, SPLIT_KG), (8, SPLIT_CH), (8, SPLIT_STD)])
+def test_general_adjoint_on_large_curved_meshes(n, op):
+    assert disc(2, n, [72, 72], op, curved=True).kernel_name(adjoint=True) == "k_vjp"

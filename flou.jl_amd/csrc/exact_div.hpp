@@ -31,6 +31,7 @@ struct Recip {
     __device__ T div(T a) const { return a / b; }                   // a / b
     __device__ T div2(T a) const { return a / (T(2) * b); }         // a / (2b)
     __device__ T fin(T a) const { return a / b; }                   // a / b, b finite and not 0, a finite
+    __device__ T fix(T q, T a) const { return q; }                  // div(a) from q = fin(a)
 };
 
 template <>
@@ -46,6 +47,7 @@ struct Recip<double> {
         const double q = a * y;
         return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
     }
+    __device__ double fix(double q, double a) const { return __builtin_amdgcn_div_fixup(q, b, a); }
     __device__ double div(double a) const { return quot(a, b, y); }
     __device__ double div2(double a) const { return quot(a, 2.0 * b, 0.5 * y); }
     __device__ double fin(double a) const {
@@ -65,6 +67,7 @@ struct Recip<float> {
         const float q = a * y;
         return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-b, q, a), y, q), b, a);
     }
+    __device__ float fix(float q, float a) const { return __builtin_amdgcn_div_fixupf(q, b, a); }
     __device__ float div(float a) const { return quot(a, b, y); }
     __device__ float div2(float a) const { return quot(a, 2.0f * b, 0.5f * y); }
     __device__ float fin(float a) const {

@@ -739,23 +739,27 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
         // elements of 6x6 nodes: 55 -> 40 us, 0.5 M nodes of 8x8x8: 238 -> 72); below that lines are
         // too short for it.  A line is a chain of n(n-1)/2 pairs: on meshes that leave CUs idle the
         // thread per node is done sooner, but not StdAverage's, a sum of node terms.  Its times over the
-        // line's in 2-D, Chandrasekhar and Kennedy-Gruber: 4 nodes 1.07 to 1.14 at every size; 5: 0.92 and 1.00 at
-        // 4624 elements, 1.13 and 1.18 at 5184; 6: 0.86 and 1.00 at 3025, 1.07 and 1.17 at 3844; 7: 0.77 and 0.81 at
-        // 1024, 1.06 and 0.95 at 3025, 1.23 at 3844; 8: 0.77 and 0.79 at 1024, 0.90 and 1.03 at 3025, 1.07 and 1.15
-        // at 3844 (all above 1 from there).  3-D, 6 nodes: 0.91 and 0.98 at 216, 1.23 and 1.30 at 343; other
-        // node counts 1.04 and more from 8 elements.
-        const int64_t many = n == 5 ? 5120 : 3584;
-        const int64_t fill = h->tp == FLOU_HIP_TP_STDAVG || n == 4 ? 0 : nd == 2 ? many : (n == 6 ? 256 : 0);
+        // line's in 2-D, Kennedy-Gruber: 4 nodes 1.07 to 1.14 at every size; 5: 1.00 at 4624 elements, 1.18 at
+        // 5184; 6: 1.00 at 3025, 1.17 at 3844; 7: 0.95 and 1.23; 8: 1.03 and 1.15.  Chandrasekhar on smooth states and
+        // on rough ones (every pair in the logarithm's branch, which costs a line twice a node's share): 5: 1.04 and 0.95
+        // at 7225, 1.36 at 8100, 1.33 on rough states at 10404; 6: 1.04 and 0.92 at 5184, 1.32 at 5776, 1.33 on
+        // rough ones at 7225; 7: 1.44 and 1.16 at 5184; 8: 1.07 and 0.83 at 3844, 1.42 and 1.19 at 5184.  3-D: 5 nodes,
+        // Chandrasekhar 1.07 and 0.80 at 343, 1.33 and 1.12 at 1000; 6 nodes 0.91 to 0.98 at 216, 1.23 and 0.96 at
+        // 343, 1.51 and 1.15 at 2744; other node counts 1.1 and more.
+        const bool logs = h->tp == FLOU_HIP_TP_CHANDRASEKHAR;
+        const int64_t many = 256 * (n == 5 ? (logs ? 30 : 20) : (logs ? 22 : 14));
+        const int64_t fill = h->tp == FLOU_HIP_TP_STDAVG || n == 4 ? 0
+                             : nd == 2 ? many : (n == 6 ? 256 : (n == 5 && logs ? 768 : 0));
         if (h->v64 && h->vol == FLOU_HIP_SPLIT && h->eq == FLOU_HIP_EULER && !gen && nd >= 2 && n >= 4 && diag &&
             !oriented && h->gather && h->lift_end && ne >= fill && sbp(d)) {
             h->v64 = nd == 2 ? split_vjp_f64_2(n, h->tp, false) : split_vjp_f64_3(n, h->tp, false);
             h->vjp_name = "k_svjp";
         }
         // and on curved elements: 3-D (600 k nodes, Chandrasekhar: 4 nodes per line 92 -> 65 us, 7 146 ->
-        // 87, 8 378 -> 131; 1.04 and more from one element up, Kennedy-Gruber with 6 nodes 0.98 to 1.12); 2-D with 4
-        // nodes (1.03 to 1.09) or, as above, on many elements (5 nodes 0.88 at 4096, 1.07 at 5184; 6: 0.85
-        // at 3025, 1.07 at 3844; 7: 1.06 and 1.23).  Not in 2-D: 8 nodes, and Kennedy-Gruber with 5 and 7, 0.82 to
-        // 1.2 without a trend up to 25,600 elements.
+        // 87, 8 378 -> 131; 1.04 and more from one element up; 6 nodes 1.05 to 1.12, on rough states 0.92 to
+        // 0.99, Kennedy-Gruber 0.98 to 1.12); 2-D with 4 nodes (1.03 to 1.09) or, as above, on many elements
+        // (StdAverage's lines are chains here: 5 nodes 0.95 at 4096, 1.10 at 5184; 6: 0.93 at 3025, 1.09 at 3844).
+        // Not in 2-D: 8 nodes, and Kennedy-Gruber with 5 and 7, 0.82 to 1.2 without a trend up to 25,600 elements.
         const bool cv = nd == 3 || n == 4 ||
                         (ne >= many && n < 8 && (n == 6 || h->tp != FLOU_HIP_TP_KENNEDY_GRUBER));
         if (h->v64 && h->vol == FLOU_HIP_SPLIT && h->eq == FLOU_HIP_EULER && !gen && n >= 4 && h->curved && h->gather &&

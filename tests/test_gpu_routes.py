@@ -82,14 +82,18 @@ def test_size_rules_of_the_rhs(inside, outside, args, nel_in, nel_out):
 # meshes that take the line adjoint, and ones too small for it (or None)
 @pytest.mark.parametrize("args,nel,small", [
     ((2, 4, SPLIT_CH, False), [1, 2], None),
-    ((2, 5, SPLIT_CH, False), [80, 64], [79, 64]),
+    ((2, 5, SPLIT_CH, False), [96, 80], [95, 80]),
+    ((2, 5, SPLIT_KG, False), [80, 64], [79, 64]),
     ((2, 6, SPLIT_KG, False), [64, 56], [63, 56]),
-    ((2, 8, SPLIT_CH, False), [64, 56], [63, 56]),
+    ((2, 8, SPLIT_CH, False), [88, 64], [87, 64]),
     ((2, 8, SPLIT_STD, False), [3, 3], None),
     ((3, 6, SPLIT_CH, False), [8, 8, 4], [17, 5, 3]),
-    ((3, 7, SPLIT_KG, False), [1, 2, 2], None),
+    ((3, 5, SPLIT_CH, False), [12, 8, 8], [11, 8, 8]),
+    ((3, 5, SPLIT_KG, False), [1, 2, 2], None),
+    ((3, 7, SPLIT_CH, False), [1, 2, 2], None),
     ((2, 4, SPLIT_STD, True), [2, 2], None),
-    ((2, 5, SPLIT_CH, True), [80, 64], [79, 64]),
+    ((2, 5, SPLIT_CH, True), [96, 80], [95, 80]),
+    ((2, 5, SPLIT_STD, True), [80, 64], [79, 64]),
     ((2, 6, SPLIT_KG, True), [64, 56], [63, 56]),
     ((2, 7, SPLIT_STD, True), [64, 56], [63, 56]),
     ((3, 6, SPLIT_KG, True), [1, 2, 2], None),
@@ -103,4 +107,4 @@ def test_size_rules_of_the_adjoint(args, nel, small):
 
 @pytest.mark.parametrize("n,op", [(5, SPLIT_KG), (7, SPLIT_KG), (8, SPLIT_CH), (8, SPLIT_STD)])
 def test_general_adjoint_on_large_curved_meshes(n, op):
-    assert disc(2, n, [72, 72], op, curved=True).kernel_name(adjoint=True) == "k_vjp"
+    assert disc(2, n, [100, 80], op, curved=True).kernel_name(adjoint=True) == "k_vjp"

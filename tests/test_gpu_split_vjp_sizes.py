@@ -15,11 +15,12 @@ pytest.importorskip("torch")
 
 
 @pytest.mark.parametrize("nd,n,tp,nel,curved", [
-    (2, 5, "ch", [80, 64], False), (2, 5, "kg", [83, 62], False), (2, 6, "ch", [64, 56], False),
-    (2, 6, "kg", [61, 59], False), (2, 7, "ch", [64, 56], False), (2, 7, "kg", [61, 59], False),
-    (2, 8, "ch", [64, 56], False), (2, 8, "kg", [61, 59], False), (3, 6, "kg", [8, 8, 4], False),
-    (2, 5, "ch", [83, 62], True), (2, 5, "std", [80, 64], True), (2, 6, "ch", [61, 59], True),
-    (2, 6, "kg", [64, 56], True), (2, 6, "std", [61, 59], True), (2, 7, "ch", [64, 56], True),
+    (2, 5, "ch", [96, 80], False), (2, 5, "kg", [83, 62], False), (2, 6, "ch", [88, 64], False),
+    (2, 6, "kg", [61, 59], False), (2, 7, "ch", [83, 68], False), (2, 7, "kg", [61, 59], False),
+    (2, 8, "ch", [83, 68], False), (2, 8, "kg", [61, 59], False), (3, 5, "ch", [11, 10, 7], False),
+    (3, 6, "ch", [8, 8, 4], False), (3, 6, "kg", [11, 6, 4], False),
+    (2, 5, "ch", [101, 77], True), (2, 5, "std", [80, 64], True), (2, 6, "ch", [83, 68], True),
+    (2, 6, "kg", [64, 56], True), (2, 6, "std", [61, 59], True), (2, 7, "ch", [88, 64], True),
     (2, 7, "std", [61, 59], True), (3, 6, "kg", [3, 2, 1], True)])
 def test_dot_product_with_oracle_jvp(nd, n, tp, nel, curved):
     if curved:

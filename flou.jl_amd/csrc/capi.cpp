@@ -685,7 +685,7 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
         if (!h->l64) return bad(FLOU_HIP_EUNSUPPORTED, "no kernel for this combination");
         // split-form Euler with the StdAverage/LxF surface flux on axis-aligned affine elements:
         // the same results from a kernel without the terms that this geometry makes exact
-        // zeros (3-D N=5, 10.5 M nodes: 0.99 ms per stage against 1.65 ms)
+        // zeros (3-D N=5, 10.5 M nodes: 0.90 ms per stage against 1.65 ms)
         const bool lxf = h->savg == FLOU_HIP_AVG_STD &&
                          (h->sdiss == FLOU_HIP_DISS_NONE || h->sdiss == FLOU_HIP_DISS_LXF);
         if (kvol == VOL_SPLIT && h->eq == FLOU_HIP_EULER && lxf && diag && !oriented && h->gather &&
@@ -693,7 +693,7 @@ int flou_hip_create(const flou_hip_desc* d, flou_hip_handle** out) {
             h->l64 = nd == 1 ? split_f64_1(n, h->tp) : (nd == 2 ? split_f64_2(n, h->tp) : split_f64_3(n, h->tp));
             h->rhs_name = "k_split";
         }
-        // and on curved elements (3-D N=6, 11.2 M nodes: 3.0 -> 1.0 ms per stage)
+        // and on curved elements (3-D N=6, 11.2 M nodes: 3.0 -> 1.03 ms per stage)
         else if (kvol == VOL_SPLIT && h->eq == FLOU_HIP_EULER && lxf && h->curved && h->gather && h->lift_end) {
             h->l64 = nd == 2 ? split_curved_f64_2(n, h->tp) : split_curved_f64_3(n, h->tp);
             h->rhs_name = "k_split_curved";

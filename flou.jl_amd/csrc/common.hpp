@@ -240,7 +240,7 @@ RhsLauncherF32 strong_f32_3(int n, int eq);
 typedef hipError_t (*VjpLauncherF64)(const VjpArgs<double>&, hipStream_t);
 typedef hipError_t (*VjpLauncherF32)(const VjpArgs<float>&, hipStream_t);
 // FP64 adjoint of the split form on axis-aligned affine or curved elements (vjp_split.hip),
-// n = 4..8.
+// n = 4..8 (curved 2-D: not 8, nor 5 and 7 with Kennedy-Gruber).
 VjpLauncherF64 split_vjp_f64_2(int n, int tp, bool curved);
 VjpLauncherF64 split_vjp_f64_3(int n, int tp, bool curved);
 VjpLauncherF64 vjp_f64_1d(int n, int eq, int vol, int tp, int curved, int gen);

@@ -7,14 +7,14 @@
 // limit leaves under it (1.8 to 2.0 of 2.4 GHz).  k_plain<double, 3, 6, ..> spends about 4000
 // VALU slots per node, most of them on divisions, on the two components of every flux that a
 // diagonal metric multiplies by zero, and on rotations by 0 and ±1.  Measured against it (same
-// bits): 3-D N=5, 10.5 M nodes, Chandrasekhar: 1.65 -> 0.96 ms per CK2N54 stage; 2-D N=5, 0.59 M
-// nodes: 66 -> 43 us.  With the same results:
+// bits): 3-D N=5, 10.5 M nodes, Chandrasekhar: 1.65 -> 0.90 ms per CK2N54 stage; 2-D N=5, 0.59 M
+// nodes: 66 -> 40 us.  With the same results:
 //   * only the flux component along the line's direction is formed: f·n̄ has one term, the
 //     others are exact zeros.  The direction is a compile-time constant of each phase;
 //   * flux inputs are staged halved, so that means are one addition (pair_flux);
 //   * a node's own contravariant flux goes into the same table as the pairs, so that its row
 //     reads N entries without a case for the diagonal, at offsets that advance by constants
-//     (2504 -> 2186 VALU per wave at 3-D N=5 with the above, 0.99 -> 0.96 ms);
+//     (2504 -> 2186 VALU per wave at 3-D N=5 with the above, 2084 with all that follows);
 //   * face states are read in the order of the face frame by index (faces.hpp);
 //   * quotients share reciprocals (exact_div.hpp), the node's contravariant flux reuses its
 //     primitives, the lift touches the end nodes only (∂g is exactly zero elsewhere);
@@ -452,9 +452,10 @@ static RhsLauncherF64 pick_tp(int tp) {
 // to a CU up to 128 registers: they read a node's velocities from its slots again for each direction (3-D
 // N=6, held in registers: 133, one block per CU, 84 us against 61 at 0.6 M nodes).  Faces: the flux along n from the master's frame; every sum over the two sides
 // commutes and is rounded the same way on both, so that the sides' fluxes are opposite bit for bit.
-// What bounds it: waits between the barriers at two or three blocks per CU; HBM moves 1.6 GB a
-// stage at 11.2 M nodes, 0.34 ms at a copy's rate.  Measured, Chandrasekhar, SSPRK33 steps: 3-D N=6,
-// 11.2 M nodes: 9.1 -> 3.0 ms; N=5, 7.1 M nodes: 3.6 -> 1.8 ms.
+// What bounds it: waits between the barriers at two or three blocks per CU.  A stage at 11.2 M nodes needs
+// 2.1 GB (187 bytes per node) and moves 1.75 GB (FETCH_SIZE 1.30, WRITE_SIZE 0.45: part of the rest comes from the
+// cache behind the L2s), 0.37 ms at a copy's rate.  Measured, Chandrasekhar, SSPRK33 steps: 3-D N=6,
+// 11.2 M nodes: 9.1 -> 3.1 ms; N=5, 7.1 M nodes: 3.6 -> 1.8 ms.
 
 // One direction: pairs and the nodes' own fluxes into the table, then (LOADS between) the
 // nodes' D♯ rows over it.  m: the metric row of the own node.
